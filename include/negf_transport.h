@@ -295,6 +295,14 @@ int nt_set_multi_workers(nt_ctx* ctx, int n);
  * counterpart in the reference. */
 int nt_set_point_split(nt_ctx* ctx, int n);
 
+/* FP64 batched solves without extra outputs run on the planes that the zero
+ * blocks of the principal layers divide them into, where every plane holds at
+ * most 64 degrees of freedom (default on): the same block elimination on
+ * smaller blocks.  Points with a singular or nearly singular plane are solved
+ * on the layers.  on = 0: always on the layers.  No counterpart in the
+ * reference. */
+int nt_set_planes(nt_ctx* ctx, int on);
+
 /* Host-pointer variant (copies in and out; same layout). */
 int nt_solve_tdb_batched(nt_ctx* ctx, const nt_params* p, int nl, int nr, int b, int L,
                          int npts, const double* E, const int* kidx, int nk,
@@ -674,7 +682,7 @@ int nt_zsqrtm_batched_dev(nt_ctx* ctx, int n, const nt_c128* A, long long stride
 
 /* ------------------------------------------------------- measurement */
 /* Kernel classes for nt_profile_get. */
-enum { NT_K_GEMM = 0, NT_K_INV = 1, NT_K_ELEM = 2, NT_K_EIG = 3, NT_K_COUNT = 4 };
+enum { NT_K_GEMM = 0, NT_K_INV = 1, NT_K_ELEM = 2, NT_K_EIG = 3, NT_K_PLANES = 4, NT_K_COUNT = 5 };
 /* While enabled, each launch is bracketed by HIP events on the context's
  * stream; nt_profile_get returns launches, summed milliseconds and the summed
  * algorithmic flops (GEMM 8mnk, inverse 8n^3 per active item) of a class. */

@@ -197,8 +197,13 @@ __global__ void k_make_shifts(const double* E, int batch, double eta, double eta
     if (zd32) { zd32[2 * p] = (float)e; zd32[2 * p + 1] = (float)ed; }
 }
 
+// An item whose alpha is not finite (the maximum's +inf) can never converge:
+// its next inverse reads a NaN and every later step is a masked-in step of NaN
+// blocks up to max_iter.  It ends here with the status and the count it would
+// end with; k_dec_dead gives it the NaN blocks (the ribbon at eta = 1e-8 eV
+// has 0 to 3 such points in 2048, whose steps 33 .. 300 were 100 ms).
 __global__ void k_dec_step_update(int* active, unsigned long long* maxabs, int* iters, double conv, int* count,
-                                  int* clear, int batch)
+                                  int* clear, int batch, int* status, int max_iter)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     int still = 0;
@@ -206,12 +211,27 @@ __global__ void k_dec_step_update(int* active, unsigned long long* maxabs, int* 
         const double m = __longlong_as_double((long long)maxabs[p]);
         if (iters) iters[p] += 1;
         still = (m > conv) ? 1 : 0;     // inf (NaN marker) stays active and hits the cap
+        if (still && status && m > 1.7976931348623157e308 && iters[p] + 2 <= max_iter) {
+            still = 0;
+            iters[p] = max_iter;
+            if (status[p] == 0) status[p] = -1;
+        }
         active[p] = still;
     }
     if (p < batch) maxabs[p] = 0ull;
     if (p == 0) *clear = 0;
     for (int off = 32; off > 0; off >>= 1) still += __shfl_xor(still, off);
     if ((threadIdx.x & 63) == 0 && still) atomicAdd(count, still);
+}
+
+// NaN over the n x n block of every item with status -1
+__global__ void k_dec_dead(const int* status, double* es, long elems, int batch)
+{
+    for (int q = blockIdx.x; q < batch; q += gridDim.x) {
+        if (status[q] != -1) continue;
+        double* e = es + (long)q * 2 * elems;
+        for (long i = threadIdx.x; i < 2 * elems; i += blockDim.x) e[i] = __longlong_as_double(0x7ff8000000000000LL);
+    }
 }
 
 __global__ void k_fill_int(int* p, int v, int n)
@@ -310,11 +330,18 @@ hipError_t launch_make_shifts(const double* E, int batch, double eta, double eta
 }
 
 hipError_t launch_dec_step_update(int* active, unsigned long long* maxabs, int* iters, double conv, int* count,
-                                  int* clear, int batch, hipStream_t s)
+                                  int* clear, int batch, int* status, int max_iter, hipStream_t s)
 {
     if (batch <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_dec_step_update, dim3(blocks_for(batch)), dim3(NT), 0, s, active, maxabs, iters, conv,
-                       count, clear, batch);
+                       count, clear, batch, status, max_iter);
+    return hipGetLastError();
+}
+
+hipError_t launch_dec_dead(const int* status, double* es, long elems, int batch, hipStream_t s)
+{
+    if (batch <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_dec_dead, dim3(batch < 1024 ? batch : 1024), dim3(NT), 0, s, status, es, elems, batch);
     return hipGetLastError();
 }
 

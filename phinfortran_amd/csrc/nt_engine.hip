@@ -144,6 +144,13 @@ __global__ void k_corner_blocks(int nl, int nr, BMat<double> G00, BMat<double> G
     o[1] = sg * (gr * di + gi * dr);
 }
 
+// the initial active flags of a masked decimation: `per` items per point
+__global__ void k_expand_mask(const int* mask, int* active, int Q, int per)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < Q) active[q] = mask[q / per] != 0;
+}
+
 // fb[p] = !accept[p]; *count += number of rejected points
 __global__ void k_reject_mask(const int* accept, int* fb, int* count, int P)
 {
@@ -161,10 +168,10 @@ __global__ void k_dec_finish(const int* active, int* status, int Q)
 
 // point status = first nonzero of (dec left, dec right, rgf); iters = mean
 __global__ void k_point_status(const int* st_dec, const int* it_dec, const int* st_rgf, int P, int* status, int* iters,
-                               const int* first_mask, double* T_LR, double* T_RL)
+                               const int* first_mask, const int* mask, double* T_LR, double* T_RL)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= P) return;
+    if (p >= P || (mask && !mask[p])) return;
     int s = st_dec[2 * p];
     if (!s) s = st_dec[2 * p + 1];
     if (!s) s = st_rgf[p];
@@ -202,7 +209,8 @@ struct DecimationOut {
 
 template <typename T>
 void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger, const T* z, double conv,
-              int max_iter, DecimationOut<T> out, int* status, int* iters, Arena& ar, size_t scratch_off)
+              int max_iter, DecimationOut<T> out, int* status, int* iters, Arena& ar, size_t scratch_off,
+              const int* mask = nullptr, int per = 1)
 {
     const long nn = (long)n * n;
     const size_t mb = sizeof(T) * 2 * nn;
@@ -232,14 +240,21 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
     zero_dev(c, iters, sizeof(int) * Q, s);
     zero_dev(c, maxabs, sizeof(unsigned long long) * Q, s);
     zero_dev(c, nact, sizeof(int) * 2, s);
-    launch(c, NT_K_ELEM, 0, "fill", [&] { return launch_fill_int(active, 1, Q, s); });
+    if (mask) {
+        // items of the points left out start as converged
+        check_range(c, mask, sizeof(int) * (Q / per), "dec mask");
+        hipLaunchKernelGGL(k_expand_mask, dim3(nblk(Q)), dim3(256), 0, s, mask, active, Q, per);
+        hipcheck(c, hipGetLastError(), "dec mask");
+    } else {
+        launch(c, NT_K_ELEM, 0, "fill", [&] { return launch_fill_int(active, 1, Q, s); });
+    }
     // initial maxdiff = max|alpha| (surface.f90:484): the GEMM epilogue's
     // maxabs on a K = 0 product with Cin = alpha0 (a copy), then one update
     // (update 0: slot 0) that does not count as an iteration
     gemm<T>(c, n, n, 0, OP_N, none<T>(), OP_N, none<T>(), bw(W, nn, n), 1.0, bm<T>(ab0, 2 * nn, n), 1.0, nullptr, Q,
             0.0, nullptr, 1, nonew<T>(), maxabs);
     launch(c, NT_K_ELEM, 0, "dec_update",
-           [&] { return launch_dec_step_update(active, maxabs, nullptr, conv, nact, nact + 1, Q, s); });
+           [&] { return launch_dec_step_update(active, maxabs, nullptr, conv, nact, nact + 1, Q, nullptr, 0, s); });
 
     // Iteration it runs its launches on the items still active (converged
     // items are masked inside every kernel, so an extra iteration changes
@@ -284,7 +299,8 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
                 nonew<T>(), maxabs);
         const int u = it + 1;
         launch(c, NT_K_ELEM, 0, "dec_update", [&] {
-            return launch_dec_step_update(active, maxabs, iters, conv, nact + (u & 1), nact + ((u + 1) & 1), Q, s);
+            return launch_dec_step_update(active, maxabs, iters, conv, nact + (u & 1), nact + ((u + 1) & 1), Q, status,
+                                          max_iter, s);
         });
         std::swap(abc, abn);
     }
@@ -301,14 +317,23 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
     }
     hipLaunchKernelGGL(k_dec_finish, dim3(nblk(Q)), dim3(256), 0, s, active, status, Q);
     hipcheck(c, hipGetLastError(), "dec_finish");
+    if (std::is_same<T, double>::value)
+        launch(c, NT_K_ELEM, 0, "dec_dead",
+               [&] { return launch_dec_dead(status, reinterpret_cast<double*>(es), nn, Q, s); });
+    const int* fin = nullptr;
+    if (mask) {
+        hipLaunchKernelGGL(k_expand_mask, dim3(nblk(Q)), dim3(256), 0, s, mask, active, Q, per);
+        hipcheck(c, hipGetLastError(), "dec mask");
+        fin = active;
+    }
     // g = (z - es)^-1 for every item (surface.f90:497)
-    inverse<T>(c, n, bw(W, nn, n), bm<T>(es, nn, n), z, out.g, status, Q);
+    inverse<T>(c, n, bw(W, nn, n), bm<T>(es, nn, n), z, out.g, status, Q, -1, fin);
     if (out.sigma.base) {
         // Sigma = alpha0 g beta0 = V^+ g V (alpha_dagger) ; t1 = V^+ g
         gemm<T>(c, n, n, n, alpha_dagger ? OP_C : OP_N, V, OP_N, ro(out.g), bw(t12, 2 * nn, n), 1.0, none<T>(), 0.0,
-                nullptr, Q);
+                nullptr, Q, -1, fin);
         gemm<T>(c, n, n, n, OP_N, bm<T>(t12, 2 * nn, n), alpha_dagger ? OP_N : OP_C, V, out.sigma, 1.0, none<T>(),
-                0.0, nullptr, Q);
+                0.0, nullptr, Q, -1, fin);
         if (out.gamma.base) gamma_op<T>(c, n, ro(out.sigma), out.gamma, Q);
     }
 }
@@ -527,7 +552,7 @@ size_t decimate_circular_scratch(int n, int Q, int nm, int NB)
 // Surface GFs (and Sigma, Gamma) of Q lead items; direct or circular decimation.
 void lead_gfs(nt_ctx* c, const nt_params* prm, int n, int Q, int nm, const double* H00s, const double* Vs,
               const int* idx, int alpha_dagger, const double* z, DecimationOut<double> out, int* status, int* iters,
-              Arena& ar, size_t scratch_off)
+              Arena& ar, size_t scratch_off, const int* mask = nullptr, int per = 1)
 {
     if (prm->circular && prm->n_bloch_x * prm->n_bloch_y > 1) {
         decimate_circular(c, prm, n, Q, nm, H00s, Vs, idx, alpha_dagger, z, out, status, iters, ar, scratch_off);
@@ -535,7 +560,7 @@ void lead_gfs(nt_ctx* c, const nt_params* prm, int n, int Q, int nm, const doubl
         const long nn = (long)n * n;
         decimate<double>(c, n, Q, bm<double>(H00s, nm > 1 || idx ? nn : 0, n, idx, 0, idx ? nm : 0),
                          bm<double>(Vs, nm > 1 || idx ? nn : 0, n, idx, 0, idx ? nm : 0), alpha_dagger, z,
-                         prm->convergence, prm->max_iter, out, status, iters, ar, scratch_off);
+                         prm->convergence, prm->max_iter, out, status, iters, ar, scratch_off, mask, per);
     }
 }
 
@@ -1350,6 +1375,26 @@ constexpr double MIXED_BUDGET_BYTES = 64.0 * 1024 * 1024 * 1024;
 void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
 {
     typedef double T;
+    if (planes_candidate(c, prm, a)) {
+        // every device whose layers fall into planes is solved on them
+        std::vector<const TdbArgs*> rest;
+        std::vector<const TdbArgs*> all{&a};
+        all.insert(all.end(), a.siblings.begin(), a.siblings.end());
+        double sum = 0.0;
+        for (const TdbArgs* d : all) {
+            if (!planes_solve(c, prm, *d)) rest.push_back(d);
+            else sum += c->last_mean_iters;
+        }
+        if (rest.empty()) {
+            c->last_mean_iters = sum / all.size();
+            return;
+        }
+        TdbArgs g = *rest[0];
+        g.no_planes = true;
+        g.siblings.assign(rest.begin() + 1, rest.end());
+        solve_tdb_dev(c, prm, g);
+        return;
+    }
     const int nl = a.nl, nr = a.nr, b = a.b, L = a.L;
     const long nll = (long)nl * nl, nrr = (long)nr * nr, bb = (long)b * b;
     const bool same = nl == nr;
@@ -1464,7 +1509,7 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         }
         // the static scratch, or a workspace cap of the context (worker
         // contexts of a multi-device call share the device's memory)
-        const size_t cap = a.noalloc ? NT_SCRATCH_BYTES : c->ws_cap;
+        const size_t cap = a.noalloc ? NT_SCRATCH_BYTES - a.scratch_reserve : c->ws_cap;
         if (cap == 0 || pa.off <= cap) break;
         if (Pmax == 1) {
             if (!a.noalloc) break;     // one point over a workspace cap: solve it anyway
@@ -1551,6 +1596,7 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         const int P = std::min(Pmax, a.npts - p0);
         const double* E = a.E + p0;
         const int* kidx = a.kidx ? a.kidx + p0 : nullptr;
+        const int* mask = a.mask ? a.mask + p0 : nullptr;
         hipLaunchKernelGGL(k_lead_setup, dim3(nblk(P)), dim3(256), 0, s, E, kidx, a.nk, P, 1, prm->eta,
                            prm->eta0, prm->eta_mode, prm->device_eta_factor, idx, zdec, pm ? zpm : nullptr, zdev);
         hipcheck(c, hipGetLastError(), "lead setup");
@@ -1569,7 +1615,7 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         if (same) {
             const long n2 = nll;
             DecimationOut<T> o{bw(gbuf, n2, nl), bw(sigbuf, n2, nl), bw(gambuf, n2, nl)};
-            lead_gfs(c, prm, nl, 2 * P, 2 * a.nk, lh, lv, idx, 1, zdec, o, stdec, itdec, ar, o_scr);
+            lead_gfs(c, prm, nl, 2 * P, 2 * a.nk, lh, lv, idx, 1, zdec, o, stdec, itdec, ar, o_scr, mask, 2);
             if (pm) {
                 DecimationOut<T> o2{bw(gpmbuf, n2, nl), nonew<T>(), nonew<T>()};
                 lead_gfs(c, prm, nl, 2 * P, 2 * a.nk, lh, lv, idx, 0, zpm, o2, stpm, itpm, ar, o_scr);
@@ -1590,10 +1636,10 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
                 zero_dev(c, sts, sizeof(int) * 2 * P, s);
                 DecimationOut<T> ol{bw(g, 2 * nmm, nl), sg ? bw(sg, 2 * nmm, nl) : nonew<T>(),
                                     gm ? bw(gm, 2 * nmm, nl) : nonew<T>()};
-                lead_gfs(c, prm, nl, P, a.nk, Haml, Hamlv, idx1, adag, zz, ol, sts, its, ar, o_scr);
+                lead_gfs(c, prm, nl, P, a.nk, Haml, Hamlv, idx1, adag, zz, ol, sts, its, ar, o_scr, mask);
                 DecimationOut<T> orr{bw(g + 2 * nmm, 2 * nmm, nr), sg ? bw(sg + 2 * nmm, 2 * nmm, nr) : nonew<T>(),
                                      gm ? bw(gm + 2 * nmm, 2 * nmm, nr) : nonew<T>()};
-                lead_gfs(c, prm, nr, P, a.nk, Hamr, Hamrv, idx1, adag, zz + 2 * P, orr, sts + P, its + P, ar, o_scr);
+                lead_gfs(c, prm, nr, P, a.nk, Hamr, Hamrv, idx1, adag, zz + 2 * P, orr, sts + P, its + P, ar, o_scr, mask);
                 hipLaunchKernelGGL(k_lead_merge, dim3(nblk(P)), dim3(256), 0, s, sts, its, P, st2, it2);
                 hipcheck(c, hipGetLastError(), "lead merge");
             };
@@ -1628,6 +1674,7 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         in.gmr = bm<T>(gambuf + 2 * nmm, 2 * nmm, nr);
         in.zlead = zdec + 2;          // right retarded E + i eta(E) of each point (stride 4)
         in.zlead_stride = 4;
+        in.act = mask;
         if (probe) {
             in.zl = ar.ptr<T>(o_pzl);
             in.keep = ar.ptr<T>(o_pkeep);
@@ -1776,7 +1823,7 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         // ---- status, iterations, clamps
         hipLaunchKernelGGL(k_point_status, dim3(nblk(P)), dim3(256), 0, s, stdec, itdec, strgf, P,
                            a.status ? a.status + p0 : nullptr, a.iters ? a.iters + p0 : nullptr,
-                           a.first_mask ? a.first_mask + p0 : nullptr, a.T_LR + p0, a.T_RL + p0);
+                           a.first_mask ? a.first_mask + p0 : nullptr, mask, a.T_LR + p0, a.T_RL + p0);
         hipcheck(c, hipGetLastError(), "point status");
         // ---- devices sharing these leads: their own sweeps on the same lead GFs
         for (const TdbArgs* sb : a.siblings) {
@@ -1807,7 +1854,8 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
             if (sb->first_mask) check_range(c, sb->first_mask + p0, sizeof(int) * P, "sibling mask");
             hipLaunchKernelGGL(k_point_status, dim3(nblk(P)), dim3(256), 0, s, stdec, itdec, strgf, P,
                                sb->status ? sb->status + p0 : nullptr, nullptr,
-                               sb->first_mask ? sb->first_mask + p0 : nullptr, sb->T_LR + p0, sb->T_RL + p0);
+                               sb->first_mask ? sb->first_mask + p0 : nullptr, nullptr, sb->T_LR + p0,
+                               sb->T_RL + p0);
             hipcheck(c, hipGetLastError(), "sibling point status");
         }
         // mean iterations (host side, for the flop model); not read when the
@@ -1985,6 +2033,7 @@ int nt_create(nt_ctx** out, int device_ordinal)
         hipEventCreateWithFlags(&c->join, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->chk[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->chk[1], hipEventDisableTiming) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&c->host_plan), 16 * sizeof(int)) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&c->host_flag), 2 * sizeof(int)) != hipSuccess) {
         nt_destroy(c);        // releases whatever was created
         return NT_ERR_HIP;
@@ -2020,6 +2069,9 @@ int nt_destroy(nt_ctx* c)
     for (auto& u : c->circ_u) (void)hipFree(u.d);
     if (c->deg_buf) (void)hipFree(c->deg_buf);
     for (nt_ctx* s : c->subs) nt_destroy(s);
+    if (c->plan_buf) (void)hipFree(c->plan_buf);
+    if (c->left_buf) (void)hipFree(c->left_buf);
+    if (c->host_plan) (void)hipHostFree(c->host_plan);
     if (c->host_flag) (void)hipHostFree(c->host_flag);
     if (c->own) (void)hipStreamDestroy(c->own);
     if (c->aux) (void)hipStreamDestroy(c->aux);
@@ -2199,6 +2251,10 @@ static int tdb_entry(nt_ctx* c, const nt_params* p, int nl, int nr, int b, int L
         // the other's GEMMs.  Not the probe solve, whose grouped GEMMs fill
         // the GPU by themselves (two parts: 287 against 297 probe solves/s at
         // b = 192, L = 40, 128 points)
+        if (planes_candidate(c, p, a)) {
+            if (planes_solve(c, p, a)) return 0;
+            a.no_planes = true;
+        }
         const int parts = c->point_split;
         if (parts > 1 && !noalloc && !pd && npts >= parts * NT_SPLIT_MIN_POINTS) {
             solve_split(c, p, a, parts);
@@ -2304,6 +2360,10 @@ int nt_solve_tdb_adjoint_batched_dev(nt_ctx* c, const nt_params* p, int nl, int 
         a.dHdv = nc > 0 ? dW_dHamdv : nullptr;
         // many points: parts solved side by side by worker contexts, as the
         // batched solve (the adjoint sweep runs in FP64 whatever the precision)
+        if (planes_candidate(c, p, a)) {
+            if (planes_solve(c, p, a)) return 0;
+            a.no_planes = true;
+        }
         const int parts = c->point_split;
         if (parts > 1 && npts >= parts * NT_SPLIT_MIN_POINTS) {
             solve_split(c, p, a, parts);

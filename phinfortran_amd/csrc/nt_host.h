@@ -85,6 +85,16 @@ struct nt_ctx {
     // degenerate-group descriptors and statuses of the path_mode = 1 rotation
     void* deg_buf = nullptr;
     size_t deg_bytes = 0;
+    // batched FP64 solves on the planes of the layers (nt_planes.hip); its plan
+    // and a pinned copy of the plan's header
+    bool planes = true;
+    void* plan_buf = nullptr;
+    size_t plan_bytes = 0;
+    int* host_plan = nullptr;
+    // its points left to the layers (gathered inputs and results)
+    void* left_buf = nullptr;
+    size_t left_bytes = 0;
+    bool worker = false;           // a worker context of another one
     // uneven-device calls: worker contexts (own stream and workspace, one host
     // thread each) that solve groups of devices concurrently
     int multi_workers = 4;
@@ -491,6 +501,7 @@ inline int guarded(nt_ctx* c, F&& f)
         hipcheck(c, hipSetDevice(c->device), "hipSetDevice");
         c->regions.clear();
         reg_region(c, c->ws, c->ws_bytes);
+        reg_region(c, c->plan_buf, c->plan_bytes);
         size_t sb = 0;
         if (void* sp = scratch_region(c->device, &sb)) reg_region(c, sp, sb);
         int r = f();

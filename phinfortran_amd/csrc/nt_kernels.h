@@ -261,7 +261,8 @@ hipError_t launch_make_shifts(const double* E, int batch, double eta, double eta
 // (the two words of a two-slot counter: update u adds to slot u % 2 and clears
 // the other, so after any update its slot holds that update's count)
 hipError_t launch_dec_step_update(int* active, unsigned long long* maxabs, int* iters, double conv, int* count,
-                                  int* clear, int batch, hipStream_t s);
+                                  int* clear, int batch, int* status, int max_iter, hipStream_t s);
+hipError_t launch_dec_dead(const int* status, double* es, long elems, int batch, hipStream_t s);
 hipError_t launch_fill_int(int* p, int v, int n, hipStream_t s);
 // Final transmission clean-up: clamp < 1e-60 to 0, zero when flagged, status merge.
 hipError_t launch_finish_T(double* T, int n, int zero_all, hipStream_t s);

@@ -1,0 +1,64 @@
+// The plane solver's argument blocks and host entry (nt_planes.hip).
+#pragma once
+#include "nt_solve.h"
+
+struct PlanHdr {
+    int ok;        // every layer falls into planes of one size class
+    int nt;        // class: planes padded to 16 nt
+    int M;         // planes of the whole system
+    int m0, m1;    // planes of the left and right lead cell
+};
+
+struct DecPlArgs {
+    const PlanHdr* h;
+    const int* psize;
+    const double2 *H, *U, *Lw, *LV;
+    const double* E;
+    const int* kidx;
+    double eta, eta0, conv;
+    int eta_mode, max_iter;
+    double2* scratch;      // DEC_SLOTS matrices per item
+    double2* sigma;        // retarded self-energy per item (point, lead)
+    int *status, *iters;
+    double* grow;
+};
+
+struct SweepPlArgs {
+    const PlanHdr* h;
+    const int* psize;
+    const double2 *H, *U, *Lw;
+    const unsigned long long* masks;       // per (k, plane): U's 4 x 16 and 16 x 4 pieces, Lw's
+    const double* E;
+    const int* kidx;
+    double eta, eta0, dev_factor;
+    int eta_mode;
+    const int* need;       // points left out
+    const double2* sigma;
+    double* T;             // per item (point, direction)
+    int* status;
+    // adjoint: G^L_j and (G^L_{0,j})^T of the planes from *keep_from on, two
+    // matrices per plane, keep_stride matrices per point (null: not kept)
+    double2* keep;
+    const int* keep_from;
+    long keep_stride;
+};
+
+struct AdjPlArgs {
+    const PlanHdr* h;
+    const int *psize, *player, *poff, *perm;
+    const double2 *U, *Lw;
+    const unsigned long long* masks;
+    const double2 *sigma, *keep;
+    long keep_stride;
+    const int* kidx;
+    const int *need, *status, *dstatus, *first;
+    const double* w;
+    const int* place;      // place of a point among the points of its chunk, by k
+    int lo, hi1;           // window layers (device layers, 0-based), with the one after
+    int b;
+    long K;                // rows of the gathered row matrices: points of the chunk x NP
+    double2 *CA, *RW;      // per window layer: b x K and K x b
+};
+
+// n worker contexts of c set up for a call (nt_workers.hip)
+int prepare_workers(nt_ctx* c, int n);

@@ -1,0 +1,1869 @@
+// nt_planes.hip -- batched solve on the planes of the principal layers.
+//
+// Force constants and hoppings of short range couple a principal layer to the
+// next one through a few of its degrees of freedom only, and inside the layer
+// they couple neighbours.  The degrees of freedom of every layer, sorted by
+// their distance (in couplings) from the ones the previous layer touches, then
+// form planes that couple to the plane before and after only: a diamond layer
+// one conventional cell thick has four, of a quarter of its size.  The same
+// block elimination (lead decimation, both sweeps, Caroli T) on these smaller
+// blocks gives the same Green's functions with (planes per layer)^2 fewer
+// operations: b = 192, L = 40 takes 1.9 GFLOP per point instead of 29.
+//
+//   k_pl_pattern  which elements of the blocks are nonzero at any k-point
+//   k_pl_levels   per layer: distances from the previous layer, plane counts
+//   k_pl_plan     plane size class (16, 32, 48, 64), plane offsets, validity
+//   k_pl_perm     degrees of freedom of every plane
+//   k_pl_pack     diagonal and coupling blocks of the planes, per k-point,
+//                 zero padded to the class size
+//   k_pl_decimate one workgroup per (point, lead): the lead's self-energy
+//   k_pl_sweep    one workgroup per (point, direction): the whole sweep and T
+//   k_pl_finish   statuses, iteration counts, clamps
+//
+// The plan stays on the device: no kernel needs the host to know it, so a
+// solve can be captured in a HIP graph.  Blocks without zeros form one plane
+// per layer; layers of planes over 64 are left to the block path.
+//
+// Inside the two solver kernels a wave owns 16 columns of every matrix, in
+// registers, in the layout in which v_mfma_f64_16x16x4 returns its result:
+// row 4 r + lane / 16 of a tile is element r, and that is the layout in which
+// the same instruction takes its B operand, so a chain of products needs no
+// exchange between lanes or waves; only A operands come from memory.
+#include <type_traits>
+
+#include "nt_host.h"
+#include "nt_kernels.h"
+#include "nt_planes.h"
+
+namespace {
+
+typedef double2 C2;
+
+constexpr int PL_MAXNT = 4;         // largest class: planes of 64
+constexpr int PL_WAVES = 2;          // waves per SIMD the solver kernels are built for
+constexpr int PL_NLV = 128;         // levels a layer may have
+// A decimation step whose cell is nearly singular at E loses digits that the
+// later steps do not bring back, on planes and on layers alike: two correct
+// evaluations of T then differ by more than rounding (1e-6 and more on the
+// graphene ribbon at eta = 1e-8 eV, where some points overflow).  Such points
+// are left to the layers, so that the planes do not move them.  The measure is
+// g = |z - e|_max |(z - e)^-1|_max over the steps, and as the loss grows with
+// how far the broadening is below the energy scale, g (1e-7 scale / eta)^2 is
+// what is bounded: with the bound below the rest of the ribbon's points agree
+// to 1e-8, at 250 of 2048 left to the layers; of the phonon workloads (eta
+// about 1e-6 of the scale) at most a few in a thousand are.
+constexpr double PL_GROWTH = 2.0e8;
+
+// ------------------------------------------------------------------ the plan
+// Device arrays of the plan (ints), carved from one buffer.
+struct PlanView {
+    PlanHdr* h;
+    unsigned* adj;      // (layer, dof) rows of adjacency bits, W words each
+    unsigned* cbits;    // (layer) W words: dofs coupled to the previous layer
+    unsigned* rbits;    // (layer) W words: dofs coupled to the next layer
+    int* bad;           // leads not Hermitian
+    int* level;         // (layer, dof)
+    int* nlev;          // (layer)
+    int* cnt;           // (layer, PL_NLV) dofs per level
+    int* npl;           // (layer, PL_MAXNT) planes per class, -1: a level does not fit
+    int* poff;          // (layer + 1) first plane
+    int* psize;         // (plane)
+    int* player;        // (plane) layer
+    int* perm;          // (plane, 64) dof of the layer at each place
+};
+
+// sizes a plan depends on
+struct PlanDims {
+    int nl, nr, b, L, nk;
+    int nmax, W, Mcap;
+};
+
+PlanDims plan_dims(int nl, int nr, int b, int L, int nk)
+{
+    PlanDims d{nl, nr, b, L, nk, 0, 0, 0};
+    d.nmax = std::max(b, std::max(nl, nr));
+    d.W = (d.nmax + 31) / 32;
+    // two neighbouring planes of a layer hold more than 16 dofs together
+    d.Mcap = (2 * (nl / 16) + 2) + (2 * (nr / 16) + 2) + L * (2 * (b / 16) + 2);
+    return d;
+}
+
+PlanView plan_carve(Arena& a, const PlanDims& d)
+{
+    const size_t nL = d.L + 2, i4 = sizeof(int);
+    PlanView v;
+    // zeroed region first: header, bits, flags
+    const size_t oh = a.take(sizeof(PlanHdr)), oa = a.take(i4 * nL * d.nmax * d.W), oc = a.take(i4 * nL * d.W),
+                 orr = a.take(i4 * nL * d.W), ob = a.take(i4);
+    const size_t ol = a.take(i4 * nL * d.nmax), on = a.take(i4 * nL), oq = a.take(i4 * nL * PL_NLV),
+                 op = a.take(i4 * nL * PL_MAXNT), oo = a.take(i4 * (nL + 1)), os = a.take(i4 * d.Mcap),
+                 oy = a.take(i4 * d.Mcap), om = a.take(i4 * (size_t)d.Mcap * 64);
+    v.h = a.ptr<PlanHdr>(oh);
+    v.adj = a.ptr<unsigned>(oa);
+    v.cbits = a.ptr<unsigned>(oc);
+    v.rbits = a.ptr<unsigned>(orr);
+    v.bad = a.ptr<int>(ob);
+    v.level = a.ptr<int>(ol);
+    v.nlev = a.ptr<int>(on);
+    v.cnt = a.ptr<int>(oq);
+    v.npl = a.ptr<int>(op);
+    v.poff = a.ptr<int>(oo);
+    v.psize = a.ptr<int>(os);
+    v.player = a.ptr<int>(oy);
+    v.perm = a.ptr<int>(om);
+    return v;
+}
+
+// the caller's blocks
+struct BlocksIn {
+    const C2 *Haml, *Hamlv, *Hamr, *Hamrv, *Hamd, *Hamdv, *Hamld, *Hamrd;
+};
+
+__device__ __forceinline__ int layer_size(const PlanDims& d, int layer)
+{
+    return layer == 0 ? d.nl : layer == d.L + 1 ? d.nr : d.b;
+}
+
+// diagonal block of a layer at k-point k (ld = its size)
+__device__ __forceinline__ const C2* layer_H(const PlanDims& d, const BlocksIn& B, int layer, int k)
+{
+    if (layer == 0) return B.Haml + (long)k * d.nl * d.nl;
+    if (layer == d.L + 1) return B.Hamr + (long)k * d.nr * d.nr;
+    return B.Hamd + ((long)k * d.L + layer - 1) * d.b * d.b;
+}
+
+__device__ __forceinline__ void set_bit(unsigned* w, int i)
+{
+    const unsigned m = 1u << (i & 31);
+    if (!(w[i >> 5] & m)) atomicOr(&w[i >> 5], m);
+}
+
+// blockIdx.y: the L + 2 diagonal blocks, then the couplings lead-lead (left),
+// lead-device, device-device, device-lead, lead-lead (right); blockIdx.z: k
+__global__ void k_pl_pattern(PlanDims d, PlanView v, BlocksIn B, int k0)
+{
+    // (more k-points only add nonzeros: a plan refused stays refused)
+    if (k0 && !v.h->ok) return;
+    const int k = k0 + blockIdx.z, nL = d.L + 2;
+    const long step = (long)gridDim.x * blockDim.x, e0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    int m = blockIdx.y;
+    if (m < nL) {
+        const int n = layer_size(d, m);
+        const C2* H = layer_H(d, B, m, k);
+        unsigned* adj = v.adj + (long)m * d.nmax * d.W;
+        const bool lead = m == 0 || m == nL - 1;
+        for (long e = e0; e < (long)n * n; e += step) {
+            const int r = (int)(e % n), c = (int)(e / n);
+            const C2 x = H[e];
+            if (!(x.x == 0.0 && x.y == 0.0) && r != c) {
+                set_bit(adj + (long)r * d.W, c);
+                set_bit(adj + (long)c * d.W, r);
+            }
+            if (lead && r <= c) {
+                // the left lead is decimated at E - i eta and daggered: only
+                // for a Hermitian lead is that its retarded function
+                const C2 y = H[c + (long)r * n], hr = H[r + (long)r * n], hc = H[c + (long)c * n];
+                const double df = fabs(x.x - y.x) + fabs(x.y + y.y);
+                const double off = fabs(x.x) + fabs(x.y), dg = fabs(hr.x) + fabs(hc.x);
+                if (df > 1e-10 * off && df > 1e-13 * dg) *v.bad = 1;
+            }
+        }
+        return;
+    }
+    m -= nL;
+    const C2* V;
+    int rows, cols;
+    unsigned *rb, *cb;
+    auto R = [&](int layer) { return v.rbits + (long)layer * d.W; };
+    auto Cc = [&](int layer) { return v.cbits + (long)layer * d.W; };
+    if (m == 0) {                    // V_{-1,0}: rows face the device, columns the lead
+        V = B.Hamlv + (long)k * d.nl * d.nl, rows = cols = d.nl, rb = R(0), cb = Cc(0);
+    } else if (m == 1) {             // V_{0,1}
+        V = B.Hamld + (long)k * d.nl * d.b, rows = d.nl, cols = d.b, rb = R(0), cb = Cc(1);
+    } else if (m <= d.L) {           // V_{i,i+1}
+        V = B.Hamdv + ((long)k * (d.L > 1 ? d.L - 1 : 1) + m - 2) * d.b * d.b, rows = cols = d.b, rb = R(m - 1),
+        cb = Cc(m);
+    } else if (m == d.L + 1) {       // V_{N+1,N}
+        V = B.Hamrd + (long)k * d.nr * d.b, rows = d.nr, cols = d.b, rb = Cc(d.L + 1), cb = R(d.L);
+    } else {                         // V_{N+2,N+1}: rows face the device, columns the lead
+        V = B.Hamrv + (long)k * d.nr * d.nr, rows = cols = d.nr, rb = Cc(d.L + 1), cb = R(d.L + 1);
+    }
+    for (long e = e0; e < (long)rows * cols; e += step) {
+        const C2 x = V[e];
+        if (!(x.x == 0.0 && x.y == 0.0)) {
+            set_bit(rb, (int)(e % rows));
+            set_bit(cb, (int)(e / rows));
+        }
+    }
+}
+
+// whether a level begins a plane: it does not fit into the one before, or it
+// is the last of a lead cell that has one plane so far (the decimation works
+// on a cell's first and last plane)
+__device__ __forceinline__ bool plane_starts(bool full, bool lead, bool last, int planes)
+{
+    return full || (lead && last && planes == 1);
+}
+
+// One workgroup per layer: level of every dof = distance from the dofs that
+// face the previous layer; everything from the first dof that faces the next
+// layer on is one level (the next layer couples to the last plane only).
+__global__ __launch_bounds__(256) void k_pl_levels(PlanDims d, PlanView v)
+{
+    const int layer = blockIdx.x, n = layer_size(d, layer), t = threadIdx.x;
+    const unsigned* adj = v.adj + (long)layer * d.nmax * d.W;
+    const unsigned* cb = v.cbits + (long)layer * d.W;
+    const unsigned* rb = v.rbits + (long)layer * d.W;
+    __shared__ short lev[1024];
+    __shared__ unsigned front[32];
+    __shared__ int found, last, cnt[PL_NLV];
+    for (int i = t; i < n; i += 256) lev[i] = (cb[i >> 5] >> (i & 31)) & 1 ? 0 : -1;
+    if (t < PL_NLV) cnt[t] = 0;
+    if (t == 0) last = PL_NLV - 1;
+    int lv = 0;
+    for (; lv < PL_NLV - 1; ++lv) {
+        if (t < 32) front[t] = 0;
+        if (t == 0) found = 0;
+        __syncthreads();
+        for (int i = t; i < n; i += 256)
+            if (lev[i] == lv) atomicOr(&front[i >> 5], 1u << (i & 31));
+        __syncthreads();
+        for (int i = t; i < n; i += 256) {
+            if (lev[i] >= 0) continue;
+            unsigned hit = 0;
+            for (int w = 0; w < d.W; ++w) hit |= adj[(long)i * d.W + w] & front[w];
+            if (hit) {
+                lev[i] = (short)(lv + 1);
+                found = 1;
+            }
+        }
+        __syncthreads();
+        const int f = found;
+        __syncthreads();
+        if (!f) break;
+    }
+    for (int i = t; i < n; i += 256)
+        if (((rb[i >> 5] >> (i & 31)) & 1) && lev[i] >= 0) atomicMin(&last, (int)lev[i]);
+    __syncthreads();
+    const int m = min(last, lv);
+    for (int i = t; i < n; i += 256) {
+        const int l = lev[i] < 0 || lev[i] > m ? m : lev[i];
+        v.level[(long)layer * d.nmax + i] = l;
+        atomicAdd(&cnt[l], 1);
+    }
+    __syncthreads();
+    if (t < PL_NLV) v.cnt[(long)layer * PL_NLV + t] = cnt[t];
+    if (t == 0) v.nlev[layer] = m + 1;
+    if (t < PL_MAXNT) {
+        // planes of at most 16 (t + 1): consecutive levels merged while they
+        // fit (plane_starts); a lead cell keeps two at least
+        const int lim = 16 * (t + 1);
+        const bool lead = layer == 0 || layer == d.L + 1;
+        int planes = 0, fill = lim + 1;
+        for (int l = 0; l <= m; ++l) {
+            const int k = cnt[l];
+            if (k > lim) {
+                planes = -1;
+                break;
+            }
+            if (plane_starts(fill + k > lim, lead, l == m, planes)) {
+                ++planes;
+                fill = k;
+            } else {
+                fill += k;
+            }
+        }
+        v.npl[layer * PL_MAXNT + t] = planes;
+    }
+}
+
+// One workgroup of four waves: wave t sums the planes of class t + 1, the
+// cheapest class wins: per plane about five products of the class size and as
+// many pivots as it has columns (5120 SIMD cycles per 16^3 of products and
+// 12000 per 16 pivots).
+__global__ __launch_bounds__(256) void k_pl_plan(PlanDims d, PlanView v)
+{
+    const int nL = d.L + 2, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ int tot[PL_MAXNT];
+    __shared__ int pick;
+    int s = 0, bad = 0;
+    for (int i = lane; i < nL; i += 64) {
+        const int p = v.npl[i * PL_MAXNT + w];
+        bad |= p < 0;
+        s += p;
+    }
+    for (int o = 32; o; o >>= 1) {
+        s += __shfl_xor(s, o);
+        bad |= __shfl_xor(bad, o);
+    }
+    if (lane == 0) tot[w] = bad ? -1 : s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double best = 0.0;
+        int nt = 0;
+        for (int t = 0; t < PL_MAXNT; ++t) {
+            if (tot[t] < 0) continue;
+            const double u = t + 1, c = tot[t] * (5120.0 * u * u * u + 12000.0 * u);
+            if (!nt || c < best) {
+                best = c;
+                nt = t + 1;
+            }
+        }
+        pick = nt;
+        v.h->nt = nt;
+        v.h->M = nt ? tot[nt - 1] : 0;
+        // one plane per layer: nothing is gained over the layers themselves; a
+        // lead cell of one plane: not written for that
+        v.h->ok = nt > 0 && !*v.bad && tot[nt - 1] <= d.Mcap && tot[nt - 1] > nL &&
+                  v.npl[nt - 1] > 1 && v.npl[(nL - 1) * PL_MAXNT + nt - 1] > 1;
+        v.h->m0 = nt ? v.npl[nt - 1] : 0;
+        v.h->m1 = nt ? v.npl[(nL - 1) * PL_MAXNT + nt - 1] : 0;
+    }
+    __syncthreads();
+    const int nt = pick;
+    if (!nt || w) return;
+    int base = 0;
+    for (int i0 = 0; i0 < nL; i0 += 64) {
+        const int i = i0 + lane;
+        int x = i < nL ? v.npl[i * PL_MAXNT + nt - 1] : 0, inc = x;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(inc, o);
+            if (lane >= o) inc += y;
+        }
+        if (i < nL) v.poff[i] = base + inc - x;
+        base += __shfl(inc, 63);
+    }
+    if (lane == 0) v.poff[nL] = base;
+}
+
+// One workgroup per layer: plane and place of every dof (in dof order)
+__global__ __launch_bounds__(256) void k_pl_perm(PlanDims d, PlanView v)
+{
+    if (!v.h->ok) return;
+    const int layer = blockIdx.x, n = layer_size(d, layer), t = threadIdx.x;
+    const int lim = 16 * v.h->nt, p0 = v.poff[layer], np = v.poff[layer + 1] - p0;
+    __shared__ short pl[1024];
+    __shared__ short of_level[PL_NLV];
+    if (t == 0) {
+        const int nlev = v.nlev[layer];
+        int p = -1, fill = lim + 1;
+        for (int l = 0; l < nlev; ++l) {
+            const int k = v.cnt[(long)layer * PL_NLV + l];
+            if (plane_starts(fill + k > lim, layer == 0 || layer == d.L + 1, l == nlev - 1, p + 1)) {
+                ++p;
+                fill = k;
+            } else {
+                fill += k;
+            }
+            of_level[l] = (short)p;
+        }
+    }
+    __syncthreads();
+    for (int i = t; i < n; i += 256) pl[i] = of_level[v.level[(long)layer * d.nmax + i]];
+    __syncthreads();
+    for (int i = t; i < n; i += 256) {
+        int pos = 0;
+        for (int j = 0; j < i; ++j) pos += pl[j] == pl[i];
+        v.perm[(long)(p0 + pl[i]) * 64 + pos] = i;
+    }
+    for (int p = t; p < np; p += 256) {
+        int c = 0;
+        for (int j = 0; j < n; ++j) c += pl[j] == p;
+        v.psize[p0 + p] = c;
+        v.player[p0 + p] = layer;
+    }
+}
+
+// blockIdx.x: plane, blockIdx.y: k, blockIdx.z: 0 diagonal block, 1 coupling
+// to the next plane, 2 coupling from it (and the two's masks), 3 the leads' cell coupling (planes 0
+// and M - 1 only)
+__global__ __launch_bounds__(256) void k_pl_pack(PlanDims d, PlanView v, BlocksIn B, C2* H, C2* U, C2* Lw, C2* LV,
+                                                 unsigned long long* masks)
+{
+    const PlanHdr& h = *v.h;
+    const int pl = blockIdx.x, k = blockIdx.y, what = blockIdx.z, M = h.M;
+    if (!h.ok || pl >= M) return;
+    const int NP = 16 * h.nt, NN = NP * NP;
+    const int la = v.player[pl], na = layer_size(d, la), sa = v.psize[pl];
+    const int* pa = v.perm + (long)pl * 64;
+    if (what == 3) {
+        if (pl != 0 && pl != M - 1) return;
+        // V from the plane that faces the device (rows) to the one that faces
+        // the lead (columns) of the next cell
+        const int side = pl != 0;
+        const int fb = side ? M - h.m1 : h.m0 - 1;        // plane facing the device
+        const int* pb = v.perm + (long)fb * 64;
+        const int sb = v.psize[fb];
+        const C2* V = side ? B.Hamrv + (long)k * na * na : B.Hamlv + (long)k * na * na;
+        C2* o = LV + ((long)k * 2 + side) * NN;
+        for (int e = threadIdx.x; e < NN; e += 256) {
+            const int r = e % NP, c = e / NP;
+            C2 x = make_double2(0.0, 0.0);
+            if (r < sb && c < sa) x = V[pb[r] + (long)pa[c] * na];
+            o[e] = x;
+        }
+        return;
+    }
+    C2* o = (what == 0 ? H : what == 1 ? U : Lw) + ((long)k * M + pl) * NN;
+    if (what == 0) {
+        const C2* S = layer_H(d, B, la, k);
+        for (int e = threadIdx.x; e < NN; e += 256) {
+            const int r = e % NP, c = e / NP;
+            C2 x = make_double2(0.0, 0.0);
+            if (r < sa && c < sa) x = S[pa[r] + (long)pa[c] * na];
+            o[e] = x;
+        }
+        return;
+    }
+    if (pl + 1 >= M) return;
+    const int lb = v.player[pl + 1], nb = layer_size(d, lb), sb = v.psize[pl + 1];
+    const int* pb = v.perm + (long)(pl + 1) * 64;
+    // U (rows of this plane, columns of the next), Lw (rows of the next)
+    const C2* S = nullptr;
+    int ld = 0;
+    bool dag = false;              // element (r, c) is conj(S[c, r])
+    if (la == lb) {
+        S = layer_H(d, B, la, k);
+        ld = na;
+    } else if (lb == d.L + 1) {    // V_{N,N+1} = V_{N+1,N}^+
+        S = B.Hamrd + (long)k * d.nr * d.b;
+        ld = d.nr;
+        dag = what == 1;
+    } else {
+        S = la == 0 ? B.Hamld + (long)k * d.nl * d.b
+                    : B.Hamdv + ((long)k * (d.L > 1 ? d.L - 1 : 1) + la - 1) * d.b * d.b;
+        ld = na;
+        dag = what == 2;
+    }
+    // which of its 4 x 16 and 16 x 4 pieces are not zero (blk_mul's masks)
+    __shared__ unsigned long long piece[2];
+    if (threadIdx.x < 2) piece[threadIdx.x] = 0;
+    __syncthreads();
+    const int* pr = what == 1 ? pa : pb;
+    const int* pc = what == 1 ? pb : pa;
+    const int sr = what == 1 ? sa : sb, sc = what == 1 ? sb : sa;
+    for (int e = threadIdx.x; e < NN; e += 256) {
+        const int r = e % NP, c = e / NP;
+        C2 x = make_double2(0.0, 0.0);
+        if (r < sr && c < sc) {
+            if (dag) {
+                x = S[pc[c] + (long)pr[r] * ld];
+                x.y = -x.y;
+            } else {
+                x = S[pr[r] + (long)pc[c] * ld];
+            }
+        }
+        o[e] = x;
+        if (!(x.x == 0.0 && x.y == 0.0)) {
+            atomicOr(&piece[0], 1ull << (h.nt * (r / 4) + c / 16));
+            atomicOr(&piece[1], 1ull << (h.nt * (c / 4) + r / 16));
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) masks[(((long)k * M + pl) * 2 + (what - 1)) * 2 + threadIdx.x] = piece[threadIdx.x];
+}
+
+// ------------------------------------------------- one wave's 16 columns
+// The lane's number as a value the compiler takes for a new one at every use:
+// addresses and masks formed from it are formed where they are used instead of
+// being kept, by the hundred, in registers across the solver kernels' loops.
+__device__ __forceinline__ int lane_new()
+{
+    int l = lane_id();
+    asm volatile("" : "+v"(l));
+    return l;
+}
+
+template <int NT>
+struct Blk {
+    v4d re[NT], im[NT];
+};
+
+template <int NT>
+__device__ __forceinline__ void blk_zero(Blk<NT>& x)
+{
+#pragma unroll
+    for (int t = 0; t < NT; ++t) x.re[t] = x.im[t] = v4d{0, 0, 0, 0};
+}
+
+// Operands in memory: element (cm + lm, ck + lk) of a column-major matrix, of
+// its transpose, of its adjoint, and of Gamma^T = (i (S - S^+))^T.  cm, ck are
+// the same for all lanes and lm, lk for all uses, so the address is a scalar
+// base and one 32-bit lane offset (in LDS an immediate offset).
+template <class P>
+__device__ __forceinline__ C2 at(P p, int uni, int lane)
+{
+    return p[uni + lane];
+}
+template <>
+__device__ __forceinline__ C2 at<const C2*>(const C2* p, int uni, int lane)
+{
+    return *reinterpret_cast<const C2*>(reinterpret_cast<const char*>(p + uni) + (unsigned)(lane * 16));
+}
+struct LdN {
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const
+    {
+        return at(p, cm + ck * ld, lm + lk * ld);
+    }
+};
+struct LdT {
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const
+    {
+        return at(p, ck + cm * ld, lk + lm * ld);
+    }
+};
+struct LdC {
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const
+    {
+        const C2 v = at(p, ck + cm * ld, lk + lm * ld);
+        return make_double2(v.x, -v.y);
+    }
+};
+struct LdGamT {
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const
+    {
+        const C2 a = at(p, ck + cm * ld, lk + lm * ld), b = at(p, cm + ck * ld, lm + lk * ld);   // S[k][m], S[m][k]
+        return make_double2(-(a.y + b.y), a.x - b.x);
+    }
+};
+struct LdNc {           // conjugate
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const
+    {
+        const C2 v = at(p, cm + ck * ld, lm + lk * ld);
+        return make_double2(v.x, -v.y);
+    }
+};
+struct LdGam {          // Gamma
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const
+    {
+        const C2 a = at(p, cm + ck * ld, lm + lk * ld), b = at(p, ck + cm * ld, lk + lm * ld);   // S[m][k], S[k][m]
+        return make_double2(-(a.y + b.y), a.x - b.x);
+    }
+};
+struct LsN {            // the same in LDS
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const { return p[cm + ck * ld + lm + lk * ld]; }
+};
+struct LsT {
+    const C2* p;
+    int ld;
+    __device__ __forceinline__ C2 operator()(int cm, int ck, int lm, int lk) const { return p[ck + cm * ld + lk + lm * ld]; }
+};
+
+// this wave's number, known to be the same in all its lanes
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// columns 16 w .. 16 w + 15 of a matrix given by a loader
+template <int NT, class F>
+__device__ __forceinline__ void blk_load(Blk<NT>& x, F ld, int w)
+{
+    const int lane = lane_new(), l15 = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const C2 v = ld(16 * t + 4 * r, 16 * w, q, l15);
+            x.re[t][r] = v.x;
+            x.im[t][r] = v.y;
+        }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int NT>
+__device__ __forceinline__ void blk_store(const Blk<NT>& x, C2* p, int ld, int w)
+{
+    const int lane = lane_new(), l15 = lane & 15, q = lane >> 4;
+    const unsigned off = (unsigned)(q + l15 * ld) * 16;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<C2*>(reinterpret_cast<char*>(p + (16 * t + 4 * r + 16 * w * ld)) + off) =
+                make_double2(x.re[t][r], x.im[t][r]);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// y += A x; A by a loader, 16 NT square.  The A operands of a step are loaded
+// during the step before; the scheduling barrier keeps the compiler from
+// loading all of them first, which takes the registers of a second wave.
+// Bit NT i + t of mask is clear where A's rows 16 t .. 16 t + 15 are zero in
+// its columns 4 i .. 4 i + 3 (such a piece is neither loaded nor multiplied).
+template <int NT, bool MASK = false, class F>
+__device__ __forceinline__ void blk_mul(Blk<NT>& y, F A, const Blk<NT>& x, unsigned long long mask = ~0ull)
+{
+    const int lane = lane_new(), l15 = lane & 15, q = lane >> 4;
+    C2 a[2][NT];
+    auto on = [&](int i, int t) __attribute__((always_inline)) { return !MASK || ((mask >> (NT * i + t)) & 1); };
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        if (on(0, t)) a[0][t] = A(16 * t, 0, l15, q);
+#pragma unroll
+    for (int i = 0; i < 4 * NT; ++i) {
+        const int s = i / 4, r = i % 4, c = i & 1;
+        if (i + 1 < 4 * NT) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                if (on(i + 1, t)) a[c ^ 1][t] = A(16 * t, 4 * (i + 1), l15, q);
+        }
+        const double xr = x.re[s][r], xi = x.im[s][r];
+        if (MASK) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                if (on(i, t)) {
+                    y.re[t] = mfma16x16x4(a[c][t].x, xr, y.re[t]);
+                    y.im[t] = mfma16x16x4(a[c][t].x, xi, y.im[t]);
+                    y.re[t] = mfma16x16x4(-a[c][t].y, xi, y.re[t]);
+                    y.im[t] = mfma16x16x4(a[c][t].y, xr, y.im[t]);
+                }
+        } else {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                y.re[t] = mfma16x16x4(a[c][t].x, xr, y.re[t]);
+                y.im[t] = mfma16x16x4(a[c][t].x, xi, y.im[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                y.re[t] = mfma16x16x4(-a[c][t].y, xi, y.re[t]);
+                y.im[t] = mfma16x16x4(a[c][t].y, xr, y.im[t]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// y += A x where x's rows 4 i .. 4 i + 3 are zero unless bit NT i of mask is set
+template <int NT, class F>
+__device__ __forceinline__ void blk_mul_rows(Blk<NT>& y, F A, const Blk<NT>& x, unsigned long long mask)
+{
+    const int lane = lane_new(), l15 = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4 * NT; ++i) {
+        if (!((mask >> (NT * i)) & 1)) continue;
+        const int s = i / 4, r = i % 4;
+        C2 a[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) a[t] = A(16 * t, 4 * i, l15, q);
+        const double xr = x.re[s][r], xi = x.im[s][r];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            y.re[t] = mfma16x16x4(a[t].x, xr, y.re[t]);
+            y.im[t] = mfma16x16x4(a[t].x, xi, y.im[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            y.re[t] = mfma16x16x4(-a[t].y, xi, y.re[t]);
+            y.im[t] = mfma16x16x4(a[t].y, xr, y.im[t]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// ------------------------------------------------------------- LDS of a workgroup
+// One region holds either an inverse (column-major, ld = NP + 1: rows and
+// columns both read without bank conflicts) or, while a matrix is being
+// inverted in registers, two panels and one pivot-row buffer per wave.
+template <int NT>
+struct PlSmem {
+    static constexpr int NP = 16 * NT, LD = NP + 1;
+    static constexpr int MAT = NP * LD, WORK = 2 * 16 * LD + NT * 256;
+    C2 g[MAT > WORK ? MAT : WORK];
+    int piv[NP], cinv[NP], info;
+    double red[NT];
+};
+
+// running |A|, |A^-1| maxima of a wave's inverses
+struct Grow {
+    double a = 0.0, g = 0.0;
+};
+
+__device__ __forceinline__ double read_lane(double v, int lane)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | lo);
+}
+
+// largest of 64 lanes' values, in every lane
+__device__ __forceinline__ unsigned wave_max(unsigned v)
+{
+    auto step = [](unsigned x, unsigned y) { return x > y ? x : y; };
+    v = step(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));   // row_shr:1
+    v = step(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));   // row_shr:2
+    v = step(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));   // row_shr:4
+    v = step(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));   // row_shr:8
+    v = step(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));   // row_bcast:15
+    v = step(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));   // row_bcast:31
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Inverse of the matrix of 16 NT rows whose columns NT waves hold in m;
+// element (i, j) of it goes to out(i, j, value).  Blocked Gauss-Jordan with
+// partial pivoting, rows never exchanged: panel J is the 16 columns of wave J,
+// swept with one row per lane (two from 65 rows on; the pivot row reaches the
+// other lanes through scalar registers); the other waves then add panel x
+// pivot rows by MFMA.  The implicit exchanges are undone by the indexes of the
+// final store.  A pivot is the largest |re| + |im| of the free rows to 13 bits
+// (the first one of those).  Contains barriers: all waves call it.  work (2
+// panels of LD = 16 NT + 1 and 256 elements per wave) must be free, i.e. there
+// was a barrier since its last reader; a barrier ends the call.
+struct InvLds {
+    int *piv;          // pivot row of every column
+    int *cinv;         // column a row was the pivot of, or -1
+    int *info;         // first zero pivot (1-based) or -1 (NaN)
+};
+
+template <int NT, class Out>
+__device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m, Grow& gr, Out out)
+{
+    constexpr int NP = 16 * NT, LD = NP + 1, RPL = (NP + 63) / 64, KM = RPL > 1 ? 255 : 127;
+    const int lane = lane_new(), l15 = lane & 15, q = lane >> 4, w = wave_id();
+    if (threadIdx.x < NP) s.cinv[threadIdx.x] = -1;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) gr.a = fmax(gr.a, fabs(m.re[t][r]) + fabs(m.im[t][r]));
+    __syncthreads();
+    C2* pb = work + 2 * 16 * LD + w * 256;
+#pragma unroll 1
+    for (int J = 0; J < NT; ++J) {
+        C2* wb = work + (J & 1) * 16 * LD;
+        if (w == J) {
+            // columns -> rows
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    wb[l15 * LD + 16 * t + 4 * r + q] = make_double2(m.re[t][r], m.im[t][r]);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            double xr[RPL][16], xi[RPL][16];
+            bool free_row[RPL];
+            int row[RPL];
+#pragma unroll
+            for (int l = 0; l < RPL; ++l) {
+                row[l] = lane + 64 * l < NP ? lane + 64 * l : NP - 1;
+                free_row[l] = lane + 64 * l < NP && s.cinv[row[l]] < 0;
+#pragma unroll
+                for (int c = 0; c < 16; ++c) {
+                    const C2 v = wb[c * LD + row[l]];
+                    xr[l][c] = v.x;
+                    xi[l][c] = v.y;
+                }
+            }
+            // column c is always element 0: the columns move down by one per
+            // step and the finished one goes to the end, so the loop needs no
+            // register indexing
+#pragma unroll 1
+            for (int c = 0; c < 16; ++c) {
+                unsigned key = 0;
+#pragma unroll
+                for (int l = 0; l < RPL; ++l) {
+                    const unsigned hi =
+                        (unsigned)(__double_as_longlong(fabs(xr[l][0]) + fabs(xi[l][0])) >> 32);
+                    const unsigned k = free_row[l] ? ((hi & ~(unsigned)KM) | (unsigned)(64 * RPL - 64 * l - lane)) : 0u;
+                    key = k > key ? k : key;
+                }
+                const int p =
+                    __builtin_amdgcn_readfirstlane(64 * RPL - (int)(wave_max(key) & (unsigned)KM)), pl = p & 63;
+                // the step with the pivot row in slot SL of its lane
+                auto step = [&](auto slot) __attribute__((always_inline)) {
+                    constexpr int SL = decltype(slot)::value;
+                    const double dr = read_lane(xr[SL][0], pl), di = read_lane(xi[SL][0], pl);
+                    const double den = dr * dr + di * di;
+                    double vr = 0.0, vi = 0.0;      // 1 / pivot
+                    if (den != 0.0) {
+                        const double rc = 1.0 / den;
+                        vr = dr * rc;
+                        vi = -di * rc;
+                    }
+                    if (lane == 0) {
+                        s.piv[16 * J + c] = p;
+                        s.cinv[p] = 16 * J + c;
+                        if (!(den > 0.0) || den > 1.0e300) {
+                            if (*s.info == 0) *s.info = den == 0.0 ? 16 * J + c + 1 : -1;
+                        }
+                    }
+                    // multiplier f / pivot; the pivot row becomes row / pivot
+                    double gxr[RPL], gxi[RPL], keep[RPL];
+#pragma unroll
+                    for (int l = 0; l < RPL; ++l) {
+                        const bool own = l == SL && lane == pl;
+                        if (own) free_row[l] = false;
+                        const double fr = xr[l][0], fi = xi[l][0];
+                        gxr[l] = own ? -vr : fr * vr - fi * vi;
+                        gxi[l] = own ? -vi : fr * vi + fi * vr;
+                        keep[l] = own ? 0.0 : 1.0;
+                    }
+#pragma unroll
+                    for (int j = 1; j < 16; ++j) {
+                        const double pr = read_lane(xr[SL][j], pl), pim = read_lane(xi[SL][j], pl);
+#pragma unroll
+                        for (int l = 0; l < RPL; ++l) {
+                            const double a = l == SL ? xr[l][j] * keep[l] : xr[l][j];
+                            const double b = l == SL ? xi[l][j] * keep[l] : xi[l][j];
+                            xr[l][j - 1] = a - gxr[l] * pr + gxi[l] * pim;
+                            xi[l][j - 1] = b - gxr[l] * pim - gxi[l] * pr;
+                        }
+                    }
+#pragma unroll
+                    for (int l = 0; l < RPL; ++l) {
+                        xr[l][15] = -gxr[l];
+                        xi[l][15] = -gxi[l];
+                    }
+                };
+                if (RPL == 1 || p < 64) step(std::integral_constant<int, 0>{});
+                else step(std::integral_constant<int, RPL - 1>{});
+            }
+#pragma unroll
+            for (int l = 0; l < RPL; ++l)
+                if (lane + 64 * l < NP) {
+#pragma unroll
+                    for (int c = 0; c < 16; ++c) wb[c * LD + row[l]] = make_double2(xr[l][c], xi[l][c]);
+                }
+            // (a barrier in either branch: m is not live while its wave sweeps)
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const C2 v = wb[l15 * LD + 16 * t + 4 * r + q];
+                    m.re[t][r] = v.x;
+                    m.im[t][r] = v.y;
+                }
+        } else {
+            __syncthreads();
+            // the panel's pivot rows of this wave's columns, in pivot order;
+            // the rows themselves start from zero
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int k = s.cinv[16 * t + 4 * r + q] - 16 * J;
+                    if (k >= 0 && k < 16) {
+                        pb[k * 16 + l15] = make_double2(m.re[t][r], m.im[t][r]);
+                        m.re[t][r] = 0.0;
+                        m.im[t][r] = 0.0;
+                    }
+                }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const C2 pv = pb[(4 * r + q) * 16 + l15];
+                C2 a[NT];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) a[t] = wb[(4 * r + q) * LD + 16 * t + l15];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    m.re[t] = mfma16x16x4(a[t].x, pv.x, m.re[t]);
+                    m.im[t] = mfma16x16x4(a[t].x, pv.y, m.im[t]);
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    m.re[t] = mfma16x16x4(-a[t].y, pv.y, m.re[t]);
+                    m.im[t] = mfma16x16x4(a[t].y, pv.x, m.im[t]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    __syncthreads();
+    const int oc = s.piv[16 * w + l15];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            out(s.cinv[16 * t + 4 * r + q], oc, make_double2(m.re[t][r], m.im[t][r]));
+            gr.g = fmax(gr.g, fabs(m.re[t][r]) + fabs(m.im[t][r]));
+        }
+    __syncthreads();
+}
+
+// m = z - m on the n x n block, the identity on the padding
+template <int NT>
+__device__ __forceinline__ void blk_shift(Blk<NT>& m, double zr, double zi, int n, int w)
+{
+    const int lane = lane_new(), q = lane >> 4, col = 16 * w + (lane & 15);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * t + 4 * r + q;
+            const bool in = row < n && col < n, dg = row == col;
+            m.re[t][r] = in ? (dg ? zr : 0.0) - m.re[t][r] : (dg ? 1.0 : 0.0);
+            m.im[t][r] = in ? (dg ? zi : 0.0) - m.im[t][r] : 0.0;
+        }
+}
+
+// largest value over the workgroup, in every thread
+template <int NW>
+__device__ __forceinline__ double wg_max(double* red, double v)
+{
+#pragma unroll
+    for (int o = 32; o; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+    __syncthreads();
+    if (lane_id() == 0) red[wave_id()] = v;
+    __syncthreads();
+    double r = red[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) r = fmax(r, red[i]);
+    return r;
+}
+
+template <int NT>
+__device__ __forceinline__ double blk_maxabs(const Blk<NT>& x)
+{
+    double v = 0.0;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const double a = sqrt(x.re[t][r] * x.re[t][r] + x.im[t][r] * x.im[t][r]);
+            v = a > v || a != a ? (a != a ? INFINITY : a) : v;      // NaN never converges
+        }
+    return v;
+}
+
+// ------------------------------------------------------------------ decimation
+// Lopez-Sancho decimation (negf/surface.f90:479-497) of a lead cell whose
+// couplings run from its plane B (facing the device) to plane A of the next
+// cell: alpha = V^+ lives on A x B, beta = V on B x A, so of
+//   e += alpha g beta + beta g alpha, es += alpha g beta,
+//   alpha' = alpha g alpha, beta' = beta g beta
+// only the A and B blocks of e and g enter.  The planes between A and B are
+// eliminated once per point, two at a time; every step then inverts the cell
+// of two planes as one matrix, with pivots from both (inverting the planes one
+// after the other takes as many operations but lost 10 to 50 times the digits:
+// 1.8e-8 against 3.2e-10 at the 99th percentile of the ribbon's energies, the
+// full cell's inverse 2.7e-10).  The elements of alpha are the ones of the
+// full recursion, so the count of steps to max|alpha| <= convergence is too.
+// 2 NT waves: the first NT own the columns of A, the others those of B.
+constexpr int DEC_SLOTS = 19;       // matrices of NP^2 per item
+
+template <int NT>
+struct DecSmem {
+    static constexpr int NP2 = 32 * NT;
+    C2 work[2 * 16 * (NP2 + 1) + 2 * NT * 256];
+    int piv[NP2], cinv[NP2], info;
+    double red[2 * NT];
+};
+
+template <int NT>
+__global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
+{
+    constexpr int NP = 16 * NT, NN = NP * NP, NP2 = 2 * NP;
+    const PlanHdr& h = *a.h;
+    if (!h.ok || h.nt != NT) return;
+    __shared__ DecSmem<NT> s;
+    const InvLds il{s.piv, s.cinv, &s.info};
+    const int item = blockIdx.x, p = item >> 1, side = item & 1;
+    const int w = wave_id(), half = w >= NT, wc = half ? w - NT : w;
+    const int l15 = lane_id() & 15, q = lane_id() >> 4;
+    const int k = a.kidx ? a.kidx[p] : 0, M = h.M, mc = side ? h.m1 : h.m0;
+    const double E = a.E[p], et = a.eta_mode == NT_ETA_RELATIVE ? E * a.eta + a.eta0 : a.eta;
+    const double zr = E, zi = side ? et : -et;
+    // plane j of the cell counted from A; couplings j -> j + 1 and back
+    auto plane = [&](int j) { return side ? M - 1 - j : j; };
+    const C2* Hk = a.H + (long)k * M * NN;
+    const C2* Uk = a.U + (long)k * M * NN;
+    const C2* Lk = a.Lw + (long)k * M * NN;
+    auto Hp = [&](int j) { return Hk + (long)plane(j) * NN; };
+    auto Fp = [&](int j) { return side ? Lk + (long)(M - 2 - j) * NN : Uk + (long)j * NN; };
+    auto Bp = [&](int j) { return side ? Uk + (long)(M - 2 - j) * NN : Lk + (long)j * NN; };
+    const C2* V = a.LV + ((long)k * 2 + side) * NN;       // rows B, columns A
+    C2* sc = a.scratch + (long)item * DEC_SLOTS * NN;
+    auto slot = [&](int i) { return sc + (long)i * NN; };
+    C2 *eA = slot(0), *eB = slot(1), *esA = slot(2), *eB0 = slot(3), *al = slot(4), *be = slot(5), *aln = slot(6),
+       *ben = slot(7), *cf = slot(8), *cb = slot(9), *cfn = slot(10);
+    C2 *T1 = slot(11), *T2 = slot(13), *G = slot(15);     // NP x 2 NP twice, 2 NP square
+    C2* cbn = T1;                                         // (before the steps)
+    if (threadIdx.x == 0) s.info = 0;
+    Grow gr;
+    Blk<NT> x, y;
+    auto load = [&](Blk<NT>& b, const C2* m) __attribute__((always_inline)) { blk_load<NT>(b, LdN{m, NP}, wc); };
+    auto store = [&](const Blk<NT>& b, C2* m) __attribute__((always_inline)) { blk_store<NT>(b, m, NP, wc); };
+    auto copy = [&](C2* to, const C2* from) __attribute__((always_inline)) {
+        load(x, from);
+        store(x, to);
+    };
+    // G = (z - [[a, b], [c, d]])^-1 of planes of n1 and n2; no second plane
+    // where n2 = 0.  Wave w holds column 16 w + lane % 16 of the 2 NP.
+    auto invert = [&](const C2* ma, const C2* mb, const C2* mcc, const C2* md, int n1, int n2) __attribute__((always_inline)) {
+        Blk<2 * NT> m;
+        {
+            Blk<NT> u, v;
+            load(u, half ? mb : ma);
+            load(v, half ? md : mcc);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) m.re[t] = u.re[t], m.im[t] = u.im[t], m.re[NT + t] = v.re[t], m.im[NT + t] = v.im[t];
+        }
+        const int lane = lane_new(), q = lane >> 4, c0 = 16 * wc + (lane & 15);
+        const bool cin = c0 < (half ? n2 : n1);
+#pragma unroll
+        for (int t = 0; t < 2 * NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int r0 = 16 * (t % NT) + 4 * r + q;
+                const bool in = cin && r0 < (t < NT ? n1 : n2), dg = (t >= NT) == (half != 0) && r0 == c0;
+                m.re[t][r] = in ? (dg ? zr : 0.0) - m.re[t][r] : (dg ? 1.0 : 0.0);
+                m.im[t][r] = in ? (dg ? zi : 0.0) - m.im[t][r] : 0.0;
+            }
+        __syncthreads();
+        wg_inverse<2 * NT>(s.work, il, m, gr, [&](int i, int j, C2 v) { G[i + j * NP2] = v; });
+    };
+    const C2 *G11 = G, *G21 = G + NP, *G12 = G + (long)NP * NP2, *G22 = G + NP + (long)NP * NP2;
+    const int nA = a.psize[plane(0)], nB = a.psize[plane(mc - 1)];
+    // alpha0 = V^+, beta0 = V
+    blk_load<NT>(x, LdC{V, NP}, wc);
+    store(x, al);
+    double amax = blk_maxabs<NT>(x);
+    copy(be, V);
+    copy(eA, Hp(0));
+    double scale = fmax(amax, blk_maxabs<NT>(x));
+    copy(cf, Fp(0));
+    copy(cb, Bp(0));
+    copy(eB, Hp(1));
+    __syncthreads();
+    // One inverse per pass: the elimination of planes j (and j + 1) between A
+    // and B (cf = A -> j, cb = j -> A) while there are any, then the steps,
+    // then the last one with es (one copy of the inverse's code, and the
+    // registers of one).
+    int it = 0, j = 1, mode = mc > 2 ? 0 : 1;
+    auto steps_begin = [&]() __attribute__((always_inline)) {
+        if (cbn != T1) {              // T1's slot is needed by the steps
+            copy(cbn, cb);
+            cb = cbn;
+        }
+        copy(eB0, eB);
+        copy(esA, eA);
+        amax = wg_max<2 * NT>(s.red, half ? 0.0 : amax);      // its barriers also publish the slots
+    };
+    if (mode) steps_begin();
+    for (;;) {
+        if (mode == 1 && !(it < a.max_iter && amax > a.conv && s.info == 0)) mode = 2;
+        const bool two = j + 2 < mc;
+        const C2 *ma = mode == 0 ? eB : mode == 1 ? eA : esA, *mb = mode ? cf : two ? Fp(j) : eB,
+                 *mcc = mode ? cb : two ? Bp(j) : eB, *md = mode == 0 ? (two ? Hp(j + 1) : eB) : mode == 1 ? eB : eB0;
+        const int n1 = mode ? nA : a.psize[plane(j)], n2 = mode ? nB : two ? a.psize[plane(j + 1)] : 0;
+        invert(ma, mb, mcc, md, n1, n2);
+        if (mode == 2) break;
+        if (mode == 0) {
+            const int o = two ? j + 1 : j;
+            // half 0, through A:  e_AA += cf (g cb),  cb' = B_o (g cb)
+            // half 1, onward:     cf' = cf (g F_o),   e = H_{o + 1} + B_o (g F_o)
+            Blk<NT> u;
+            load(x, half ? Fp(o) : cb);
+            blk_zero<NT>(y);
+            blk_mul<NT>(y, LdN{half && two ? G12 : G11, NP2}, x);
+            if (half) blk_zero<NT>(u);
+            else load(u, eA);
+            blk_mul<NT>(u, LdN{cf, NP}, y);
+            store(u, half ? cfn : eA);
+            blk_zero<NT>(y);
+            blk_mul<NT>(y, LdN{two ? (half ? G22 : G21) : G11, NP2}, x);
+            if (half) load(u, Hp(o + 1));
+            else blk_zero<NT>(u);
+            blk_mul<NT>(u, LdN{Bp(o), NP}, y);
+            store(u, half ? eB : cbn);
+            C2* v = cf;
+            cf = cfn;
+            cfn = v;
+            v = cb;
+            cb = cbn;
+            cbn = v;
+            __syncthreads();
+            j = o + 1;
+            if (j + 1 >= mc) {
+                mode = 1;
+                steps_begin();
+            }
+            continue;
+        }
+        // T1 = alpha [g_BA, g_BB], T2 = beta [g_AA, g_AB]
+        blk_load<NT>(x, LdN{G21, NP2}, w);
+        blk_zero<NT>(y);
+        blk_mul<NT>(y, LdN{al, NP}, x);
+        blk_store<NT>(y, T1, NP, w);
+        blk_load<NT>(x, LdN{G11, NP2}, w);
+        blk_zero<NT>(y);
+        blk_mul<NT>(y, LdN{be, NP}, x);
+        blk_store<NT>(y, T2, NP, w);
+        __syncthreads();
+        // half 0: alpha g_BB beta to es and e_AA, alpha' = alpha g_BA alpha
+        // half 1: beta g_AA alpha to e_BB, beta' = beta g_AB beta
+        load(x, half ? al : be);
+        blk_zero<NT>(y);
+        blk_mul<NT>(y, LdN{half ? T2 : T1 + (long)NN, NP}, x);
+        if (!half) {
+            load(x, esA);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) x.re[t] += y.re[t], x.im[t] += y.im[t];
+            store(x, esA);
+        }
+        load(x, half ? eB : eA);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) x.re[t] += y.re[t], x.im[t] += y.im[t];
+        store(x, half ? eB : eA);
+        load(x, half ? be : al);
+        blk_zero<NT>(y);
+        blk_mul<NT>(y, LdN{half ? T2 + (long)NN : T1, NP}, x);
+        store(y, half ? ben : aln);
+        C2* sw = al;
+        al = aln;
+        aln = sw;
+        sw = be;
+        be = ben;
+        ben = sw;
+        ++it;
+        amax = wg_max<2 * NT>(s.red, half ? 0.0 : blk_maxabs<NT>(y));
+    }
+    const int not_conv = amax > a.conv;
+    // Sigma = V^+ g_BB V on A with g = (z - es)^-1
+    if (!half) {
+        load(x, V);
+        blk_zero<NT>(y);
+        blk_mul<NT>(y, LdN{G22, NP2}, x);
+        blk_zero<NT>(x);
+        blk_mul<NT>(x, LdC{V, NP}, y);
+        C2* out = a.sigma + (long)item * NN;
+        if (side) {
+            store(x, out);
+        } else {
+            // retarded = adjoint of the advanced
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    out[16 * wc + l15 + (16 * t + 4 * r + q) * NP] = make_double2(x.re[t][r], -x.im[t][r]);
+        }
+    }
+    const double ga = wg_max<2 * NT>(s.red, gr.a), gg = wg_max<2 * NT>(s.red, gr.g);
+    scale = fmax(wg_max<2 * NT>(s.red, scale), fabs(E));
+    if (threadIdx.x == 0) {
+        const double rb = 1.0e-7 * scale / fabs(et);
+        a.iters[item] = it;
+        a.status[item] = s.info ? s.info : not_conv ? NT_ERR_NOT_CONVERGED : 0;
+        a.grow[item] = ga * gg * rb * rb;      // (eta = 0: not finite, left to the layers)
+    }
+}
+
+// ----------------------------------------------------------------------- sweep
+// One direction of one point: system 0 left to right (left lead planes at the
+// lead's broadening, everything else at the device's), system 1 right to left
+// (the roles swapped), negf/lesser.f90:556-793 on the planes.  Step i:
+//   A = z_i - H_i - L X,  X = G U            (U, L: couplings to and from step i)
+//   G = A^-1                                  in LDS
+//   R = G_{first,i}^T = G^T (U^T R)           in registers
+// and at the end T = Re Tr[(R^T Gamma_e)(R^* Gamma_s)].
+template <int NT>
+__global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArgs a)
+{
+    constexpr int NP = 16 * NT, LD = NP + 1, NN = NP * NP;
+    const PlanHdr& h = *a.h;
+    if (!h.ok || h.nt != NT) return;
+    __shared__ PlSmem<NT> s;
+    const InvLds il{s.piv, s.cinv, &s.info};
+    const int item = blockIdx.x, p = item >> 1, sys = item & 1;
+    const int w = wave_id();
+    const int k = a.kidx ? a.kidx[p] : 0, M = h.M;
+    const double E = a.E[p], et = a.eta_mode == NT_ETA_RELATIVE ? E * a.eta + a.eta0 : a.eta;
+    if (a.need[p]) return;
+    const int lead_planes = sys ? h.m1 : h.m0;
+    const C2* Hk = a.H + (long)k * M * NN;
+    const C2* Uk = a.U + (long)k * M * NN;
+    const C2* Lk = a.Lw + (long)k * M * NN;
+    // self-energies of the starting and of the closing lead
+    const C2* Ss = a.sigma + (long)(2 * p + sys) * NN;
+    const C2* Se = a.sigma + (long)(2 * p + 1 - sys) * NN;
+    if (threadIdx.x == 0) s.info = 0;
+    Grow gr;
+    Blk<NT> R;
+    blk_zero<NT>(R);
+#pragma unroll 1
+    for (int i = 0; i < M; ++i) {
+        const int j = sys ? M - 1 - i : i;
+        Blk<NT> m;
+        blk_load<NT>(m, LdN{Hk + (long)j * NN, NP}, w);
+        if (i == 0 || i == M - 1) {
+            Blk<NT> sg;
+            blk_load<NT>(sg, LdN{i ? Se : Ss, NP}, w);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) m.re[t] += sg.re[t], m.im[t] += sg.im[t];
+        }
+        if (i) {
+            const C2* U = sys ? Lk + (long)j * NN : Uk + (long)(j - 1) * NN;      // step i - 1 -> i
+            const C2* Lo = sys ? Uk + (long)j * NN : Lk + (long)(j - 1) * NN;     // step i -> i - 1
+            // masks of U's 4 x 16 pieces and of Lo's 16 x 4 pieces
+            const unsigned long long* mk = a.masks + ((long)k * M + (sys ? j : j - 1)) * 4;
+            const unsigned long long mu = mk[sys ? 2 : 0], ml = mk[sys ? 1 : 3];
+            Blk<NT> t2;
+            blk_zero<NT>(t2);
+            blk_mul<NT, true>(t2, LdT{U, NP}, R, mu);
+            R = t2;
+            blk_load<NT>(t2, LdN{U, NP}, w);
+            Blk<NT> X;
+            blk_zero<NT>(X);
+            blk_mul_rows<NT>(X, LsN{s.g, LD}, t2, mu >> w);
+            blk_mul<NT, true>(m, LdN{Lo, NP}, X, ml);
+        }
+        blk_shift<NT>(m, E, i < lead_planes ? et : a.dev_factor * et, a.psize[j], w);
+        __syncthreads();
+        wg_inverse<NT>(s.g, il, m, gr, [&](int r, int c, C2 v) { s.g[r + c * LD] = v; });
+        if (i) {
+            Blk<NT> n;
+            blk_zero<NT>(n);
+            blk_mul<NT>(n, LsT{s.g, LD}, R);
+            R = n;
+        } else {
+            blk_load<NT>(R, LsT{s.g, LD}, w);
+        }
+        if (a.keep && !sys && j >= *a.keep_from) {
+            C2* kp = a.keep + (p * a.keep_stride + 2 * (j - *a.keep_from)) * NN;
+            Blk<NT> g;
+            blk_load<NT>(g, LsN{s.g, LD}, w);
+            blk_store<NT>(g, kp, NP, w);
+            blk_store<NT>(R, kp + NN, NP, w);
+        }
+    }
+    // Y^T = Gamma_e^T R into LDS, Q = Y^T Gamma_s^T, T = Re sum conj(R) Q
+    Blk<NT> y;
+    blk_zero<NT>(y);
+    blk_mul<NT>(y, LdGamT{Se, NP}, R);
+    __syncthreads();
+    blk_store<NT>(y, s.g, LD, w);
+    Blk<NT> g;
+    blk_load<NT>(g, LdGamT{Ss, NP}, w);
+    __syncthreads();
+    blk_zero<NT>(y);
+    blk_mul<NT>(y, LsN{s.g, LD}, g);
+    double tr = 0.0;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tr += R.re[t][r] * y.re[t][r] + R.im[t][r] * y.im[t][r];
+#pragma unroll
+    for (int o = 32; o; o >>= 1) tr += __shfl_xor(tr, o);
+    __syncthreads();
+    if (lane_id() == 0) s.red[w] = tr;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int i = 0; i < NT; ++i) t += s.red[i];
+        a.T[item] = t;
+        a.status[item] = s.info;
+    }
+}
+
+// --------------------------------------------------------------------- adjoint
+// Column and row of the full Green's function on the window's planes, one
+// workgroup per point, from the left-connected blocks the sweep kept:
+//   C_j = G^L_j U_j C_{j+1},  R_j^T = (G^L_{0,j})^T + (G^L_j)^T L_j^T R_{j+1}^T
+// from C_{M-1} = G_{M-1,M-1} A, A = w Gamma_R G_{0,M-1}^+ Gamma_L, so that
+// X_{j,i} = C_j R_i (the block path's adjoint_backward).  No LDS and no
+// barrier: every wave works on its own columns, all A operands are read from
+// memory.  The window's blocks are written in the layers' own order, the rows
+// of R of all points above one another and the columns of C beside one
+// another: the sums over the points of X_{j,i}^+ = R_i^+ C_j^+ are then one
+// product per layer and k-point, over 16 NT rows per point instead of a b x b
+// block of each point summed afterwards.
+template <int NT>
+__global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
+{
+    constexpr int NP = 16 * NT, NN = NP * NP;
+    const PlanHdr& h = *a.h;
+    if (!h.ok || h.nt != NT) return;
+    const int p = blockIdx.x, w = wave_id(), M = h.M;
+    const int k = a.kidx ? a.kidx[p] : 0;
+    const C2* Uk = a.U + (long)k * M * NN;
+    const C2* Lk = a.Lw + (long)k * M * NN;
+    const int jw = a.poff[a.lo + 1], je = a.poff[a.hi1 + 2];       // the window's planes
+    const C2* keep = a.keep + (long)p * a.keep_stride * NN;
+    auto gl = [&](int j) { return keep + 2L * (j - jw) * NN; };
+    auto g0 = [&](int j) { return keep + (2L * (j - jw) + 1) * NN; };
+    const bool on = !a.need[p] && !a.status[2 * p] && !a.status[2 * p + 1] && !a.dstatus[2 * p] &&
+                    !a.dstatus[2 * p + 1] && !(a.first && a.first[p]);
+    const C2* Ss = a.sigma + (long)(2 * p) * NN;
+    const C2* Se = Ss + NN;
+    Blk<NT> C, R, y;
+    blk_zero<NT>(C);
+    blk_zero<NT>(R);
+    if (on) {
+        blk_load<NT>(y, LdGam{Ss, NP}, w);
+        blk_mul<NT>(R, LdNc{g0(M - 1), NP}, y);
+        blk_zero<NT>(y);
+        blk_mul<NT>(y, LdGam{Se, NP}, R);
+        const double f = a.w[p];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) y.re[t] *= f, y.im[t] *= f;
+        blk_mul<NT>(C, LdN{gl(M - 1), NP}, y);
+        blk_load<NT>(R, LdN{g0(M - 1), NP}, w);
+    }
+    const int place = a.place ? a.place[p] : p;
+    // rows of a point: its place among the points, NP each
+#pragma unroll 1
+    for (int j = M - 2; j >= jw; --j) {
+        if (on) {
+            blk_zero<NT>(y);
+            const unsigned long long* mk = a.masks + ((long)k * M + j) * 4;
+            blk_mul<NT, true>(y, LdN{Uk + (long)j * NN, NP}, C, mk[1]);
+            blk_zero<NT>(C);
+            blk_mul<NT>(C, LdN{gl(j), NP}, y);
+            blk_zero<NT>(y);
+            blk_mul<NT, true>(y, LdT{Lk + (long)j * NN, NP}, R, mk[2]);
+            blk_load<NT>(R, LdN{g0(j), NP}, w);
+            blk_mul<NT>(R, LdT{gl(j), NP}, y);
+        }
+        if (j < je) {
+            const int lane = lane_new(), q = lane >> 4, n = a.psize[j], l = a.player[j] - 1 - a.lo;
+            const long cc = (long)place * NP + 16 * w + (lane & 15);
+            C2* CA = a.CA + l * a.K * a.b + cc * a.b;
+            C2* RW = a.RW + l * a.K * a.b + cc;
+            const int* pm = a.perm + (long)j * 64;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 16 * t + 4 * r + q;
+                    if (row < n) {
+                        const int d = pm[row];
+                        CA[d] = make_double2(C.re[t][r], C.im[t][r]);
+                        RW[d * a.K] = make_double2(R.re[t][r], R.im[t][r]);
+                    }
+                }
+        }
+    }
+}
+
+// need[p]: the point is left to the layers (plan refused, a singular plane of
+// a lead, a value not finite, too much growth); *count: how many are
+__global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const double* grow, int* need, int* count)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= P) return;
+    bool bad = !h->ok;
+    if (!bad)
+        for (int i = 0; i < 2; ++i) {
+            const int d = dst[2 * p + i];
+            bad = bad || (d != 0 && d != NT_ERR_NOT_CONVERGED) || (d == 0 && !(grow[2 * p + i] <= PL_GROWTH));
+        }
+    need[p] = bad;
+    if (bad) atomicAdd(count, 1);
+}
+
+// Points solved on the planes: statuses, iteration counts, clamps.  A singular
+// plane in the sweep sets need[p] too (counted in count[1]); count[2] sums the
+// decimation steps.
+__global__ void k_pl_finish(int P, const int* dst, const int* dit, const int* sst, const double* T,
+                            const int* first_mask, int* need, int* count, double* T_LR, double* T_RL, int* status,
+                            int* iters)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= P || need[p]) return;
+    if (sst[2 * p] || sst[2 * p + 1]) {
+        need[p] = 2;
+        atomicAdd(count + 1, 1);
+        return;
+    }
+    atomicAdd(count + 2, dit[2 * p] + dit[2 * p + 1]);
+    double tl = T[2 * p], tr = T[2 * p + 1];
+    if (tl < 1.0e-60) tl = 0.0;       // negf/lesser.f90:795-800
+    if (tr < 1.0e-60) tr = 0.0;
+    if (first_mask && first_mask[p]) tl = tr = 0.0;      // negf/lesser.f90:802-807
+    T_LR[p] = tl;
+    T_RL[p] = tr;
+    if (status) status[p] = dst[2 * p] ? dst[2 * p] : dst[2 * p + 1];
+    if (iters) iters[p] = (dit[2 * p] + dit[2 * p + 1] + 1) / 2;
+}
+
+// the points with need[p] == which, in order, at most `most` of them: their
+// indexes and inputs.  One workgroup.
+__global__ __launch_bounds__(1024) void k_pl_gather(int P, const int* need, int which, int most, const double* E,
+                                                    const int* kidx, const int* first, int* idx, double* gE, int* gk,
+                                                    int* gf, const double* wt, double* gw)
+{
+    __shared__ int wsum[16];
+    int base = 0;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int p0 = 0; p0 < P; p0 += 1024) {
+        const int p = p0 + threadIdx.x;
+        const bool on = p < P && need[p] == which;
+        const unsigned long long m = __ballot(on);
+        if (lane == 0) wsum[w] = __popcll(m);
+        __syncthreads();
+        int off = base, all = 0;
+        for (int i = 0; i < 16; ++i) {
+            if (i < w) off += wsum[i];
+            all += wsum[i];
+        }
+        const int o = off + __popcll(m & ((1ull << lane) - 1));
+        if (on && o < most) {
+            idx[o] = p;
+            gE[o] = E[p];
+            if (kidx) gk[o] = kidx[p];
+            if (first) gf[o] = first[p];
+            if (wt) gw[o] = wt[p];
+        }
+        base += all;
+        __syncthreads();
+    }
+}
+
+__global__ void k_pl_scatter(int n, const int* idx, const double* Tl, const double* Tr, const int* st, const int* it,
+                             double* T_LR, double* T_RL, int* status, int* iters)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int p = idx[i];
+    T_LR[p] = Tl[i];
+    T_RL[p] = Tr[i];
+    if (status) status[p] = st[i];
+    if (iters) iters[p] = it[i];
+}
+
+}  // namespace
+
+namespace {
+
+void ensure_plan_buf(nt_ctx* c, size_t bytes)
+{
+    if (c->plan_bytes >= bytes) return;
+    if (c->plan_buf) {
+        hipcheck(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        unreg_region(c, c->plan_buf);
+        hipcheck(c, hipFree(c->plan_buf), "hipFree");
+        c->plan_buf = nullptr;
+        c->plan_bytes = 0;
+    }
+    hipcheck(c, hipMalloc(&c->plan_buf, bytes), "hipMalloc plan");
+    c->plan_bytes = bytes;
+    reg_region(c, c->plan_buf, bytes);
+}
+
+// gathered inputs and results of the points left to the layers
+void ensure_left_buf(nt_ctx* w, size_t bytes)
+{
+    if (w->left_bytes >= bytes) return;
+    if (w->left_buf) {
+        hipcheck(w, hipStreamSynchronize(w->stream), "hipStreamSynchronize");
+        unreg_region(w, w->left_buf);
+        hipcheck(w, hipFree(w->left_buf), "hipFree");
+        w->left_buf = nullptr;
+        w->left_bytes = 0;
+    }
+    hipcheck(w, hipMalloc(&w->left_buf, 2 * bytes), "hipMalloc points");
+    w->left_bytes = 2 * bytes;
+}
+
+// per point of a chunk: the two leads' decimation slots and self-energies,
+// statuses, counts, growth, T of both directions
+struct ChunkView {
+    C2 *scratch, *sigma;
+    int *dst, *dit, *sst;
+    double *dgrow, *T;
+    C2 *keep = nullptr, *CA = nullptr, *RW = nullptr;      // adjoint
+    int* place = nullptr;
+};
+
+ChunkView chunk_carve(Arena& a, int P, int NN)
+{
+    const size_t it = 2 * (size_t)P;
+    ChunkView v;
+    v.scratch = a.ptr<C2>(a.take(sizeof(C2) * it * DEC_SLOTS * NN));
+    v.sigma = a.ptr<C2>(a.take(sizeof(C2) * it * NN));
+    v.dst = a.ptr<int>(a.take(sizeof(int) * it));
+    v.dit = a.ptr<int>(a.take(sizeof(int) * it));
+    v.sst = a.ptr<int>(a.take(sizeof(int) * it));
+    v.dgrow = a.ptr<double>(a.take(sizeof(double) * it));
+    v.T = a.ptr<double>(a.take(sizeof(double) * it));
+    return v;
+}
+
+// bytes a chunk of points may take
+constexpr double PL_CHUNK_BYTES = 6.0 * 1024 * 1024 * 1024;
+constexpr double PL_ADJ_BYTES = 24.0 * 1024 * 1024 * 1024;
+constexpr int PL_MAX_ITER = 20000;      // decimation steps inside one kernel
+
+template <int NT>
+void launch_adjoint(const AdjPlArgs& a, int n, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_pl_adjoint<NT>, dim3(n), dim3(64 * NT), 0, s, a);
+}
+
+// Gradients of one chunk's points, added to a's dHd and dHdv.
+void planes_adjoint(nt_ctx* c, const TdbArgs& a, const PlanDims& d, const PlanView& v, const PlanHdr& h,
+                    const ChunkView& cv, const C2* pU, const C2* pL, const unsigned long long* pM, int p0, int n, const std::vector<int>& hk,
+                    const int* need, long kept, int hi1)
+{
+    typedef double T;
+    hipStream_t s = c->stream;
+    const int NP = 16 * h.nt, b = a.b, lo = a.adj_lo, hi = a.adj_hi, nw = hi - lo + 1, hc = std::min(hi, a.L - 2),
+              nc = hc - lo + 1;
+    const long K = (long)n * NP;
+    // points of one k-point stand together
+    std::vector<int> place, k0(a.nk + 1, 0);
+    if (a.nk > 1) {
+        for (int i = 0; i < n; ++i) ++k0[hk[p0 + i] + 1];
+        for (int k = 0; k < a.nk; ++k) k0[k + 1] += k0[k];
+        std::vector<int> at(k0.begin(), k0.end() - 1);
+        place.resize(n);
+        for (int i = 0; i < n; ++i) place[i] = at[hk[p0 + i]]++;
+        hipcheck(c, hipMemcpyAsync(cv.place, place.data(), sizeof(int) * n, hipMemcpyHostToDevice, s), "H2D");
+        hipcheck(c, hipStreamSynchronize(s), "sync");
+    } else {
+        k0[1] = n;
+    }
+    const AdjPlArgs aa{v.h, v.psize, v.player, v.poff, v.perm, pU, pL, pM, cv.sigma, cv.keep, kept,
+                       a.kidx ? a.kidx + p0 : nullptr, need, cv.sst, cv.dst, a.first_mask ? a.first_mask + p0 : nullptr,
+                       a.adj_w + p0, a.nk > 1 ? cv.place : nullptr, lo, hi1, b, K, cv.CA, cv.RW};
+    check_range(c, a.adj_w + p0, sizeof(double) * n, "adjoint weights");
+    const double m = NP;
+    launch(c, NT_K_PLANES, 4.0 * 8 * m * m * m * n * (kept / 2), "plane adjoint", [&] {
+        if (h.nt == 1) launch_adjoint<1>(aa, n, s);
+        if (h.nt == 2) launch_adjoint<2>(aa, n, s);
+        if (h.nt == 3) launch_adjoint<3>(aa, n, s);
+        if (h.nt == 4) launch_adjoint<4>(aa, n, s);
+        return hipGetLastError();
+    });
+    // dHd_l += 2 sum_p R_l^+ C_l^+, dHdv_l += 2 sum_p (R_l^+ C_{l+1}^+ + C_l R_{l+1}),
+    // one launch for all layers of the window
+    const long bb = (long)b * b, per = K * b;
+    const T* CA = reinterpret_cast<const T*>(cv.CA);
+    const T* RW = reinterpret_cast<const T*>(cv.RW);
+    for (int k = 0; k < a.nk; ++k) {
+        const long q0 = (long)k0[k] * NP;
+        const int Kk = (k0[k + 1] - k0[k]) * NP;
+        if (!Kk) continue;
+        const BMat<T> Rm = bm<T>(RW + 2 * q0, per, (int)K), Cm = bm<T>(CA + 2 * q0 * b, per, b);
+        const BMat<T> Rn = bm<T>(RW + 2 * (per + q0), per, (int)K), Cn = bm<T>(CA + 2 * (per + q0 * b), per, b);
+        T* gd = reinterpret_cast<T*>(a.dHd) + 2 * (long)k * nw * bb;
+        gemm<T>(c, b, b, Kk, OP_C, Rm, OP_C, Cm, bw(gd, bb, b), 2.0, bm<T>(gd, bb, b), 1.0, nullptr, nw);
+        if (nc > 0 && a.dHdv) {
+            T* gv = reinterpret_cast<T*>(a.dHdv) + 2 * (long)k * nc * bb;
+            gemm<T>(c, b, b, Kk, OP_C, Rm, OP_C, Cn, bw(gv, bb, b), 2.0, bm<T>(gv, bb, b), 1.0, nullptr, nc);
+            gemm<T>(c, b, b, Kk, OP_N, Cm, OP_N, Rn, bw(gv, bb, b), 2.0, bm<T>(gv, bb, b), 1.0, nullptr, nc);
+        }
+    }
+    (void)d;
+}
+
+template <int NT>
+void launch_decimate(const DecPlArgs& a, int items, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_pl_decimate<NT>, dim3(items), dim3(128 * NT), 0, s, a);
+}
+template <int NT>
+void launch_sweep(const SweepPlArgs& a, int items, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_pl_sweep<NT>, dim3(items), dim3(64 * NT), 0, s, a);
+}
+
+}  // namespace
+
+// The n points of a's points [p0, p0 + P) with need == which, on the layers.
+// beside: on a worker context, from where c's stream stands at chk[0] (the
+// decimation's end) on, c's stream waiting for it; else on c's stream.
+static void solve_left(nt_ctx* c, const nt_params* prm, const TdbArgs& a, int p0, int P, const int* need, int which,
+                       int n, bool beside)
+{
+    nt_ctx* w = c;
+    if (beside) {
+        if (const int st = prepare_workers(c, 1)) {
+            c->err = "could not set up a worker context";
+            throw Fail{st};
+        }
+        w = c->subs[0];
+        hipcheck(c, hipStreamWaitEvent(w->stream, c->chk[0], 0), "wait check");
+    }
+    const size_t nd = sizeof(double) * n, ni = sizeof(int) * n;
+    hipStream_t s = w->stream;
+    TdbArgs g = a;
+    g.no_planes = true;
+    g.siblings.clear();
+    Arena la;
+    const size_t oi = la.take(ni), oe = la.take(nd), ok = la.take(ni), of = la.take(ni), ol = la.take(nd),
+                 orr = la.take(nd), os = la.take(ni), ot = la.take(ni), ow = la.take(nd);
+    ensure_left_buf(w, la.off);
+    la.base = static_cast<char*>(w->left_buf);
+    int *idx = la.ptr<int>(oi), *gk = la.ptr<int>(ok), *gf = la.ptr<int>(of);
+    double* gE = la.ptr<double>(oe);
+    hipLaunchKernelGGL(k_pl_gather, dim3(1), dim3(1024), 0, s, P, need, which, n, a.E + p0,
+                       a.kidx ? a.kidx + p0 : nullptr, a.first_mask ? a.first_mask + p0 : nullptr, idx, gE, gk, gf,
+                       a.adj_w ? a.adj_w + p0 : nullptr, la.ptr<double>(ow));
+    hipcheck(w, hipGetLastError(), "gather");
+    if (a.adj_w) g.adj_w = la.ptr<double>(ow);
+    g.npts = n;
+    g.E = gE;
+    g.kidx = a.kidx ? gk : nullptr;
+    g.first_mask = a.first_mask ? gf : nullptr;
+    g.T_LR = la.ptr<double>(ol);
+    g.T_RL = la.ptr<double>(orr);
+    g.status = la.ptr<int>(os);
+    g.iters = la.ptr<int>(ot);
+    if (w != c) {
+        w->regions = c->regions;
+        if (w->ws) reg_region(w, w->ws, w->ws_bytes);
+    }
+    reg_region(w, w->left_buf, w->left_bytes);
+    try {
+        solve_tdb_dev(w, prm, g);
+    } catch (const Fail&) {
+        if (w != c) c->err = w->err;
+        throw;
+    }
+    if (w != c) {
+        hipcheck(c, hipEventRecord(w->join, s), "event join");
+        hipcheck(c, hipStreamWaitEvent(c->stream, w->join, 0), "wait join");
+        if (w->prof) harvest_profile(w);
+        for (int k = 0; k < NT_K_COUNT; ++k) {
+            c->launches[k] += w->launches[k];
+            c->ms[k] += w->ms[k];
+            c->flops[k] += w->flops[k];
+            w->launches[k] = 0;
+            w->ms[k] = 0;
+            w->flops[k] = 0;
+        }
+    }
+    hipLaunchKernelGGL(k_pl_scatter, dim3(nblk(n)), dim3(256), 0, c->stream, n, idx, g.T_LR, g.T_RL, g.status, g.iters,
+                       a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr, a.iters ? a.iters + p0 : nullptr);
+    hipcheck(c, hipGetLastError(), "scatter");
+}
+
+bool planes_candidate(const nt_ctx* c, const nt_params* prm, const TdbArgs& a)
+{
+    const nt_solve_extras& x = a.ex;
+    const bool extras = x.gl_adv || x.gr_ret || x.gl_plus || x.gr_minus || x.gml_adv || x.gmr_ret || x.sl_adv ||
+                        x.sr_ret || x.G_D_LR || x.G_D_RL || x.G_L || x.G_R || x.sdos_l || x.sdos_r || x.ldos ||
+                        x.ddos;
+    // (an adjoint solve needs the plan's sizes on the host)
+    return c->planes && !a.no_planes && !a.mask && !(a.adj_w && c->dec_check == 0) && !a.probe && !extras &&
+           !(prm->circular && prm->n_bloch_x * prm->n_bloch_y > 1) && c->one_sweep && !c->gemm_m3 &&
+           prm->max_iter <= PL_MAX_ITER && a.nk <= 65535 && 2 * a.L + 5 <= 65535;
+}
+
+// Solve a's points on their planes.  False: the blocks do not fall into planes
+// of at most 64 (nothing was written).  Points the planes are no good for (a
+// singular plane, growth) are solved by the block path before it returns.
+bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
+{
+    const bool wait = c->dec_check > 0;        // the host may wait for the device
+    const PlanDims d = plan_dims(a.nl, a.nr, a.b, a.L, a.nk);
+    hipStream_t s = c->stream;
+    // the plan, the mask of points left to the block path, the counters
+    Arena pa;
+    plan_carve(pa, d);
+    const size_t o_need = pa.take(sizeof(int) * (size_t)a.npts), o_cnt = pa.take(sizeof(int) * 4);
+    const size_t plan_need = pa.off;
+    size_t scratch_bytes = 0;
+    char* scratch = static_cast<char*>(scratch_region(c->device, &scratch_bytes));
+    size_t reserve = 0;
+    if (a.noalloc) {
+        // at the end of the static scratch, which the block path then keeps off
+        reserve = (plan_need + 4095) / 4096 * 4096;
+        if (!scratch || 2 * reserve > scratch_bytes) return false;
+        pa = Arena();
+        pa.base = scratch + (scratch_bytes - reserve);
+    } else {
+        ensure_plan_buf(c, plan_need);
+        pa = Arena();
+        pa.base = static_cast<char*>(c->plan_buf);
+    }
+    const PlanView v = plan_carve(pa, d);
+    int* need = pa.ptr<int>(o_need);
+    int* cnt = pa.ptr<int>(o_cnt);
+    if (c->ws_poison) poison_dev(c, pa.base, plan_need, s);
+    zero_dev(c, v.h, (char*)v.level - (char*)v.h, s);
+    zero_dev(c, cnt, sizeof(int) * 4, s);
+    const BlocksIn B{reinterpret_cast<const C2*>(a.Haml), reinterpret_cast<const C2*>(a.Hamlv),
+                     reinterpret_cast<const C2*>(a.Hamr), reinterpret_cast<const C2*>(a.Hamrv),
+                     reinterpret_cast<const C2*>(a.Hamd), reinterpret_cast<const C2*>(a.Hamdv),
+                     reinterpret_cast<const C2*>(a.Hamld), reinterpret_cast<const C2*>(a.Hamrd)};
+    const size_t z = sizeof(C2);
+    check_range(c, B.Haml, z * a.nl * a.nl * a.nk, "planes Haml");
+    check_range(c, B.Hamlv, z * a.nl * a.nl * a.nk, "planes Hamlv");
+    check_range(c, B.Hamr, z * a.nr * a.nr * a.nk, "planes Hamr");
+    check_range(c, B.Hamrv, z * a.nr * a.nr * a.nk, "planes Hamrv");
+    check_range(c, B.Hamd, z * a.b * a.b * a.L * a.nk, "planes Hamd");
+    if (a.L > 1) check_range(c, B.Hamdv, z * a.b * a.b * (a.L - 1) * a.nk, "planes Hamdv");
+    check_range(c, B.Hamld, z * a.nl * a.b * a.nk, "planes Hamld");
+    check_range(c, B.Hamrd, z * a.nr * a.b * a.nk, "planes Hamrd");
+    check_range(c, a.E, sizeof(double) * a.npts, "planes E");
+    check_range(c, a.kidx, sizeof(int) * a.npts, "planes kidx");
+    check_range(c, a.first_mask, sizeof(int) * a.npts, "planes first mask");
+    check_range(c, a.T_LR, sizeof(double) * a.npts, "planes T_LR");
+    check_range(c, a.T_RL, sizeof(double) * a.npts, "planes T_RL");
+    check_range(c, a.status, sizeof(int) * a.npts, "planes status");
+    check_range(c, a.iters, sizeof(int) * a.npts, "planes iters");
+    const int nL = a.L + 2;
+    launch(c, NT_K_ELEM, 0, "plane pattern", [&] {
+        const unsigned gx = nblk((long)d.nmax * d.nmax, 1024);
+        // the first k-point's pattern alone refuses dense blocks (49 k-points
+        // of b = 48, L = 2 took 1.1 ms to be refused together)
+        for (int k0 = 0; k0 < a.nk; k0 += k0 ? a.nk : 1) {
+            hipLaunchKernelGGL(k_pl_pattern, dim3(gx, 2 * a.L + 5, k0 ? a.nk - 1 : 1), dim3(256), 0, s, d, v, B, k0);
+            hipLaunchKernelGGL(k_pl_levels, dim3(nL), dim3(256), 0, s, d, v);
+            hipLaunchKernelGGL(k_pl_plan, dim3(1), dim3(256), 0, s, d, v);
+        }
+        hipLaunchKernelGGL(k_pl_perm, dim3(nL), dim3(256), 0, s, d, v);
+        return hipGetLastError();
+    });
+    // sizes: the plan's when the host may wait for it, else their bounds
+    PlanHdr h{1, PL_MAXNT, d.Mcap, 0, 0};
+    if (wait) {
+        hipcheck(c, hipMemcpyAsync(c->host_plan, v.h, sizeof(PlanHdr), hipMemcpyDeviceToHost, s), "plan D2H");
+        hipcheck(c, hipStreamSynchronize(s), "plan sync");
+        h = *reinterpret_cast<const PlanHdr*>(c->host_plan);
+        if (!h.ok) return false;
+        if (h.nt < 1 || h.nt > PL_MAXNT || h.M < 3 || h.M > d.Mcap) {
+            c->err = "plane plan out of range";
+            throw Fail{NT_ERR_HIP};
+        }
+    }
+    const int NN = 256 * h.nt * h.nt;
+    // adjoint: planes from the window's first on are kept
+    const bool adj = a.adj_w != nullptr;
+    const int hi1 = adj ? std::min(a.adj_hi + 1, a.L - 1) : 0, nw1 = hi1 - a.adj_lo + 1;
+    int jw = 0;
+    std::vector<int> hk;
+    if (adj) {
+        hipcheck(c, hipMemcpyAsync(c->host_plan, v.poff + a.adj_lo + 1, sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
+        if (a.nk > 1) {
+            hk.resize(a.npts);
+            hipcheck(c, hipMemcpyAsync(hk.data(), a.kidx, sizeof(int) * a.npts, hipMemcpyDeviceToHost, s), "D2H");
+        }
+        hipcheck(c, hipStreamSynchronize(s), "sync");
+        jw = c->host_plan[0];
+        if (jw < 0 || jw >= h.M) {
+            c->err = "plane plan out of range";
+            throw Fail{NT_ERR_HIP};
+        }
+    }
+    const long kept = 2L * (h.M - jw);      // matrices per point
+    // packed blocks, then one chunk of points
+    Arena w;
+    const size_t blk = z * NN * (size_t)h.M * a.nk;
+    const size_t oH = w.take(blk), oU = w.take(blk), oL = w.take(blk), oV = w.take(z * NN * 2 * a.nk),
+                 oM = w.take(sizeof(unsigned long long) * 4 * (size_t)h.M * a.nk);
+    const size_t fixed = w.off;
+    const int NP = 16 * h.nt;
+    auto carve = [&](Arena& ar, int P) {
+        ChunkView cv = chunk_carve(ar, P, NN);
+        if (adj) {
+            cv.keep = ar.ptr<C2>(ar.take(z * NN * kept * P));
+            cv.CA = ar.ptr<C2>(ar.take(z * NP * a.b * nw1 * P));
+            cv.RW = ar.ptr<C2>(ar.take(z * NP * a.b * nw1 * P));
+            cv.place = ar.ptr<int>(ar.take(sizeof(int) * (size_t)P));
+        }
+        return cv;
+    };
+    Arena one;
+    carve(one, 64);
+    const double per_pt = (double)one.off / 64;
+    double room = adj ? PL_ADJ_BYTES : PL_CHUNK_BYTES;
+    if (a.noalloc) room = (double)scratch_bytes - reserve - fixed - 65536.0;
+    else if (c->ws_cap) room = std::min(room, (double)c->ws_cap - fixed);
+    int P = std::min((double)a.npts, room / per_pt);
+    if (P < 1) {
+        if (a.noalloc || !wait) return false;
+        P = 1;
+    }
+    carve(w, P);
+    if (a.noalloc) {
+        if (w.off > scratch_bytes - reserve) return false;
+        if (c->ws_poison) poison_dev(c, scratch, w.off, s);
+    } else {
+        ensure_ws(c, w.off);
+    }
+    const size_t total = w.off;
+    w = Arena();
+    w.base = a.noalloc ? scratch : static_cast<char*>(c->ws);
+    check_range(c, w.base, total, "planes workspace");
+    w.off = fixed;
+    C2 *pH = w.ptr<C2>(oH), *pU = w.ptr<C2>(oU), *pL = w.ptr<C2>(oL), *pV = w.ptr<C2>(oV);
+    unsigned long long* pM = w.ptr<unsigned long long>(oM);
+    const ChunkView cv = carve(w, P);
+    launch(c, NT_K_ELEM, 0, "plane pack", [&] {
+        hipLaunchKernelGGL(k_pl_pack, dim3(h.M, a.nk, 4), dim3(256), 0, s, d, v, B, pH, pU, pL, pV, pM);
+        return hipGetLastError();
+    });
+    int left = 0, later[2] = {0, 0};      // points solved on the layers, those not beside the sweep
+    for (int p0 = 0; p0 < a.npts; p0 += P) {
+        const int n = std::min(P, a.npts - p0);
+        const int* kidx = a.kidx ? a.kidx + p0 : nullptr;
+        const int* first = a.first_mask ? a.first_mask + p0 : nullptr;
+        const DecPlArgs da{v.h, v.psize, pH, pU, pL, pV, a.E + p0, kidx, prm->eta, prm->eta0, prm->convergence,
+                           prm->eta_mode, prm->max_iter, cv.scratch, cv.sigma, cv.dst, cv.dit, cv.dgrow};
+        const SweepPlArgs sa{v.h, v.psize, pH, pU, pL, pM, a.E + p0, kidx, prm->eta, prm->eta0, prm->device_eta_factor,
+                             prm->eta_mode, need + p0, cv.sigma, cv.T, cv.sst, cv.keep, v.poff + a.adj_lo + 1, kept};
+        if (p0) zero_dev(c, cnt, sizeof(int) * 2, s);
+        launch(c, NT_K_PLANES, 0, "plane decimation", [&] {
+            if (!wait || h.nt == 1) launch_decimate<1>(da, 2 * n, s);
+            if (!wait || h.nt == 2) launch_decimate<2>(da, 2 * n, s);
+            if (!wait || h.nt == 3) launch_decimate<3>(da, 2 * n, s);
+            if (!wait || h.nt == 4) launch_decimate<4>(da, 2 * n, s);
+            return hipGetLastError();
+        });
+        hipLaunchKernelGGL(k_pl_check, dim3(nblk(n)), dim3(256), 0, s, v.h, n, cv.dst, cv.dgrow, need + p0, cnt);
+        hipcheck(c, hipGetLastError(), "plane check");
+        if (wait) {
+            hipcheck(c, hipMemcpyAsync(c->host_plan, cnt, sizeof(int), hipMemcpyDeviceToHost, s), "count D2H");
+            hipcheck(c, hipEventRecord(c->chk[0], s), "event check");
+        }
+        const double m = 16.0 * h.nt;
+        launch(c, NT_K_PLANES, wait ? 2.0 * n * h.M * 5 * 8 * m * m * m : 0.0, "plane sweep", [&] {
+            if (!wait || h.nt == 1) launch_sweep<1>(sa, 2 * n, s);
+            if (!wait || h.nt == 2) launch_sweep<2>(sa, 2 * n, s);
+            if (!wait || h.nt == 3) launch_sweep<3>(sa, 2 * n, s);
+            if (!wait || h.nt == 4) launch_sweep<4>(sa, 2 * n, s);
+            return hipGetLastError();
+        });
+        hipLaunchKernelGGL(k_pl_finish, dim3(nblk(n)), dim3(256), 0, s, n, cv.dst, cv.dit, cv.sst, cv.T, first,
+                           need + p0, cnt, a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr,
+                           a.iters ? a.iters + p0 : nullptr);
+        hipcheck(c, hipGetLastError(), "plane finish");
+        if (adj) planes_adjoint(c, a, d, v, h, cv, pU, pL, pM, p0, n, hk, need + p0, kept, hi1);
+        if (!wait) continue;
+        // the points for the layers are known while the sweep still runs:
+        // they are solved beside it, on a worker context
+        hipcheck(c, hipEventSynchronize(c->chk[0]), "event sync");
+        const int n1 = c->host_plan[0];
+        // (an adjoint solve of them adds to the same gradients: afterwards)
+        const bool beside = !c->worker && !a.noalloc && !adj;
+        if (n1 && beside) solve_left(c, prm, a, p0, n, need + p0, 1, n1, true);
+        hipcheck(c, hipMemcpyAsync(c->host_plan, cnt + 1, 2 * sizeof(int), hipMemcpyDeviceToHost, s), "count D2H");
+        hipcheck(c, hipStreamSynchronize(s), "count sync");
+        left += n1 + c->host_plan[0];
+        later[0] += beside ? 0 : n1;
+        later[1] += c->host_plan[0];
+    }
+    const double steps = wait ? (double)c->host_plan[1] : 0.0;
+    if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - left;
+    TdbArgs g = a;
+    g.siblings.clear();
+    g.no_planes = true;
+    g.scratch_reserve = reserve;
+    if (!wait || (a.noalloc && left)) {
+        // every point whose need is set, masked inside the layers' kernels
+        g.mask = need;
+        solve_tdb_dev(c, prm, g);
+    } else {
+        // (in c's own workspace, which the planes have no use for any more)
+        for (int i = 0; i < 2; ++i)
+            if (later[i]) solve_left(c, prm, a, 0, a.npts, need, i + 1, later[i], false);
+    }
+    c->last_mean_iters = !wait ? -1.0 : left < a.npts ? steps / (2.0 * (a.npts - left)) : 0.0;
+    return true;
+}

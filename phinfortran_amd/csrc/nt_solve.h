@@ -33,6 +33,13 @@ struct TdbArgs {
     // workspace in the static scratch (no device allocation); the chunk of
     // points shrinks until the plan fits
     bool noalloc = false;
+    // solve only the points with a nonzero mask (FP64, no extras; the other
+    // points' outputs stay)
+    const int* mask = nullptr;
+    // not on the planes of the layers (nt_planes.hip)
+    bool no_planes = false;
+    // bytes at the end of the static scratch that are in use (noalloc)
+    size_t scratch_reserve = 0;
     // devices with the same leads, points (E, k map) and lead sizes: their
     // RGF sweeps reuse this call's lead Green's functions (FP64, no extras)
     std::vector<const TdbArgs*> siblings;
@@ -48,3 +55,8 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a);
 // solve_tdb_dev on one stream (an adjoint's gradients to the rounding of the
 // sum over parts).  Throws Fail; runs inside guarded().
 void solve_split(nt_ctx* c, const nt_params* p, const TdbArgs& a, int parts);
+
+// The solve on the planes of the layers (nt_planes.hip): whether a call is of
+// its kind, and the solve itself (false: the blocks do not fall into planes).
+bool planes_candidate(const nt_ctx* c, const nt_params* prm, const TdbArgs& a);
+bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a);

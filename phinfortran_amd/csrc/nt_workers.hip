@@ -10,6 +10,7 @@
 #include "nt_host.h"
 #include "nt_kernels.h"
 #include "nt_solve.h"
+#include "nt_planes.h"
 
 // out[i] += in[i] (n doubles): the gradient of one part of a split adjoint solve
 __global__ void k_add_doubles(double* __restrict__ out, const double* __restrict__ in, long n)
@@ -21,7 +22,7 @@ __global__ void k_add_doubles(double* __restrict__ out, const double* __restrict
 // Worker contexts of c (created once, kept until nt_destroy) given c's
 // settings and each a workspace cap of its share of the device memory left
 // (its own workspace from earlier calls counts as available to it).
-static int prepare_workers(nt_ctx* c, int W)
+int prepare_workers(nt_ctx* c, int W)
 {
     while ((int)c->subs.size() < W) {
         nt_ctx* s = nullptr;
@@ -52,6 +53,8 @@ static int prepare_workers(nt_ctx* c, int W)
         s->batch_limit = c->batch_limit;
         s->one_sweep = c->one_sweep;
         s->dec_check = c->dec_check;
+        s->planes = c->planes;
+        s->worker = true;
         s->adj_ckpt = c->adj_ckpt;
         s->inv_nb = c->inv_nb;
         s->gemm_tile = c->gemm_tile;
@@ -83,6 +86,7 @@ static void run_on_workers(nt_ctx* c, const nt_params* p, int W, const std::vect
             hipcheck(s, hipSetDevice(s->device), "hipSetDevice");
             s->regions = c->regions;                       // the caller's buffers
             if (s->ws) reg_region(s, s->ws, s->ws_bytes);
+            if (s->plan_buf) reg_region(s, s->plan_buf, s->plan_bytes);
             for (;;) {
                 {
                     std::lock_guard<std::mutex> lk(mu);
@@ -430,6 +434,13 @@ int nt_set_multi_workers(nt_ctx* c, int n)
 {
     if (!c || n < 1 || n > 16) return NT_ERR_ARG;
     c->multi_workers = n;
+    return NT_OK;
+}
+
+int nt_set_planes(nt_ctx* c, int on)
+{
+    if (!c) return NT_ERR_ARG;
+    c->planes = on != 0;
     return NT_OK;
 }
 

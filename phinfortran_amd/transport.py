@@ -643,6 +643,11 @@ class Engine:
         by side on worker contexts (default 2); 1: one stream."""
         self._check(self._L.nt_set_point_split(self.ctx, int(n)), "nt_set_point_split")
 
+    def set_planes(self, on: bool):
+        """FP64 batched solves on the planes of the principal layers (default)
+        or always on whole layers."""
+        self._check(self._L.nt_set_planes(self.ctx, int(bool(on))), "nt_set_planes")
+
     def set_workspace_poison(self, on: bool):
         """Debugging aid: fill the workspace with NaN bit patterns at the start
         of every call, so that a read of workspace the call did not write

@@ -1,0 +1,217 @@
+"""Batched solves on the planes of the principal layers (nt_planes.hip).
+
+Systems whose layers are made of planes of given sizes (couplings only inside
+a plane and to the next one), with the degrees of freedom of every layer in
+random order, so that the planes have to be found: sizes at the edges of the
+kernels' 16-column tiles and classes (16, 32, 48, 64), planes of different
+sizes, leads of other sizes than the device, several k-points whose patterns
+differ.  T against the C oracle per point to max(1e-10, 256 eps kappa) (kappa
+the largest condition number the oracle inverts), gradients and left-out
+points against the layer path, which the planes replace."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle as O
+from phinfortran_amd import _native as N
+from phinfortran_amd import lattice as lt
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.220446049250313e-16
+
+
+@pytest.fixture(scope="module")
+def T():
+    from phinfortran_amd import transport
+    return transport
+
+
+@pytest.fixture
+def planes_on(engine):
+    yield
+    engine.set_planes(True)
+
+
+def oparams(p):
+    return O.OrParams(p.eta, p.eta0, p.convergence, p.device_eta_factor, p.eta_mode, p.max_iter)
+
+
+def plane_blocks(lead, dev, L, seed, lead_r=None, density=1.0, order_seed=0):
+    """Block set whose lead cells and device layers consist of planes of the
+    sizes lead (lead_r on the right) and dev, each layer's degrees of freedom
+    in a random order (of order_seed: the same for all k-points of a system).
+    The leads are periodic; density thins the couplings."""
+    rng = np.random.default_rng(seed)
+    lead_r = lead if lead_r is None else lead_r
+
+    def c(m, n):
+        x = (rng.standard_normal((m, n)) + 1j * rng.standard_normal((m, n))) / np.sqrt(max(m, n))
+        return x * (rng.random((m, n)) < density)
+
+    def herm(n):
+        x = c(n, n)
+        return 0.5 * (x + x.conj().T)
+
+    def layer(sizes):
+        off = np.concatenate([[0], np.cumsum(sizes)])
+        H = np.zeros((off[-1], off[-1]), np.complex128)
+        for i, n in enumerate(sizes):
+            H[off[i]:off[i + 1], off[i]:off[i + 1]] = herm(n)
+            if i + 1 < len(sizes):
+                u = c(n, sizes[i + 1])
+                H[off[i]:off[i + 1], off[i + 1]:off[i + 2]] = u
+                H[off[i + 1]:off[i + 2], off[i]:off[i + 1]] = u.conj().T
+        return H, off
+
+    def couple(a, oa, b, ob):
+        """last plane of a to first plane of b"""
+        V = np.zeros((oa[-1], ob[-1]), np.complex128)
+        V[oa[-2]:oa[-1], ob[0]:ob[1]] = c(a[-1], b[0])
+        return V
+    Hl, ol = layer(lead)
+    Hr, orr = layer(lead_r)
+    Vl = couple(lead, ol, lead, ol)                     # V_{-1,0}
+    Vr = couple(lead_r, orr, lead_r, orr).conj().T      # V_{N+2,N+1}
+    Hd = [layer(dev) for _ in range(L)]
+    od = Hd[0][1]
+    order = np.random.default_rng(order_seed)
+    perm = [order.permutation(od[-1]) for _ in range(L)]
+    pl, pr = order.permutation(ol[-1]), order.permutation(orr[-1])
+    return lt.Blocks(
+        Haml=Hl[np.ix_(pl, pl)], Hamlv=Vl[np.ix_(pl, pl)], Hamr=Hr[np.ix_(pr, pr)], Hamrv=Vr[np.ix_(pr, pr)],
+        Hamd=np.stack([Hd[i][0][np.ix_(perm[i], perm[i])] for i in range(L)]),
+        Hamdv=np.stack([couple(dev, od, dev, od)[np.ix_(perm[i], perm[i + 1])] for i in range(L - 1)]) if L > 1
+        else np.zeros((0, od[-1], od[-1]), np.complex128),
+        Hamld=couple(lead, ol, dev, od)[np.ix_(pl, perm[0])],
+        Hamrd=couple(dev, od, lead_r, orr).conj().T[np.ix_(pr, perm[-1])])
+
+
+def planes_launches(engine, call):
+    engine.profile_reset()
+    engine.profile(True)
+    r = call()
+    engine.profile(False)
+    return r, engine.profile_get(N.NT_K_PLANES)["launches"], engine.profile_get(N.NT_K_INV)["launches"]
+
+
+CASES = [((1, 1), (1, 1), 1, None), ((9, 9), (9, 9), 3, None), ((16, 16), (16, 16), 2, None),
+         ((17, 16), (16, 17), 2, None), ((5, 7, 6), (7, 5, 6, 4), 3, (8, 7)), ((32, 32), (32, 32), 2, None),
+         ((33, 20), (20, 33), 2, None), ((48, 48, 48, 48), (48, 48), 2, None), ((49, 48), (30, 49), 2, None),
+         ((64, 64), (64, 64, 64), 1, None), ((63, 40, 50), (64, 33), 2, (40, 64))]
+
+
+@pytest.mark.parametrize("lead,dev,L,lead_r", CASES)
+def test_planes_vs_oracle(engine, T, planes_on, lead, dev, L, lead_r):
+    p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13)
+    blocks = [plane_blocks(lead, dev, L, 10 * L + i, lead_r) for i in range(2)]
+    rng = np.random.default_rng(3)
+    E = rng.uniform(0.05, 0.9, 9)
+    kidx = rng.integers(0, 2, E.size).astype(np.int32)
+    mask = np.zeros(E.size, np.int32)
+    mask[2] = 1
+    print(f"planes: lead {lead} device {dev} L={L}", flush=True)
+    d = engine.upload_blocks(blocks)
+    r, used, inverses = planes_launches(engine, lambda: engine.solve_tdb(d, E, p, kidx=kidx, first_point_mask=mask))
+    # lim classes can merge two planes of a layer; at least one layer is divided
+    assert used > 0 and inverses == 0
+    assert (r["status"].cpu().numpy() == 0).all()
+    for i in range(2):
+        sel = (kidx == i) & (mask == 0)
+        if not sel.any():
+            continue
+        otl, otr, ost, kap = O.solve_tdb_batch_kappa(blocks[i].as_dict(), E[sel], oparams(p), nthreads=4)
+        tol = np.maximum(1e-10, 256 * EPS * kap)
+        assert (np.abs(r["T_LR"].cpu().numpy()[sel] - otl) <= tol * np.maximum(1.0, otl)).all()
+        assert (np.abs(r["T_RL"].cpu().numpy()[sel] - otr) <= tol * np.maximum(1.0, otr)).all()
+    assert float(r["T_LR"][2]) == 0.0
+    # the recursion's own counts of steps
+    engine.set_planes(False)
+    q = engine.solve_tdb(d, E, p, kidx=kidx, first_point_mask=mask)
+    assert np.array_equal(r["iters"].cpu().numpy(), q["iters"].cpu().numpy())
+
+
+@pytest.mark.parametrize("dev,lo,hi", [((9, 9), 0, 2), ((16, 20), 1, 1), ((33, 20, 40), 2, 2), ((64, 30), 0, 1)])
+def test_planes_gradient(engine, T, planes_on, dev, lo, hi):
+    """the gradient of the planes' sweep against the layers', whose own test is
+    finite differences; sums over 11 points of two k-points"""
+    p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13)
+    blocks = [plane_blocks((12, 10), dev, 3, 50 + i) for i in range(2)]
+    rng = np.random.default_rng(4)
+    E = rng.uniform(0.05, 0.9, 11)
+    kidx = rng.integers(0, 2, 11).astype(np.int32)
+    w = rng.uniform(0.5, 2.0, 11)
+    d = engine.upload_blocks(blocks)
+    print(f"planes gradient: device {dev} window {lo}..{hi}", flush=True)
+    r, used, inverses = planes_launches(engine, lambda: engine.solve_tdb_adjoint(d, E, p, w, lo, hi, kidx=kidx))
+    assert used > 0 and inverses == 0
+    engine.set_planes(False)
+    q = engine.solve_tdb_adjoint(d, E, p, w, lo, hi, kidx=kidx)
+    for k in ("T_LR", "T_RL", "dHamd", "dHamdv"):
+        x, y = r[k].cpu().numpy(), q[k].cpu().numpy()
+        assert x.shape == y.shape and np.abs(x - y).max(initial=0.0) <= 1e-9 * max(1.0, np.abs(y).max(initial=0.0)), k
+
+
+def test_left_out_points_are_the_layers(engine, T, planes_on):
+    """A plane of uncoupled sites at their own energy, at no broadening to speak
+    of: the plane is singular there though its layer is not.  Those points come
+    from the layers, bit for bit, the others from the planes."""
+    blk = lt.agnr_blocks(n_dimer=9, L=3, onsite_w=0.0, hop_noise=0.0)
+    p = T.params("tb", eta=1e-9, convergence=1e-12)
+    E = np.array([0.7, 0.0, -1.3, 1e-14, 0.9])
+    d = engine.upload_blocks(blk)
+    r, used, inverses = planes_launches(engine, lambda: engine.solve_tdb(d, E, p))
+    assert used > 0 and inverses > 0
+    engine.set_planes(False)
+    q = engine.solve_tdb(d, E, p)
+    for k in ("T_LR", "T_RL", "status", "iters"):
+        x, y = r[k].cpu().numpy(), q[k].cpu().numpy()
+        assert np.array_equal(x[[1, 3]], y[[1, 3]], equal_nan=True), (k, x, y)
+        assert np.allclose(x, y, rtol=1e-6, atol=1e-9, equal_nan=True), (k, x, y)
+
+
+@pytest.mark.parametrize("what", ["dense", "nan", "not hermitian"])
+def test_what_stays_on_the_layers(engine, T, planes_on, what):
+    """dense blocks have no planes; a block with a NaN fails on either path
+    with the same status; leads that are not Hermitian are not decimated on
+    planes (the adjoint of the advanced function is not the retarded one)"""
+    p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13)
+    blk = plane_blocks((9, 8), (9, 8), 2, 5) if what != "dense" else lt.random_blocks(12, 12, 2, seed=3)
+    E = np.array([0.1, 0.4, 0.8])
+    if what == "nan":
+        H = blk.Hamd.copy()
+        i = np.argwhere(np.abs(H[0]) > 0)[0]
+        H[0, i[0], i[1]] = np.nan
+        blk = dataclasses.replace(blk, Hamd=H)
+    if what == "not hermitian":
+        H = blk.Haml.copy()
+        i = np.argwhere(np.triu(np.abs(H), 1) > 0)[0]
+        H[i[0], i[1]] *= 1.001
+        blk = dataclasses.replace(blk, Haml=H)
+    d = engine.upload_blocks(blk)
+    r, used, _ = planes_launches(engine, lambda: engine.solve_tdb(d, E, p))
+    assert (used > 0) == (what == "nan")
+    engine.set_planes(False)
+    q = engine.solve_tdb(d, E, p)
+    for k in ("T_LR", "T_RL", "status", "iters"):
+        assert np.array_equal(r[k].cpu().numpy(), q[k].cpu().numpy(), equal_nan=True), k
+
+
+def test_noalloc_and_no_check_agree(engine, T, planes_on):
+    """the allocation-free entry and the solve without host synchronisation
+    run the same kernels: the same bits"""
+    p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13, max_iter=48)
+    d = engine.upload_blocks(plane_blocks((20, 33), (33, 20), 3, 9))
+    E = np.linspace(0.05, 0.9, 21)
+    ref = engine.solve_tdb(d, E, p)
+    try:
+        for every in (4, 0):
+            engine.set_decimation_check(every)
+            for noalloc in (False, True):
+                print(f"check every {every}, noalloc {noalloc}", flush=True)
+                r = engine.solve_tdb(d, E, p, noalloc=noalloc)
+                for k in ("T_LR", "T_RL", "status", "iters"):
+                    assert np.array_equal(ref[k].cpu().numpy(), r[k].cpu().numpy()), (every, noalloc, k)
+    finally:
+        engine.set_decimation_check(4)

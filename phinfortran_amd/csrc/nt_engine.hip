@@ -18,6 +18,7 @@
 
 #include "nt_host.h"
 #include "nt_solve.h"
+#include "nt_planes.h"
 
 // Static device scratch of the allocation-free batched solve
 // (nt_solve_tdb_batched_noalloc_dev).  Each GPU the library runs on holds its
@@ -1371,6 +1372,15 @@ constexpr double ADJ_BUDGET_BYTES = 24.0 * 1024 * 1024 * 1024;
 constexpr double MIXED_BUDGET_BYTES = 64.0 * 1024 * 1024 * 1024;
 
 }  // namespace
+
+size_t lead_sigma_scratch(int n, int Q) { return decimate_scratch<double>(n, Q); }
+
+void lead_sigma(nt_ctx* c, int n, int Q, BMat<double> H00, BMat<double> V, const double* z, double conv, int max_iter,
+                BMatW<double> g, BMatW<double> sigma, int* status, int* iters, Arena& ar, size_t scratch_off)
+{
+    DecimationOut<double> o{g, sigma, nonew<double>()};
+    decimate<double>(c, n, Q, H00, V, 1, z, conv, max_iter, o, status, iters, ar, scratch_off);
+}
 
 void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
 {

@@ -62,3 +62,10 @@ struct AdjPlArgs {
 
 // n worker contexts of c set up for a call (nt_workers.hip)
 int prepare_workers(nt_ctx* c, int n);
+
+// Decimation of Q leads (H00 of its own for every item) at the shifts z, as the
+// layers' (nt_engine.hip): g = (z - es)^-1, sigma = V^+ g V; scratch from
+// scratch_off of ar on.
+size_t lead_sigma_scratch(int n, int Q);
+void lead_sigma(nt_ctx* c, int n, int Q, BMat<double> H00, BMat<double> V, const double* z, double conv, int max_iter,
+                BMatW<double> g, BMatW<double> sigma, int* status, int* iters, Arena& ar, size_t scratch_off);

@@ -12,7 +12,7 @@
 //
 //   k_pl_pattern  which elements of the blocks are nonzero at any k-point
 //   k_pl_levels   per layer: distances from the previous layer, plane counts
-//   k_pl_plan     plane size class (16, 32, 48, 64), plane offsets, validity
+//   k_pl_plan     plane size class (16, 32, 48, 64, 96), plane offsets, validity
 //   k_pl_perm     degrees of freedom of every plane
 //   k_pl_pack     diagonal and coupling blocks of the planes, per k-point,
 //                 zero padded to the class size
@@ -22,7 +22,7 @@
 //
 // The plan stays on the device: no kernel needs the host to know it, so a
 // solve can be captured in a HIP graph.  Blocks without zeros form one plane
-// per layer; layers of planes over 64 are left to the block path.
+// per layer and are left to the block path, as are planes over 96.
 //
 // Inside the two solver kernels a wave owns 16 columns of every matrix, in
 // registers, in the layout in which v_mfma_f64_16x16x4 returns its result:
@@ -39,7 +39,11 @@ namespace {
 
 typedef double2 C2;
 
-constexpr int PL_MAXNT = 4;         // largest class: planes of 64
+constexpr int PL_MAXNT = 4;         // planes of up to 64: both solver kernels
+constexpr int PL_BIGNT = 6;         // planes of up to 96: the sweep's (planes_big_leads decimates)
+constexpr int PL_NCLS = 5;          // plane size classes 16, 32, 48, 64, 96
+constexpr int PL_PERM = 16 * PL_BIGNT;
+__host__ __device__ constexpr int class_nt(int t) { return t < PL_MAXNT ? t + 1 : PL_BIGNT; }
 constexpr int PL_WAVES = 2;          // waves per SIMD the solver kernels are built for
 constexpr int PL_NLV = 128;         // levels a layer may have
 // A decimation step whose cell is nearly singular at E loses digits that the
@@ -65,11 +69,11 @@ struct PlanView {
     int* level;         // (layer, dof)
     int* nlev;          // (layer)
     int* cnt;           // (layer, PL_NLV) dofs per level
-    int* npl;           // (layer, PL_MAXNT) planes per class, -1: a level does not fit
+    int* npl;           // (layer, PL_NCLS) planes per class, -1: a level does not fit
     int* poff;          // (layer + 1) first plane
     int* psize;         // (plane)
     int* player;        // (plane) layer
-    int* perm;          // (plane, 64) dof of the layer at each place
+    int* perm;          // (plane, PL_PERM) dof of the layer at each place
 };
 
 // sizes a plan depends on
@@ -96,8 +100,8 @@ PlanView plan_carve(Arena& a, const PlanDims& d)
     const size_t oh = a.take(sizeof(PlanHdr)), oa = a.take(i4 * nL * d.nmax * d.W), oc = a.take(i4 * nL * d.W),
                  orr = a.take(i4 * nL * d.W), ob = a.take(i4);
     const size_t ol = a.take(i4 * nL * d.nmax), on = a.take(i4 * nL), oq = a.take(i4 * nL * PL_NLV),
-                 op = a.take(i4 * nL * PL_MAXNT), oo = a.take(i4 * (nL + 1)), os = a.take(i4 * d.Mcap),
-                 oy = a.take(i4 * d.Mcap), om = a.take(i4 * (size_t)d.Mcap * 64);
+                 op = a.take(i4 * nL * PL_NCLS), oo = a.take(i4 * (nL + 1)), os = a.take(i4 * d.Mcap),
+                 oy = a.take(i4 * d.Mcap), om = a.take(i4 * (size_t)d.Mcap * PL_PERM);
     v.h = a.ptr<PlanHdr>(oh);
     v.adj = a.ptr<unsigned>(oa);
     v.cbits = a.ptr<unsigned>(oc);
@@ -254,10 +258,10 @@ __global__ __launch_bounds__(256) void k_pl_levels(PlanDims d, PlanView v)
     __syncthreads();
     if (t < PL_NLV) v.cnt[(long)layer * PL_NLV + t] = cnt[t];
     if (t == 0) v.nlev[layer] = m + 1;
-    if (t < PL_MAXNT) {
-        // planes of at most 16 (t + 1): consecutive levels merged while they
+    if (t < PL_NCLS) {
+        // planes of at most the class's size: consecutive levels merged while they
         // fit (plane_starts); a lead cell keeps two at least
-        const int lim = 16 * (t + 1);
+        const int lim = 16 * class_nt(t);
         const bool lead = layer == 0 || layer == d.L + 1;
         int planes = 0, fill = lim + 1;
         for (int l = 0; l <= m; ++l) {
@@ -273,22 +277,22 @@ __global__ __launch_bounds__(256) void k_pl_levels(PlanDims d, PlanView v)
                 fill += k;
             }
         }
-        v.npl[layer * PL_MAXNT + t] = planes;
+        v.npl[layer * PL_NCLS + t] = planes;
     }
 }
 
-// One workgroup of four waves: wave t sums the planes of class t + 1, the
-// cheapest class wins: per plane about five products of the class size and as
+// One workgroup: wave t sums the planes of class t, the cheapest of the first
+// ncls classes wins: per plane about five products of the class size and as
 // many pivots as it has columns (5120 SIMD cycles per 16^3 of products and
 // 12000 per 16 pivots).
-__global__ __launch_bounds__(256) void k_pl_plan(PlanDims d, PlanView v)
+__global__ __launch_bounds__(64 * PL_NCLS) void k_pl_plan(PlanDims d, PlanView v, int ncls)
 {
     const int nL = d.L + 2, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    __shared__ int tot[PL_MAXNT];
+    __shared__ int tot[PL_NCLS];
     __shared__ int pick;
     int s = 0, bad = 0;
     for (int i = lane; i < nL; i += 64) {
-        const int p = v.npl[i * PL_MAXNT + w];
+        const int p = v.npl[i * PL_NCLS + w];
         bad |= p < 0;
         s += p;
     }
@@ -300,32 +304,34 @@ __global__ __launch_bounds__(256) void k_pl_plan(PlanDims d, PlanView v)
     __syncthreads();
     if (threadIdx.x == 0) {
         double best = 0.0;
-        int nt = 0;
-        for (int t = 0; t < PL_MAXNT; ++t) {
+        int cl = -1;
+        for (int t = 0; t < ncls; ++t) {
             if (tot[t] < 0) continue;
-            const double u = t + 1, c = tot[t] * (5120.0 * u * u * u + 12000.0 * u);
-            if (!nt || c < best) {
+            const double u = class_nt(t), c = tot[t] * (5120.0 * u * u * u + 12000.0 * u);
+            if (cl < 0 || c < best) {
                 best = c;
-                nt = t + 1;
+                cl = t;
             }
         }
-        pick = nt;
-        v.h->nt = nt;
-        v.h->M = nt ? tot[nt - 1] : 0;
+        pick = cl;
+        const int M = cl < 0 ? 0 : tot[cl], m0 = cl < 0 ? 0 : v.npl[cl], m1 = cl < 0 ? 0 : v.npl[(nL - 1) * PL_NCLS + cl];
+        v.h->nt = cl < 0 ? 0 : class_nt(cl);
+        v.h->M = M;
+        v.h->m0 = m0;
+        v.h->m1 = m1;
         // one plane per layer: nothing is gained over the layers themselves; a
-        // lead cell of one plane: not written for that
-        v.h->ok = nt > 0 && !*v.bad && tot[nt - 1] <= d.Mcap && tot[nt - 1] > nL &&
-                  v.npl[nt - 1] > 1 && v.npl[(nL - 1) * PL_MAXNT + nt - 1] > 1;
-        v.h->m0 = nt ? v.npl[nt - 1] : 0;
-        v.h->m1 = nt ? v.npl[(nL - 1) * PL_MAXNT + nt - 1] : 0;
+        // lead cell of one plane: not written for that; the large class's
+        // leads: both cells of two to four planes
+        v.h->ok = cl >= 0 && !*v.bad && M <= d.Mcap && M > nL && m0 > 1 && m1 > 1 &&
+                  (cl < PL_MAXNT || (m0 == m1 && m0 <= 4));
     }
     __syncthreads();
-    const int nt = pick;
-    if (!nt || w) return;
+    const int cl = pick;
+    if (cl < 0 || w) return;
     int base = 0;
     for (int i0 = 0; i0 < nL; i0 += 64) {
         const int i = i0 + lane;
-        int x = i < nL ? v.npl[i * PL_MAXNT + nt - 1] : 0, inc = x;
+        int x = i < nL ? v.npl[i * PL_NCLS + cl] : 0, inc = x;
         for (int o = 1; o < 64; o <<= 1) {
             const int y = __shfl_up(inc, o);
             if (lane >= o) inc += y;
@@ -364,7 +370,7 @@ __global__ __launch_bounds__(256) void k_pl_perm(PlanDims d, PlanView v)
     for (int i = t; i < n; i += 256) {
         int pos = 0;
         for (int j = 0; j < i; ++j) pos += pl[j] == pl[i];
-        v.perm[(long)(p0 + pl[i]) * 64 + pos] = i;
+        v.perm[(long)(p0 + pl[i]) * PL_PERM + pos] = i;
     }
     for (int p = t; p < np; p += 256) {
         int c = 0;
@@ -385,14 +391,14 @@ __global__ __launch_bounds__(256) void k_pl_pack(PlanDims d, PlanView v, BlocksI
     if (!h.ok || pl >= M) return;
     const int NP = 16 * h.nt, NN = NP * NP;
     const int la = v.player[pl], na = layer_size(d, la), sa = v.psize[pl];
-    const int* pa = v.perm + (long)pl * 64;
+    const int* pa = v.perm + (long)pl * PL_PERM;
     if (what == 3) {
         if (pl != 0 && pl != M - 1) return;
         // V from the plane that faces the device (rows) to the one that faces
         // the lead (columns) of the next cell
         const int side = pl != 0;
         const int fb = side ? M - h.m1 : h.m0 - 1;        // plane facing the device
-        const int* pb = v.perm + (long)fb * 64;
+        const int* pb = v.perm + (long)fb * PL_PERM;
         const int sb = v.psize[fb];
         const C2* V = side ? B.Hamrv + (long)k * na * na : B.Hamlv + (long)k * na * na;
         C2* o = LV + ((long)k * 2 + side) * NN;
@@ -417,7 +423,7 @@ __global__ __launch_bounds__(256) void k_pl_pack(PlanDims d, PlanView v, BlocksI
     }
     if (pl + 1 >= M) return;
     const int lb = v.player[pl + 1], nb = layer_size(d, lb), sb = v.psize[pl + 1];
-    const int* pb = v.perm + (long)(pl + 1) * 64;
+    const int* pb = v.perm + (long)(pl + 1) * PL_PERM;
     // U (rows of this plane, columns of the next), Lw (rows of the next)
     const C2* S = nullptr;
     int ld = 0;
@@ -454,7 +460,7 @@ __global__ __launch_bounds__(256) void k_pl_pack(PlanDims d, PlanView v, BlocksI
             }
         }
         o[e] = x;
-        if (!(x.x == 0.0 && x.y == 0.0)) {
+        if (h.nt <= PL_MAXNT && !(x.x == 0.0 && x.y == 0.0)) {
             atomicOr(&piece[0], 1ull << (h.nt * (r / 4) + c / 16));
             atomicOr(&piece[1], 1ull << (h.nt * (c / 4) + r / 16));
         }
@@ -1212,13 +1218,15 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
             const unsigned long long mu = mk[sys ? 2 : 0], ml = mk[sys ? 1 : 3];
             Blk<NT> t2;
             blk_zero<NT>(t2);
-            blk_mul<NT, true>(t2, LdT{U, NP}, R, mu);
+            // (a mask has room for the pieces of classes up to 64)
+            blk_mul<NT, NT <= PL_MAXNT>(t2, LdT{U, NP}, R, mu);
             R = t2;
             blk_load<NT>(t2, LdN{U, NP}, w);
             Blk<NT> X;
             blk_zero<NT>(X);
-            blk_mul_rows<NT>(X, LsN{s.g, LD}, t2, mu >> w);
-            blk_mul<NT, true>(m, LdN{Lo, NP}, X, ml);
+            if constexpr (NT <= PL_MAXNT) blk_mul_rows<NT>(X, LsN{s.g, LD}, t2, mu >> w);
+            else blk_mul<NT>(X, LsN{s.g, LD}, t2);
+            blk_mul<NT, NT <= PL_MAXNT>(m, LdN{Lo, NP}, X, ml);
         }
         blk_shift<NT>(m, E, i < lead_planes ? et : a.dev_factor * et, a.psize[j], w);
         __syncthreads();
@@ -1319,11 +1327,11 @@ __global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
         if (on) {
             blk_zero<NT>(y);
             const unsigned long long* mk = a.masks + ((long)k * M + j) * 4;
-            blk_mul<NT, true>(y, LdN{Uk + (long)j * NN, NP}, C, mk[1]);
+            blk_mul<NT, NT <= PL_MAXNT>(y, LdN{Uk + (long)j * NN, NP}, C, mk[1]);
             blk_zero<NT>(C);
             blk_mul<NT>(C, LdN{gl(j), NP}, y);
             blk_zero<NT>(y);
-            blk_mul<NT, true>(y, LdT{Lk + (long)j * NN, NP}, R, mk[2]);
+            blk_mul<NT, NT <= PL_MAXNT>(y, LdT{Lk + (long)j * NN, NP}, R, mk[2]);
             blk_load<NT>(R, LdN{g0(j), NP}, w);
             blk_mul<NT>(R, LdT{gl(j), NP}, y);
         }
@@ -1332,7 +1340,7 @@ __global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
             const long cc = (long)place * NP + 16 * w + (lane & 15);
             C2* CA = a.CA + l * a.K * a.b + cc * a.b;
             C2* RW = a.RW + l * a.K * a.b + cc;
-            const int* pm = a.perm + (long)j * 64;
+            const int* pm = a.perm + (long)j * PL_PERM;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -1482,7 +1490,7 @@ ChunkView chunk_carve(Arena& a, int P, int NN)
 {
     const size_t it = 2 * (size_t)P;
     ChunkView v;
-    v.scratch = a.ptr<C2>(a.take(sizeof(C2) * it * DEC_SLOTS * NN));
+    v.scratch = a.ptr<C2>(a.take(NN <= 256 * PL_MAXNT * PL_MAXNT ? sizeof(C2) * it * DEC_SLOTS * NN : 0));
     v.sigma = a.ptr<C2>(a.take(sizeof(C2) * it * NN));
     v.dst = a.ptr<int>(a.take(sizeof(int) * it));
     v.dit = a.ptr<int>(a.take(sizeof(int) * it));
@@ -1492,10 +1500,187 @@ ChunkView chunk_carve(Arena& a, int P, int NN)
     return v;
 }
 
+// ---------------------------------------- leads whose planes hold more than 64
+// The two planes of a lead cell, as one matrix, no longer fit the decimation
+// kernel's registers: their cell (the planes between eliminated by one batched
+// inverse and four products) goes through the layers' decimation instead, as a
+// lead of 2 NP degrees of freedom of its own (half of the layer's: an eighth
+// of its operations).
+
+// shift and (k, lead) of item 2 p + lead
+__global__ void k_pl_items(int P, const double* E, const int* kidx, double eta, double eta0, int mode, double* z,
+                           int* idx)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= 2 * P) return;
+    const double e = E[q / 2], et = mode == NT_ETA_RELATIVE ? e * eta + eta0 : eta;
+    z[2 * q] = e;
+    z[2 * q + 1] = q & 1 ? et : -et;
+    idx[q] = 2 * (kidx ? kidx[q / 2] : 0) + (q & 1);
+}
+
+// packed block of a lead cell's planes counted from A: 0 diagonal block of
+// plane j, 1 coupling j -> j + 1, 2 coupling back
+__device__ __forceinline__ const C2* cell_block(const C2* H, const C2* U, const C2* Lw, int M, long NN, int k, int side,
+                                                int what, int j)
+{
+    const long o = (long)k * M;
+    if (what == 0) return H + (o + (side ? M - 1 - j : j)) * NN;
+    return ((what == 1) != (side != 0) ? U : Lw) + (o + (side ? M - 2 - j : j)) * NN;
+}
+
+// per (k, lead): F_0, B_0, F_l, B_l (l the last coupling) and V as a 2 NP square
+__global__ void k_pl_cell_stack(int M, int NP, int mc, const C2* H, const C2* U, const C2* Lw, const C2* LV, C2* CP,
+                                C2* VS)
+{
+    const int ks = blockIdx.y, k = ks / 2, side = ks & 1;
+    const long NN = (long)NP * NP;
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < 4 * NN; e += (long)gridDim.x * blockDim.x) {
+        const int m = (int)(e / NN);
+        const long i = e % NN;
+        CP[(long)ks * 4 * NN + e] = cell_block(H, U, Lw, M, NN, k, side, 1 + (m & 1), m < 2 ? 0 : mc - 2)[i];
+        const int r = (int)(e % (2 * NP)), c = (int)(e / (2 * NP));
+        VS[(long)ks * 4 * NN + e] =
+            r >= NP && c < NP ? LV[(long)ks * NN + (r - NP) + (long)c * NP] : make_double2(0.0, 0.0);
+    }
+}
+
+// z - the planes between A and B (one or two), the identity on the padding
+__global__ void k_pl_cell_mid(int M, int NP, int mc, const int* psize, const C2* H, const C2* U, const C2* Lw,
+                              const int* idx, const double* z, C2* W)
+{
+    const int q = blockIdx.y, ks = idx[q], k = ks / 2, side = ks & 1, N2 = 2 * NP;
+    const long NN = (long)NP * NP;
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < 4 * NN; e += (long)gridDim.x * blockDim.x) {
+        const int r = (int)(e % N2), c = (int)(e / N2), hr = r >= NP, hc = c >= NP, r0 = r - hr * NP, c0 = c - hc * NP;
+        const int nr = hr && mc < 4 ? 0 : psize[side ? M - 2 - hr : 1 + hr];
+        const int ncl = hc && mc < 4 ? 0 : psize[side ? M - 2 - hc : 1 + hc];
+        C2 x = make_double2(r == c ? 1.0 : 0.0, 0.0);
+        if (r0 < nr && c0 < ncl) {
+            const C2 b = cell_block(H, U, Lw, M, NN, k, side, hr == hc ? 0 : hr < hc ? 1 : 2, hr == hc ? 1 + hr : 1)[
+                r0 + (long)c0 * NP];
+            x = make_double2((r == c ? z[2 * q] : 0.0) - b.x, (r == c ? z[2 * q + 1] : 0.0) - b.y);
+        }
+        W[(long)q * 4 * NN + e] = x;
+    }
+}
+
+// the cell's own blocks added to He (cleared first where add = 0); z - 1 on the
+// padding's diagonal (the decimation inverts z - He)
+__global__ void k_pl_cell_own(int M, int NP, int mc, const int* psize, const C2* H, const C2* U, const C2* Lw,
+                              const int* idx, const double* z, int add, C2* He)
+{
+    const int q = blockIdx.y, ks = idx[q], k = ks / 2, side = ks & 1, N2 = 2 * NP;
+    const long NN = (long)NP * NP;
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < 4 * NN; e += (long)gridDim.x * blockDim.x) {
+        const int r = (int)(e % N2), c = (int)(e / N2), hr = r >= NP, hc = c >= NP, r0 = r - hr * NP, c0 = c - hc * NP;
+        C2 x = add ? He[(long)q * 4 * NN + e] : make_double2(0.0, 0.0);
+        if (hr == hc || mc == 2) {
+            const C2 b = cell_block(H, U, Lw, M, NN, k, side, hr == hc ? 0 : hr < hc ? 1 : 2,
+                                    hr == hc ? hr * (mc - 1) : 0)[r0 + (long)c0 * NP];
+            x.x += b.x;
+            x.y += b.y;
+        }
+        const int pl = hr ? mc - 1 : 0;
+        if (r == c && r0 >= psize[side ? M - 1 - pl : pl]) x = make_double2(z[2 * q] - 1.0, z[2 * q + 1]);
+        He[(long)q * 4 * NN + e] = x;
+    }
+}
+
+// retarded self-energy on plane A: the right lead's own, the left's adjoint
+__global__ void k_pl_cell_sigma(int NP, const C2* S, C2* sigma, double* grow)
+{
+    const int q = blockIdx.y, N2 = 2 * NP;
+    const long NN = (long)NP * NP;
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < NN; e += (long)gridDim.x * blockDim.x) {
+        const int r = (int)(e % NP), c = (int)(e / NP);
+        const C2* s = S + (long)q * 4 * NN;
+        C2 x = q & 1 ? s[r + (long)c * N2] : s[c + (long)r * N2];
+        if (!(q & 1)) x.y = -x.y;
+        sigma[(long)q * NN + e] = x;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) grow[q] = 0.0;
+}
+
+struct BigView {
+    C2 *CP, *VS, *W, *G1, *He, *S;
+    double* z;
+    int* idx;
+    size_t dec_off;
+};
+
+BigView big_carve(Arena& a, int P, int nk, int NP)
+{
+    const size_t N2 = 2 * (size_t)NP, mb = sizeof(C2) * N2 * N2, Q = 2 * (size_t)P;
+    BigView v;
+    v.CP = a.ptr<C2>(a.take(mb * 2 * nk));
+    v.VS = a.ptr<C2>(a.take(mb * 2 * nk));
+    v.W = a.ptr<C2>(a.take(mb * Q));
+    v.G1 = a.ptr<C2>(a.take(mb * Q));
+    v.He = a.ptr<C2>(a.take(mb * Q));
+    v.S = a.ptr<C2>(a.take(mb * Q));
+    v.z = a.ptr<double>(a.take(sizeof(double) * 2 * Q));
+    v.idx = a.ptr<int>(a.take(sizeof(int) * Q));
+    v.dec_off = a.off;
+    a.take(lead_sigma_scratch((int)N2, (int)Q));
+    return v;
+}
+
 // bytes a chunk of points may take
 constexpr double PL_CHUNK_BYTES = 6.0 * 1024 * 1024 * 1024;
 constexpr double PL_ADJ_BYTES = 24.0 * 1024 * 1024 * 1024;
 constexpr int PL_MAX_ITER = 20000;      // decimation steps inside one kernel
+
+// self-energies of a chunk's points on leads of large planes
+void planes_big_leads(nt_ctx* c, const nt_params* prm, const TdbArgs& a, const PlanView& v, const PlanHdr& h,
+                      const BigView& g, Arena& ar, const C2* pH, const C2* pU, const C2* pL, const C2* pV, int p0, int n,
+                      const ChunkView& cv)
+{
+    typedef double T;
+    hipStream_t s = c->stream;
+    const int NP = 16 * h.nt, N2 = 2 * NP, Q = 2 * n, mc = h.m0, nk2 = 2 * a.nk;
+    const long NN = (long)NP * NP, N4 = 4 * NN;
+    const unsigned gx = nblk(N4, 1024);
+    auto R = [](const C2* p) { return reinterpret_cast<const T*>(p); };
+    auto W = [](C2* p) { return reinterpret_cast<T*>(p); };
+    launch(c, NT_K_ELEM, 0, "cell items", [&] {
+        hipLaunchKernelGGL(k_pl_items, dim3(nblk(Q)), dim3(256), 0, s, n, a.E + p0, a.kidx ? a.kidx + p0 : nullptr,
+                           prm->eta, prm->eta0, prm->eta_mode, g.z, g.idx);
+        hipLaunchKernelGGL(k_pl_cell_stack, dim3(gx, nk2), dim3(256), 0, s, h.M, NP, mc, pH, pU, pL, pV, g.CP, g.VS);
+        return hipGetLastError();
+    });
+    zero_dev(c, cv.dst, sizeof(int) * Q, s);
+    if (mc > 2) {
+        launch(c, NT_K_ELEM, 0, "cell mid", [&] {
+            hipLaunchKernelGGL(k_pl_cell_mid, dim3(gx, Q), dim3(256), 0, s, h.M, NP, mc, v.psize, pH, pU, pL, g.idx, g.z,
+                               g.W);
+            return hipGetLastError();
+        });
+        inverse<T>(c, N2, bw(W(g.W), N4, N2), none<T>(), nullptr, bw(W(g.G1), N4, N2), cv.dst, Q);
+        // T = G [B_0, F_l] (into W), He = [F_0 T; B_l T]
+        const int r = mc == 4 ? NP : 0;
+        auto blk = [&](int m) { return bm<T>(R(g.CP) + 2 * m * NN, N4, NP, g.idx, 0, nk2); };
+        gemm<T>(c, N2, NP, NP, OP_N, bm<T>(R(g.G1), N4, N2), OP_N, blk(1), bw(W(g.W), N4, N2), 1.0, none<T>(), 0.0,
+                nullptr, Q);
+        gemm<T>(c, N2, NP, NP, OP_N, bm<T>(R(g.G1) + 2L * r * N2, N4, N2), OP_N, blk(2),
+                bw(W(g.W) + 2L * NP * N2, N4, N2), 1.0, none<T>(), 0.0, nullptr, Q);
+        gemm<T>(c, NP, N2, NP, OP_N, blk(0), OP_N, bm<T>(R(g.W), N4, N2), bw(W(g.He), N4, N2), 1.0, none<T>(), 0.0,
+                nullptr, Q);
+        gemm<T>(c, NP, N2, NP, OP_N, blk(3), OP_N, bm<T>(R(g.W) + 2 * r, N4, N2), bw(W(g.He) + 2 * NP, N4, N2), 1.0,
+                none<T>(), 0.0, nullptr, Q);
+    }
+    launch(c, NT_K_ELEM, 0, "cell own", [&] {
+        hipLaunchKernelGGL(k_pl_cell_own, dim3(gx, Q), dim3(256), 0, s, h.M, NP, mc, v.psize, pH, pU, pL, g.idx, g.z,
+                           mc > 2, g.He);
+        return hipGetLastError();
+    });
+    lead_sigma(c, N2, Q, bm<T>(R(g.He), N4, N2), bm<T>(R(g.VS), N4, N2, g.idx, 0, nk2), g.z, prm->convergence,
+               prm->max_iter, bw(W(g.G1), N4, N2), bw(W(g.S), N4, N2), cv.dst, cv.dit, ar, g.dec_off);
+    launch(c, NT_K_ELEM, 0, "cell sigma", [&] {
+        hipLaunchKernelGGL(k_pl_cell_sigma, dim3(nblk(NN, 1024), Q), dim3(256), 0, s, NP, g.S, cv.sigma, cv.dgrow);
+        return hipGetLastError();
+    });
+}
 
 template <int NT>
 void launch_adjoint(const AdjPlArgs& a, int n, hipStream_t s)
@@ -1536,6 +1721,7 @@ void planes_adjoint(nt_ctx* c, const TdbArgs& a, const PlanDims& d, const PlanVi
         if (h.nt == 2) launch_adjoint<2>(aa, n, s);
         if (h.nt == 3) launch_adjoint<3>(aa, n, s);
         if (h.nt == 4) launch_adjoint<4>(aa, n, s);
+        if (h.nt == PL_BIGNT) launch_adjoint<PL_BIGNT>(aa, n, s);
         return hipGetLastError();
     });
     // dHd_l += 2 sum_p R_l^+ C_l^+, dHdv_l += 2 sum_p (R_l^+ C_{l+1}^+ + C_l R_{l+1}),
@@ -1708,6 +1894,9 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     check_range(c, a.status, sizeof(int) * a.npts, "planes status");
     check_range(c, a.iters, sizeof(int) * a.npts, "planes iters");
     const int nL = a.L + 2;
+    // the large class where the host may wait, with workspace, and not at a
+    // fixed broadening (its decimation has no measure of the growth)
+    const int ncls = wait && !a.noalloc && prm->eta_mode == NT_ETA_RELATIVE ? PL_NCLS : PL_MAXNT;
     launch(c, NT_K_ELEM, 0, "plane pattern", [&] {
         const unsigned gx = nblk((long)d.nmax * d.nmax, 1024);
         // the first k-point's pattern alone refuses dense blocks (49 k-points
@@ -1715,7 +1904,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         for (int k0 = 0; k0 < a.nk; k0 += k0 ? a.nk : 1) {
             hipLaunchKernelGGL(k_pl_pattern, dim3(gx, 2 * a.L + 5, k0 ? a.nk - 1 : 1), dim3(256), 0, s, d, v, B, k0);
             hipLaunchKernelGGL(k_pl_levels, dim3(nL), dim3(256), 0, s, d, v);
-            hipLaunchKernelGGL(k_pl_plan, dim3(1), dim3(256), 0, s, d, v);
+            hipLaunchKernelGGL(k_pl_plan, dim3(1), dim3(64 * PL_NCLS), 0, s, d, v, ncls);
         }
         hipLaunchKernelGGL(k_pl_perm, dim3(nL), dim3(256), 0, s, d, v);
         return hipGetLastError();
@@ -1727,7 +1916,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         hipcheck(c, hipStreamSynchronize(s), "plan sync");
         h = *reinterpret_cast<const PlanHdr*>(c->host_plan);
         if (!h.ok) return false;
-        if (h.nt < 1 || h.nt > PL_MAXNT || h.M < 3 || h.M > d.Mcap) {
+        if (h.nt < 1 || h.nt > PL_BIGNT || h.M < 3 || h.M > d.Mcap) {
             c->err = "plane plan out of range";
             throw Fail{NT_ERR_HIP};
         }
@@ -1759,6 +1948,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
                  oM = w.take(sizeof(unsigned long long) * 4 * (size_t)h.M * a.nk);
     const size_t fixed = w.off;
     const int NP = 16 * h.nt;
+    const bool big = h.nt > PL_MAXNT;
+    BigView bv{};
     auto carve = [&](Arena& ar, int P) {
         ChunkView cv = chunk_carve(ar, P, NN);
         if (adj) {
@@ -1767,6 +1958,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
             cv.RW = ar.ptr<C2>(ar.take(z * NP * a.b * nw1 * P));
             cv.place = ar.ptr<int>(ar.take(sizeof(int) * (size_t)P));
         }
+        if (big) bv = big_carve(ar, P, a.nk, NP);
         return cv;
     };
     Arena one;
@@ -1809,7 +2001,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         const SweepPlArgs sa{v.h, v.psize, pH, pU, pL, pM, a.E + p0, kidx, prm->eta, prm->eta0, prm->device_eta_factor,
                              prm->eta_mode, need + p0, cv.sigma, cv.T, cv.sst, cv.keep, v.poff + a.adj_lo + 1, kept};
         if (p0) zero_dev(c, cnt, sizeof(int) * 2, s);
-        launch(c, NT_K_PLANES, 0, "plane decimation", [&] {
+        if (big) planes_big_leads(c, prm, a, v, h, bv, w, pH, pU, pL, pV, p0, n, cv);
+        else launch(c, NT_K_PLANES, 0, "plane decimation", [&] {
             if (!wait || h.nt == 1) launch_decimate<1>(da, 2 * n, s);
             if (!wait || h.nt == 2) launch_decimate<2>(da, 2 * n, s);
             if (!wait || h.nt == 3) launch_decimate<3>(da, 2 * n, s);
@@ -1828,6 +2021,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
             if (!wait || h.nt == 2) launch_sweep<2>(sa, 2 * n, s);
             if (!wait || h.nt == 3) launch_sweep<3>(sa, 2 * n, s);
             if (!wait || h.nt == 4) launch_sweep<4>(sa, 2 * n, s);
+            if (big) launch_sweep<PL_BIGNT>(sa, 2 * n, s);
             return hipGetLastError();
         });
         hipLaunchKernelGGL(k_pl_finish, dim3(nblk(n)), dim3(256), 0, s, n, cv.dst, cv.dit, cv.sst, cv.T, first,

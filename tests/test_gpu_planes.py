@@ -3,7 +3,7 @@
 Systems whose layers are made of planes of given sizes (couplings only inside
 a plane and to the next one), with the degrees of freedom of every layer in
 random order, so that the planes have to be found: sizes at the edges of the
-kernels' 16-column tiles and classes (16, 32, 48, 64), planes of different
+kernels' 16-column tiles and classes (16, 32, 48, 64, 96), planes of different
 sizes, leads of other sizes than the device, several k-points whose patterns
 differ.  T against the C oracle per point to max(1e-10, 256 eps kappa) (kappa
 the largest condition number the oracle inverts), gradients and left-out
@@ -99,7 +99,10 @@ def planes_launches(engine, call):
 CASES = [((1, 1), (1, 1), 1, None), ((9, 9), (9, 9), 3, None), ((16, 16), (16, 16), 2, None),
          ((17, 16), (16, 17), 2, None), ((5, 7, 6), (7, 5, 6, 4), 3, (8, 7)), ((32, 32), (32, 32), 2, None),
          ((33, 20), (20, 33), 2, None), ((48, 48, 48, 48), (48, 48), 2, None), ((49, 48), (30, 49), 2, None),
-         ((64, 64), (64, 64, 64), 1, None), ((63, 40, 50), (64, 33), 2, (40, 64))]
+         ((64, 64), (64, 64, 64), 1, None), ((63, 40, 50), (64, 33), 2, (40, 64)),
+         # planes of 65 to 96: the leads through the layers' decimation
+         ((70, 66), (65, 96), 2, None), ((65, 70, 80), (96, 70), 1, (66, 90, 70)),
+         ((65, 66, 67, 68), (66, 65), 1, None)]
 
 
 @pytest.mark.parametrize("lead,dev,L,lead_r", CASES)
@@ -114,8 +117,7 @@ def test_planes_vs_oracle(engine, T, planes_on, lead, dev, L, lead_r):
     print(f"planes: lead {lead} device {dev} L={L}", flush=True)
     d = engine.upload_blocks(blocks)
     r, used, inverses = planes_launches(engine, lambda: engine.solve_tdb(d, E, p, kidx=kidx, first_point_mask=mask))
-    # lim classes can merge two planes of a layer; at least one layer is divided
-    assert used > 0 and inverses == 0
+    assert used > 0 and (inverses == 0 or max(lead + dev) > 64)
     assert (r["status"].cpu().numpy() == 0).all()
     for i in range(2):
         sel = (kidx == i) & (mask == 0)
@@ -132,12 +134,15 @@ def test_planes_vs_oracle(engine, T, planes_on, lead, dev, L, lead_r):
     assert np.array_equal(r["iters"].cpu().numpy(), q["iters"].cpu().numpy())
 
 
-@pytest.mark.parametrize("dev,lo,hi", [((9, 9), 0, 2), ((16, 20), 1, 1), ((33, 20, 40), 2, 2), ((64, 30), 0, 1)])
+@pytest.mark.parametrize("dev,lo,hi", [((9, 9), 0, 2), ((16, 20), 1, 1), ((33, 20, 40), 2, 2), ((64, 30), 0, 1),
+                                       ((90, 65), 0, 2)])
 def test_planes_gradient(engine, T, planes_on, dev, lo, hi):
     """the gradient of the planes' sweep against the layers', whose own test is
-    finite differences; sums over 11 points of two k-points"""
+    finite differences; sums over 11 points of two k-points.  Tolerance: dT =
+    2 Re Tr[dH G Gamma G^+ Gamma G] has three factors G, each good to 256 eps
+    kappa (kappa the largest condition number the oracle inverts)."""
     p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13)
-    blocks = [plane_blocks((12, 10), dev, 3, 50 + i) for i in range(2)]
+    blocks = [plane_blocks((12, 10) if max(dev) <= 64 else (66, 65), dev, 3, 50 + i) for i in range(2)]
     rng = np.random.default_rng(4)
     E = rng.uniform(0.05, 0.9, 11)
     kidx = rng.integers(0, 2, 11).astype(np.int32)
@@ -145,12 +150,16 @@ def test_planes_gradient(engine, T, planes_on, dev, lo, hi):
     d = engine.upload_blocks(blocks)
     print(f"planes gradient: device {dev} window {lo}..{hi}", flush=True)
     r, used, inverses = planes_launches(engine, lambda: engine.solve_tdb_adjoint(d, E, p, w, lo, hi, kidx=kidx))
-    assert used > 0 and inverses == 0
+    assert used > 0 and (inverses == 0 or max(dev) > 64)
     engine.set_planes(False)
     q = engine.solve_tdb_adjoint(d, E, p, w, lo, hi, kidx=kidx)
+    kap = max(O.solve_tdb_batch_kappa(blocks[i].as_dict(), E[kidx == i], oparams(p), nthreads=4)[3].max()
+              for i in range(2) if (kidx == i).any())
+    tol = max(1e-10, 3 * 256 * EPS * kap)
+    print(f"  kappa {kap:.1e}, tolerance {tol:.1e}", flush=True)
     for k in ("T_LR", "T_RL", "dHamd", "dHamdv"):
         x, y = r[k].cpu().numpy(), q[k].cpu().numpy()
-        assert x.shape == y.shape and np.abs(x - y).max(initial=0.0) <= 1e-9 * max(1.0, np.abs(y).max(initial=0.0)), k
+        assert x.shape == y.shape and np.abs(x - y).max(initial=0.0) <= tol * max(1.0, np.abs(y).max(initial=0.0)), k
 
 
 def test_left_out_points_are_the_layers(engine, T, planes_on):

@@ -1927,6 +1927,7 @@ void tune_inverse(nt_ctx* c, int n, int batch, int* best_nb, double* best_ms)
     int bnb = widths[0];
     const bool prof = c->prof;
     c->prof = false;
+    c->tuning = true;
     for (int i = 0; i < k; ++i) {
         c->inv_nb[{(int)sizeof(T), n}] = widths[i];
         auto run = [&] {
@@ -1949,7 +1950,9 @@ void tune_inverse(nt_ctx* c, int n, int batch, int* best_nb, double* best_ms)
     c->prof = prof;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
+    c->tuning = false;
     c->inv_nb[{(int)sizeof(T), n}] = bnb;
+    if (sizeof(T) == 8) c->inv_tuned.insert(n);
     if (best_nb) *best_nb = bnb;
     if (best_ms) *best_ms = best;
 }
@@ -2945,6 +2948,7 @@ int nt_set_inverse_panel(nt_ctx* c, int n, int precision, int nb)
     if (!c || n <= 0 || n > inv_max_n()) return NT_ERR_ARG;
     if (precision != NT_PREC_FP64 && precision != NT_PREC_MIXED) return NT_ERR_ARG;
     const int bytes = precision == NT_PREC_FP64 ? 8 : 4;
+    if (bytes == 8) c->inv_tuned.erase(n);
     if (nb == 0) {
         c->inv_nb.erase({bytes, n});
         return NT_OK;

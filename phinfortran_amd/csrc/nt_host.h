@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -85,6 +86,11 @@ struct nt_ctx {
     // degenerate-group descriptors and statuses of the path_mode = 1 rotation
     void* deg_buf = nullptr;
     size_t deg_bytes = 0;
+    // inverses by panels only: set while points left out by the planes are
+    // solved, whose digits depend on the order of the sums
+    bool inv_panels = false;
+    std::set<int> inv_tuned;       // FP64 sizes whose width the autotuner chose
+    bool tuning = false;
     // batched FP64 solves on the planes of the layers (nt_planes.hip); its plan
     // and a pinned copy of the plan's header
     bool planes = true;
@@ -356,6 +362,10 @@ void inverse(nt_ctx* c, int n, BMatW<T> W, BMat<T> src, const T* z, BMatW<T> X, 
     a.batch = batch;
     auto tuned = c->inv_nb.find({(int)sizeof(T), n});
     a.nb = tuned == c->inv_nb.end() ? 0 : tuned->second;
+    // (a tuned width is one of the panel kernels', which up to INV_REG_MAX only
+    // a width set by the caller selects)
+    if (c->inv_panels) a.nb = a.nb ? a.nb : INV_PANELS;
+    else if (sizeof(T) == 8 && n <= INV_REG_MAX && !c->tuning && c->inv_tuned.count(n)) a.nb = 0;
     const double items = nitems < 0 ? (double)batch : nitems;
     audit<T>(c, W, n, n, batch, 1, "inverse W");
     audit<T>(c, src, n, n, batch, 1, "inverse src");

@@ -22,6 +22,7 @@
 // LDS: W planes NB x npad (npad = n rounded up to 16), a 16-column strip of
 // old pivot rows, the permutations and small exchange buffers.
 #include "nt_kernels.h"
+#include "nt_tile.h"
 
 namespace nt {
 
@@ -416,6 +417,71 @@ hipError_t launch_inv_t(const InvArgs<T>& a, hipStream_t s)
     }();
     (void)configured;
     hipLaunchKernelGGL((k_inv_gj<T, NB, RPT, MRT>), dim3(a.batch), dim3(NT), sm, s, a);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------
+// FP64, n <= 128: the whole matrix in the registers of ceil(n / 16) waves
+// (nt_tile.h), read and written once; the panels and pivot rows pass through
+// LDS.  Bound by the chain of pivots and by the matrix products, where the
+// kernel above reads and writes the matrix once per panel and waits for memory
+// in every strip: 64 matrices of n = 96 take the time given beside the
+// dispatch below.
+template <int NT>
+__global__ __launch_bounds__(64 * NT, 2) void k_inv_reg(InvArgs<double> a)
+{
+    constexpr int NP = 16 * NT, LD = NP + 1;
+    const int p = blockIdx.x;
+    if (a.active && !a.active[p]) return;
+    __shared__ C2 work[2 * 16 * LD + NT * 256];
+    __shared__ int piv[NP], cinv[NP], info;
+    if (threadIdx.x == 0) info = 0;
+    const int n = a.n, w = wave_id();
+    const double* S = a.src.base ? bptr(a.src, p, 0) : bptr(a.W, p, 0);
+    const int lds = a.src.base ? a.src.ld : a.W.ld;
+    const double zr = a.src.base ? a.z[2 * p] : 0.0, zi = a.src.base ? a.z[2 * p + 1] : 0.0;
+    const double sg = a.src.base ? -1.0 : 1.0;
+    Blk<NT> m;
+    __syncthreads();
+    {
+        const int lane = lane_new(), q = lane >> 4, col = 16 * w + (lane & 15);
+        bool nan = false;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * t + 4 * r + q;
+                C2 v = make_double2(row == col ? 1.0 : 0.0, 0.0);
+                if (row < n && col < n) {
+                    const C2 x = *reinterpret_cast<const C2*>(S + 2 * (row + (long)col * lds));
+                    v = make_double2((row == col ? zr : 0.0) + sg * x.x, (row == col ? zi : 0.0) + sg * x.y);
+                }
+                nan |= v.x != v.x || v.y != v.y;
+                m.re[t][r] = v.x;
+                m.im[t][r] = v.y;
+            }
+        if (nan) info = -1;
+    }
+    double* X = bptr(a.X, p, 0);
+    Grow gr;
+    const InvLds il{piv, cinv, &info};
+    wg_inverse<NT>(work, il, m, gr, [&](int i, int j, C2 v) {
+        if (i < n && j < n) *reinterpret_cast<C2*>(X + 2 * (i + (long)j * a.X.ld)) = v;
+    });
+    // merge into the caller's status: the first error of an item wins
+    if (threadIdx.x == 0 && info && a.info && a.info[p] == 0) a.info[p] = info;
+}
+
+hipError_t launch_inv_reg(const InvArgs<double>& a, hipStream_t s)
+{
+    const int nt = (a.n + 15) / 16;
+#define NT_REG(N) \
+    case N: hipLaunchKernelGGL(k_inv_reg<N>, dim3(a.batch), dim3(64 * N), 0, s, a); break;
+    switch (nt) {
+        NT_REG(1) NT_REG(2) NT_REG(3) NT_REG(4) NT_REG(5) NT_REG(6) NT_REG(7) NT_REG(8)
+        default: return hipErrorInvalidValue;
+    }
+#undef NT_REG
     return hipGetLastError();
 }
 
@@ -823,6 +889,9 @@ hipError_t launch_inv_any(const InvArgs<T>& a, hipStream_t s)
 {
     if (a.batch <= 0 || a.n <= 0) return hipSuccess;
     if (a.n > inv_max_n()) return hipErrorInvalidValue;
+    if constexpr (sizeof(T) == 8) {
+        if (a.n <= INV_REG_MAX && a.nb == 0) return launch_inv_reg(a, s);
+    }
     int w[INV_MAX_WIDTHS];
     const int k = inv_panel_widths<T>(a.n, w);
     // default: 16 columns where it fits (measured fastest at b = 192: two

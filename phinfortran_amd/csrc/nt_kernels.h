@@ -49,6 +49,10 @@ int inv_max_n();
 // panel widths launch_inv accepts for an n x n matrix of type T (largest first);
 // INV_BLOCKED selects the panel-kernel + batched-GEMM path (last in the list)
 constexpr int INV_BLOCKED = 1;
+// FP64 up to INV_REG_MAX without a requested width: the matrix in registers;
+// INV_PANELS requests the default among the panel widths instead
+constexpr int INV_REG_MAX = 128;
+constexpr int INV_PANELS = -1;
 constexpr int INV_MAX_WIDTHS = 6;
 template <typename T> int inv_panel_widths(int n, int* out);
 

@@ -57,6 +57,7 @@ int prepare_workers(nt_ctx* c, int W)
         s->worker = true;
         s->adj_ckpt = c->adj_ckpt;
         s->inv_nb = c->inv_nb;
+        s->inv_tuned = c->inv_tuned;
         s->gemm_tile = c->gemm_tile;
         s->prof = c->prof;
         s->ws_poison = c->ws_poison;

@@ -265,3 +265,29 @@ def test_zinv_singular_and_nan_n96(engine, torch_dev, width):
     inf = info.cpu().numpy()
     assert inf[0] == 41
     assert inf[1] == -1
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 33, 47, 48, 49, 64, 65, 80, 81, 96, 97, 112, 113, 127, 128])
+@pytest.mark.parametrize("batch", [1, 5])
+def test_zinv_in_registers(engine, torch_dev, n, batch):
+    """the default FP64 inverse up to n = 128 (edges of its 16-column waves and
+    of its one and two rows per lane), with rows that must be exchanged"""
+    from phinfortran_amd import _native as N
+    torch, dev = torch_dev
+    rng = np.random.default_rng(300 + n)
+    A = [crand(rng, n, n) for _ in range(batch)]
+    A[0][0, 0] = 0.0 if n > 1 else 2.0
+    dA = to_dev(torch, dev, A)
+    dX = torch.zeros_like(dA)
+    info = torch.zeros(batch, dtype=torch.int32, device=dev)
+    print(f"zinv in registers n={n} batch={batch}", flush=True)
+    st = N.lib().nt_zinv_batched_dev(engine.ctx, n, C.c_void_p(dA.data_ptr()), n * n, C.c_void_p(dX.data_ptr()),
+                                     n * n, C.c_void_p(info.data_ptr()), batch)
+    assert st == 0
+    engine.sync()
+    assert (info.cpu().numpy() == 0).all()
+    X = from_dev(dX)
+    for i in range(batch):
+        ref = np.linalg.inv(A[i])
+        # as for the panel kernels: eps n cond, and n for the growth of the pivots
+        assert np.abs(X[i] - ref).max() < 1e-14 * np.linalg.cond(A[i]) * np.abs(ref).max() * n, i

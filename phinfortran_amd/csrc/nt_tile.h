@@ -293,7 +293,8 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             double xr[RPL][16], xi[RPL][16];
-            bool free_row[RPL];
+            double svr = 0.0, svi = 0.0;     // 1 / pivot of a row that became one here
+            bool free_row[RPL], here = false;
             int row[RPL];
 #pragma unroll
             for (int l = 0; l < RPL; ++l) {
@@ -306,11 +307,8 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
                     xi[l][c] = v.y;
                 }
             }
-            // column c is always element 0: the columns move down by one per
-            // step and the finished one goes to the end, so the loop needs no
-            // register indexing
-#pragma unroll 1
-            for (int c = 0; c < 16; ++c) {
+            // largest |re| + |im| of column 0's free rows, the row in the low bits
+            auto pivot_key = [&]() __attribute__((always_inline)) {
                 unsigned key = 0;
 #pragma unroll
                 for (int l = 0; l < RPL; ++l) {
@@ -319,62 +317,141 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
                     const unsigned k = free_row[l] ? ((hi & ~(unsigned)KM) | (unsigned)(64 * RPL - 64 * l - lane)) : 0u;
                     key = k > key ? k : key;
                 }
-                const int p =
-                    __builtin_amdgcn_readfirstlane(64 * RPL - (int)(wave_max(key) & (unsigned)KM)), pl = p & 63;
-                // the step with the pivot row in slot SL of its lane
-                auto step = [&](auto slot) __attribute__((always_inline)) {
-                    constexpr int SL = decltype(slot)::value;
-                    const double dr = read_lane(xr[SL][0], pl), di = read_lane(xi[SL][0], pl);
-                    const double den = dr * dr + di * di;
-                    double vr = 0.0, vi = 0.0;      // 1 / pivot
-                    if (den != 0.0) {
-                        const double rc = 1.0 / den;
-                        vr = dr * rc;
-                        vi = -di * rc;
-                    }
-                    if (lane == 0) {
-                        s.piv[16 * J + c] = p;
-                        s.cinv[p] = 16 * J + c;
-                        if (!(den > 0.0) || den > s.big) {
-                            if (*s.info == 0) *s.info = den == 0.0 ? 16 * J + c + 1 : -1;
-                        }
-                    }
-                    // multiplier f / pivot; the pivot row becomes row / pivot
-                    double gxr[RPL], gxi[RPL], keep[RPL];
-#pragma unroll
-                    for (int l = 0; l < RPL; ++l) {
-                        const bool own = l == SL && lane == pl;
-                        if (own) free_row[l] = false;
-                        const double fr = xr[l][0], fi = xi[l][0];
-                        gxr[l] = own ? -vr : fr * vr - fi * vi;
-                        gxi[l] = own ? -vi : fr * vi + fi * vr;
-                        keep[l] = own ? 0.0 : 1.0;
-                    }
+                return wave_max(key) & (unsigned)KM;
+            };
+            // Column c is always element 0: the columns move down by one per
+            // step and the finished one goes to the end, so the loop needs no
+            // register indexing.  One wave works here and the steps follow on
+            // one another, so what counts is the chain from pivot to pivot.
+            // With one row per lane (NP <= 64) the pivot row is read into
+            // scalars at once, the next column is updated first and its pivot
+            // search overlaps the other columns' updates, the pivot row is
+            // scaled after the panel (a row's multipliers scale with it) and
+            // there is no branch in a step: 4096 matrices of 48 take 262 us
+            // (293 with the step below), of 64 534 (603).  With two rows per
+            // lane the registers do not hold that row beside the panel: the
+            // same order spills (96: 2830 us, against 2507), so there the
+            // pivot row is read as it is used and scaled in its step.
+            if constexpr (RPL == 1) {
+                unsigned key = pivot_key();
+                int pv = 0;          // lane c: pivot row of column c and its |pivot|^2
+                double dn = 1.0;
+#pragma unroll 1
+                for (int c = 0; c < 16; ++c) {
+                    const int pl = __builtin_amdgcn_readfirstlane(64 - (int)key);
+                    const double dr = read_lane(xr[0][0], pl), di = read_lane(xi[0][0], pl);
+                    double pr[16], pim[16];
 #pragma unroll
                     for (int j = 1; j < 16; ++j) {
-                        const double pr = read_lane(xr[SL][j], pl), pim = read_lane(xi[SL][j], pl);
+                        pr[j] = read_lane(xr[0][j], pl);
+                        pim[j] = read_lane(xi[0][j], pl);
+                    }
+                    const double den = dr * dr + di * di;
+                    // 1 / den: the instruction's estimate and two Newton steps
+                    double rc = __builtin_amdgcn_rcp(den);
+                    rc = fma(rc, fma(-den, rc, 1.0), rc);
+                    rc = fma(rc, fma(-den, rc, 1.0), rc);
+                    rc = den != 0.0 ? rc : 0.0;
+                    const double vr = dr * rc, vi = -di * rc;      // 1 / pivot
+                    const bool own = lane == pl;
+                    const double fr = xr[0][0], fi = xi[0][0];
+                    const double tr = fr * vr - fi * vi, ti = fr * vi + fi * vr;
+                    const double gxr = own ? 0.0 : tr, gxi = own ? 0.0 : ti;    // multiplier f / pivot
+                    free_row[0] = free_row[0] && !own;
+                    here = here || own;
+                    svr = own ? vr : svr;
+                    svi = own ? vi : svi;
+                    xr[0][0] = fma(gxi, pim[1], fma(-gxr, pr[1], xr[0][1]));
+                    xi[0][0] = fma(-gxi, pr[1], fma(-gxr, pim[1], xi[0][1]));
+                    pv = lane == c ? pl : pv;
+                    dn = lane == c ? den : dn;
+                    key = pivot_key();
+#pragma unroll
+                    for (int j = 2; j < 16; ++j) {
+                        xr[0][j - 1] = fma(-gxr, pr[j], xr[0][j]);
+                        xi[0][j - 1] = fma(-gxr, pim[j], xi[0][j]);
+                    }
+#pragma unroll
+                    for (int j = 2; j < 16; ++j) {
+                        xr[0][j - 1] = fma(gxi, pim[j], xr[0][j - 1]);
+                        xi[0][j - 1] = fma(-gxi, pr[j], xi[0][j - 1]);
+                    }
+                    xr[0][15] = own ? 1.0 : -gxr;
+                    xi[0][15] = own ? 0.0 : -gxi;
+                }
+                // the panel's pivots: their record, the first bad one, their rows' scale
+                if (lane < 16) {
+                    s.piv[16 * J + lane] = pv;
+                    s.cinv[pv] = 16 * J + lane;
+                }
+                const unsigned long long bad = __ballot(lane < 16 && (!(dn > 0.0) || dn > s.big));
+                if (bad && *s.info == 0) {
+                    const int c = __ffsll((long long)bad) - 1;
+                    if (lane == c) *s.info = dn == 0.0 ? 16 * J + c + 1 : -1;
+                }
+            } else {
+#pragma unroll 1
+                for (int c = 0; c < 16; ++c) {
+                    const int p = __builtin_amdgcn_readfirstlane(64 * RPL - (int)pivot_key()), pl = p & 63;
+                    // the step with the pivot row in slot SL of its lane
+                    auto step = [&](auto slot) __attribute__((always_inline)) {
+                        constexpr int SL = decltype(slot)::value;
+                        const double dr = read_lane(xr[SL][0], pl), di = read_lane(xi[SL][0], pl);
+                        const double den = dr * dr + di * di;
+                        double vr = 0.0, vi = 0.0;      // 1 / pivot
+                        if (den != 0.0) {
+                            const double rc = 1.0 / den;
+                            vr = dr * rc;
+                            vi = -di * rc;
+                        }
+                        if (lane == 0) {
+                            s.piv[16 * J + c] = p;
+                            s.cinv[p] = 16 * J + c;
+                            if (!(den > 0.0) || den > s.big) {
+                                if (*s.info == 0) *s.info = den == 0.0 ? 16 * J + c + 1 : -1;
+                            }
+                        }
+                        // multiplier f / pivot; the pivot row becomes row / pivot
+                        double gxr[RPL], gxi[RPL], keep[RPL];
 #pragma unroll
                         for (int l = 0; l < RPL; ++l) {
-                            const double a = l == SL ? xr[l][j] * keep[l] : xr[l][j];
-                            const double b = l == SL ? xi[l][j] * keep[l] : xi[l][j];
-                            xr[l][j - 1] = a - gxr[l] * pr + gxi[l] * pim;
-                            xi[l][j - 1] = b - gxr[l] * pim - gxi[l] * pr;
+                            const bool own = l == SL && lane == pl;
+                            if (own) free_row[l] = false;
+                            const double fr = xr[l][0], fi = xi[l][0];
+                            gxr[l] = own ? -vr : fr * vr - fi * vi;
+                            gxi[l] = own ? -vi : fr * vi + fi * vr;
+                            keep[l] = own ? 0.0 : 1.0;
                         }
-                    }
 #pragma unroll
-                    for (int l = 0; l < RPL; ++l) {
-                        xr[l][15] = -gxr[l];
-                        xi[l][15] = -gxi[l];
-                    }
-                };
-                if (RPL == 1 || p < 64) step(std::integral_constant<int, 0>{});
-                else step(std::integral_constant<int, RPL - 1>{});
+                        for (int j = 1; j < 16; ++j) {
+                            const double pr = read_lane(xr[SL][j], pl), pim = read_lane(xi[SL][j], pl);
+#pragma unroll
+                            for (int l = 0; l < RPL; ++l) {
+                                const double a = l == SL ? xr[l][j] * keep[l] : xr[l][j];
+                                const double b = l == SL ? xi[l][j] * keep[l] : xi[l][j];
+                                xr[l][j - 1] = a - gxr[l] * pr + gxi[l] * pim;
+                                xi[l][j - 1] = b - gxr[l] * pim - gxi[l] * pr;
+                            }
+                        }
+#pragma unroll
+                        for (int l = 0; l < RPL; ++l) {
+                            xr[l][15] = -gxr[l];
+                            xi[l][15] = -gxi[l];
+                        }
+                    };
+                    if (p < 64) step(std::integral_constant<int, 0>{});
+                    else step(std::integral_constant<int, RPL - 1>{});
+                }
             }
 #pragma unroll
             for (int l = 0; l < RPL; ++l)
                 if (lane + 64 * l < NP) {
 #pragma unroll
-                    for (int c = 0; c < 16; ++c) wb[c * LD + row[l]] = make_double2(xr[l][c], xi[l][c]);
+                    for (int c = 0; c < 16; ++c) {
+                        C2 v = make_double2(xr[l][c], xi[l][c]);
+                        if (RPL == 1 && here) v = make_double2(v.x * svr - v.y * svi, v.x * svi + v.y * svr);
+                        wb[c * LD + row[l]] = v;
+                    }
                 }
             // (a barrier in either branch: m is not live while its wave sweeps)
             __syncthreads();

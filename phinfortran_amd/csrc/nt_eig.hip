@@ -1,6 +1,7 @@
 // nt_eig.hip -- batched complex Schur decomposition, eigenvectors and
 // principal matrix square root (FP64), one workgroup of 256 threads per
-// matrix, working matrices in global memory (L2-resident at these sizes).
+// matrix, working matrices in global memory (L2-resident at these sizes; up
+// to n = 96 the decomposition keeps its matrix in LDS).
 //
 // These replace the LAPACK calls of the mode-resolved transmission:
 //   eigen  (negf/util.f90:226-262, ZGEEV)  -> k_schur + k_trevc + gemm + k_ev_normalize
@@ -92,6 +93,25 @@ __device__ __forceinline__ double* coef_red(unsigned char* base, int n)
     return reinterpret_cast<double*>(coef + n);
 }
 
+// item p of either set
+struct EigItem {
+    double *A, *Z, *X, *w;
+    int* status;
+};
+__device__ __forceinline__ EigItem eig_item(const EigArgs& a, int p)
+{
+    const bool two = p >= a.batch;
+    const int q = two ? p - a.batch : p;
+    EigItem e;
+    e.A = bptr(two ? a.A2 : a.A, q, 0);
+    e.Z = bptr(two ? a.Z2 : a.Z, q, 0);
+    e.X = bptr(two ? a.X2 : a.X, q, 0);
+    e.w = two ? a.w2 : a.w;
+    if (e.w) e.w += 2 * (long)q * a.n;
+    e.status = a.status ? a.status + q : nullptr;
+    return e;
+}
+
 struct SchurShared {
     double red[4];
     int ired[4];
@@ -106,7 +126,8 @@ struct SchurShared {
 __global__ __launch_bounds__(NT) void k_schur(EigArgs a)
 {
     const int p = blockIdx.x;
-    if (p >= a.batch) return;
+    if (p >= a.sets * a.batch) return;
+    const EigItem it = eig_item(a, p);
     const int n = a.n;
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
@@ -114,8 +135,7 @@ __global__ __launch_bounds__(NT) void k_schur(EigArgs a)
     extern __shared__ __align__(16) unsigned char smem_raw[];
     C2* v = reinterpret_cast<C2*>(smem_raw);     // [n] Householder vector
 
-    double* A = bptr(a.A, p, 0);
-    double* Z = bptr(a.Z, p, 0);
+    double *A = it.A, *Z = it.Z;
     const int lda = a.A.ld, ldz = a.Z.ld;
 
     // Z = I
@@ -318,17 +338,325 @@ __global__ __launch_bounds__(NT) void k_schur(EigArgs a)
         const int r = (int)(e % n), c = (int)(e / n);
         if (r > c) st(A, lda, r, c, C2{0.0, 0.0});
     }
-    if (t == 0 && a.status) {
+    if (t == 0 && it.status) {
         const int v = S.status;
-        if (v && a.status[p] == 0) a.status[p] = v;
+        if (v && *it.status == 0) *it.status = v;
     }
-    if (a.w) {
+    if (it.w) {
         for (int i = t; i < n; i += NT) {
             const C2 d = ld(A, lda, i, i);
-            a.w[2 * ((long)p * n + i)] = d.r;
-            a.w[2 * ((long)p * n + i) + 1] = d.i;
+            it.w[2 * i] = d.r;
+            it.w[2 * i + 1] = d.i;
         }
     }
+}
+
+// The same decomposition with the matrix in LDS, for n <= NS.  k_schur takes
+// about 1 us per rotation: three barriers around one thread's scalar chain,
+// rows and columns through L2.  Here a sweep is split by what its chain needs.
+// Rotation j+1 follows from rows j+1 and j+2 alone, so one wave runs down the
+// window with a row per register and a column per lane (RS columns from 65 on):
+// no barrier, the next row loaded ahead.  The rotations of the columns commute
+// with those of the rows; above the diagonal they come afterwards, one thread
+// per row, and those of Z one sweep later by two other waves, beside the next
+// sweep's rows.  Bound by that one wave's chain of dependent FP64 operations
+// per rotation.  128 matrices of n = 96: 4.8 ms (k_schur 9.6), 256 of them the
+// same: a workgroup has a CU to itself.
+namespace {
+
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// rotation [c s; -conj(s) c] with (f, g) -> (r, 0)
+__device__ __forceinline__ void make_rotation(C2 f, C2 g, double& c, C2& s, C2& r)
+{
+    const double f2 = f.r * f.r + f.i * f.i, g2 = g.r * g.r + g.i * g.i, h2 = f2 + g2;
+    if (f2 > 1e-140 && g2 > 1e-140 && h2 < 1e140) {
+        const double d = rsqrt(f2 * h2);
+        c = f2 * d;
+        s = cscale(cmul(f, cconj(g)), d);
+        r = cscale(f, h2 * d);
+    } else if (g.r == 0.0 && g.i == 0.0) {
+        c = 1.0;
+        s = C2{0.0, 0.0};
+        r = f;
+    } else if (f.r == 0.0 && f.i == 0.0) {
+        const double ag = cabs(g);
+        c = 0.0;
+        s = cscale(cconj(g), 1.0 / ag);
+        r = C2{ag, 0.0};
+    } else {
+        const double af = cabs(f), ag = cabs(g), d = hypot(af, ag);
+        const C2 ph = cscale(f, 1.0 / af);
+        c = af / d;
+        s = cscale(cmul(ph, cconj(g)), 1.0 / d);
+        r = cscale(ph, d);
+    }
+}
+
+// columns l..m of one row by the rotations from j0 on, four columns in flight
+__device__ __forceinline__ void rotate_row(double2* x0, long ldx, int l, int j0, int m, const double* rc, const C2* rs)
+{
+    if (j0 >= m) return;
+    double2 x = x0[j0 * ldx];
+    for (int j = l; j < m; j += 4) {
+        double2 y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) y[u] = x0[(j + u < m ? j + u + 1 : m) * ldx];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (j + u >= j0 && j + u < m) {
+                const double c = rc[j + u];
+                const C2 s = rs[j + u];
+                x0[(j + u) * ldx] = make_double2(c * x.x + (s.r * y[u].x + s.i * y[u].y),
+                                                 c * x.y + (s.r * y[u].y - s.i * y[u].x));
+                x = make_double2(c * y[u].x - (s.r * x.x - s.i * x.y), c * y[u].y - (s.r * x.y + s.i * x.x));
+            }
+        }
+    }
+    x0[m * ldx] = x;
+}
+
+}  // namespace
+
+template <int NS>
+__global__ __launch_bounds__(NT) void k_schur_lds(EigArgs a)
+{
+    constexpr int LD = NS + 1, RS = (NS + 63) / 64;
+    static_assert(NS <= 128 && NT >= 256, "two waves of rows");
+    __shared__ double2 H[NS * LD];
+    __shared__ C2 v[NS], rs[2][NS];
+    __shared__ double rc[2][NS];
+    __shared__ C2 s_tau;
+    __shared__ int s_l, s_m, s_status;
+    const int p = blockIdx.x, n = a.n, t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const EigItem it = eig_item(a, p);
+    double2 *A = reinterpret_cast<double2*>(it.A), *Z = reinterpret_cast<double2*>(it.Z);
+    const long lda = a.A.ld, ldz = a.Z.ld;
+    auto at = [&](int r, int c) -> double2& { return H[c * LD + r]; };
+    auto get = [&](int r, int c) { const double2 x = at(r, c); return C2{x.x, x.y}; };
+    const int zr = t - 128;                    // this thread's row of Z
+    const bool has_z = zr >= 0 && zr < n;
+    for (int e = t; e < n * n; e += NT) {
+        const int c = e / n, r = e - c * n;
+        at(r, c) = A[r + c * lda];
+    }
+    if (has_z)
+        for (int c = 0; c < n; ++c) Z[zr + c * ldz] = make_double2(zr == c ? 1.0 : 0.0, 0.0);
+    if (t == 0) s_status = 0;
+    __syncthreads();
+
+    // ---- Hessenberg reduction
+    for (int k = 0; k + 2 < n; ++k) {
+        const int m = n - k - 1;               // length of v
+        if (wave == 0) {
+            double xs = 0.0;
+            for (int i = k + 2 + lane; i < n; i += 64) {
+                const C2 x = get(i, k);
+                xs += x.r * x.r + x.i * x.i;
+            }
+            xs = wave_sum(xs);
+            const C2 alpha = get(k + 1, k);
+            C2 tau{0.0, 0.0};
+            if (!(xs == 0.0 && alpha.i == 0.0)) {
+                const double nrm = sqrt(alpha.r * alpha.r + alpha.i * alpha.i + xs);
+                const double beta = alpha.r >= 0.0 ? -nrm : nrm;
+                tau = C2{(beta - alpha.r) / beta, -alpha.i / beta};
+                const C2 scale = cdiv(C2{1.0, 0.0}, csub(alpha, C2{beta, 0.0}));
+                for (int i = lane; i < m; i += 64) {
+                    v[i] = i == 0 ? C2{1.0, 0.0} : cmul(get(k + 1 + i, k), scale);
+                    at(k + 1 + i, k) = make_double2(i == 0 ? beta : 0.0, 0.0);
+                }
+            }
+            if (lane == 0) s_tau = tau;
+        }
+        __syncthreads();
+        const C2 tau = s_tau;
+        if (tau.r != 0.0 || tau.i != 0.0) {    // uniform
+            // left: A[k+1:, j] -= conj(tau) v (v^H A[k+1:, j]), one thread per column j > k;
+            // right on Z beside it: Z[r, k+1:] -= tau (Z[r, k+1:] v) v^H, one thread per row
+            if (t < 128) {
+                const int j = k + 1 + t;
+                if (j < n) {
+                    double2* x = &at(k + 1, j);
+                    C2 f{0.0, 0.0};
+#pragma unroll 4
+                    for (int i = 0; i < m; ++i) f = cadd(f, cmul(cconj(v[i]), C2{x[i].x, x[i].y}));
+                    f = cmul(cconj(tau), f);
+#pragma unroll 4
+                    for (int i = 0; i < m; ++i) {
+                        const C2 y = csub(C2{x[i].x, x[i].y}, cmul(v[i], f));
+                        x[i] = make_double2(y.r, y.i);
+                    }
+                }
+            } else if (has_z) {
+                double2* x = Z + zr + (k + 1) * ldz;
+                C2 f{0.0, 0.0};
+#pragma unroll 8
+                for (int i = 0; i < m; ++i) f = cadd(f, cmul(C2{x[i * ldz].x, x[i * ldz].y}, v[i]));
+                f = cmul(tau, f);
+#pragma unroll 8
+                for (int i = 0; i < m; ++i) {
+                    const C2 y = csub(C2{x[i * ldz].x, x[i * ldz].y}, cmul(f, cconj(v[i])));
+                    x[i * ldz] = make_double2(y.r, y.i);
+                }
+            }
+            __syncthreads();
+            // right on A: one thread per row
+            if (t < n) {
+                double2* x = &at(t, k + 1);
+                C2 f{0.0, 0.0};
+#pragma unroll 4
+                for (int i = 0; i < m; ++i) f = cadd(f, cmul(C2{x[i * LD].x, x[i * LD].y}, v[i]));
+                f = cmul(tau, f);
+#pragma unroll 4
+                for (int i = 0; i < m; ++i) {
+                    const C2 y = csub(C2{x[i * LD].x, x[i * LD].y}, cmul(f, cconj(v[i])));
+                    x[i * LD] = make_double2(y.r, y.i);
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    // ---- shifted QR sweeps
+    const int itmax = 30 * (n > 10 ? n : 10), totmax = 60 * n + 60;
+    int mw = n - 1, its = 0, total = 0;        // wave 0's
+    int zl = 0, zm = 0;                        // window of the sweep Z still lacks
+    // uniform index j: lane j & 63, register j >> 6
+    auto pick = [&](const C2 (&row)[RS], int j) {
+        const C2 x = RS == 1 || j < 64 ? row[0] : row[RS - 1];
+        return C2{lane_value(x.r, j & 63), lane_value(x.i, j & 63)};
+    };
+    for (int buf = 0;; buf ^= 1) {
+        if (wave == 0) {
+            int l = 0;
+            while (mw >= 0) {
+                // deflation: largest k in (0, m] with a negligible subdiagonal
+                l = 0;
+#pragma unroll
+                for (int q = 0; q < RS; ++q) {
+                    const int k = lane + 64 * q;
+                    bool small = false;
+                    if (k >= 1 && k <= mw) {
+                        const double sub = cabs1(get(k, k - 1));
+                        const double tst = cabs1(get(k - 1, k - 1)) + cabs1(get(k, k));
+                        small = sub <= 100.0 * SAFMIN || sub <= ULP * tst;
+                    }
+                    const unsigned long long b = __ballot(small);
+                    if (b) l = 64 * q + 63 - __clzll((long long)b);
+                }
+                if (l > 0 && lane == 0) at(l, l - 1) = make_double2(0.0, 0.0);
+                if (l < mw) break;
+                --mw;
+                its = 0;
+            }
+            int status = 0;
+            if (mw >= 0) {
+                ++its;
+                ++total;
+                if (its > itmax || total > totmax) status = -3;
+            }
+            if (mw >= 0 && !status) {
+                const int m = mw;
+                C2 mu;
+                if (its % 10 == 0) {
+                    const C2 hm = get(m, m);
+                    mu = C2{hm.r + 0.75 * fabs(get(m, m - 1).r), hm.i};
+                } else {
+                    const C2 aa = get(m - 1, m - 1), bb = get(m - 1, m), cc = get(m, m - 1), dd = get(m, m);
+                    const C2 tr = cscale(csub(aa, dd), 0.5);
+                    const C2 disc = csqrt_p(cadd(cmul(tr, tr), cmul(bb, cc)));
+                    const C2 e1 = cadd(cadd(dd, tr), disc), e2 = csub(cadd(dd, tr), disc);
+                    mu = cabs(csub(e1, dd)) < cabs(csub(e2, dd)) ? e1 : e2;
+                }
+                C2 cur[RS], nxt[RS], ahead[RS];
+                int col[RS];
+#pragma unroll
+                for (int q = 0; q < RS; ++q) {
+                    col[q] = lane + 64 * q < n ? lane + 64 * q : n - 1;
+                    cur[q] = get(l, col[q]);
+                    nxt[q] = get(l + 1, col[q]);
+                }
+                C2 f = csub(pick(cur, l), mu), g = pick(nxt, l);
+                double c = 1.0;
+                C2 s{0.0, 0.0};
+                for (int j = l; j < m; ++j) {
+                    const int ra = j + 2 <= m ? j + 2 : m;
+#pragma unroll
+                    for (int q = 0; q < RS; ++q) ahead[q] = get(ra, col[q]);
+                    C2 r{0.0, 0.0}, d{0.0, 0.0}, b{0.0, 0.0};
+                    if (j > l) {
+                        // rotation j - 1 on columns j - 1 and j of rows j and j + 1
+                        const C2 x = pick(cur, j - 1), y = pick(cur, j), y1 = pick(nxt, j);
+                        f = cadd(cscale(x, c), cmul(cconj(s), y));
+                        d = csub(cscale(y, c), cmul(s, x));
+                        g = cmul(cconj(s), y1);
+                        b = cscale(y1, c);
+                    }
+                    make_rotation(f, g, c, s, r);
+#pragma unroll
+                    for (int q = 0; q < RS; ++q) {
+                        const int k = lane + 64 * q;
+                        if (j > l && k == j) {
+                            cur[q] = d;
+                            nxt[q] = b;
+                        }
+                        const C2 u = cadd(cscale(cur[q], c), cmul(s, nxt[q]));
+                        const C2 w = csub(cscale(nxt[q], c), cmul(cconj(s), cur[q]));
+                        const bool left = j > l && k == j - 1;
+                        const C2 o = left ? r : u;
+                        if (k < n && (left || k >= j)) at(j, k) = make_double2(o.r, o.i);
+                        cur[q] = w;
+                        nxt[q] = ahead[q];
+                    }
+                    if (lane == 0) {
+                        rc[buf][j] = c;
+                        rs[buf][j] = s;
+                    }
+                }
+                // the last row: its columns m - 1 and m by the last rotation
+                const C2 x = pick(cur, m - 1), y = pick(cur, m);
+                const C2 e = cadd(cscale(x, c), cmul(cconj(s), y)), d = csub(cscale(y, c), cmul(s, x));
+#pragma unroll
+                for (int q = 0; q < RS; ++q) {
+                    const int k = lane + 64 * q;
+                    const C2 o = k == m - 1 ? e : k == m ? d : cur[q];
+                    if (k < n && k >= m - 1) at(m, k) = make_double2(o.r, o.i);
+                }
+            }
+            if (lane == 0) {
+                s_l = l;
+                s_m = status ? -1 : mw;
+                if (status) s_status = status;
+            }
+        } else if (has_z && zl < zm) {
+            rotate_row(Z + zr, ldz, zl, zl, zm, rc[buf ^ 1], rs[buf ^ 1]);
+        }
+        __syncthreads();
+        const int l = s_l, m = s_m;
+        if (m < 0) break;
+        if (t <= m && t < 128) rotate_row(&at(t, 0), LD, l, t > l ? t : l, m, rc[buf], rs[buf]);
+        zl = l;
+        zm = m;
+        __syncthreads();
+    }
+    __syncthreads();
+    for (int e = t; e < n * n; e += NT) {
+        const int c = e / n, r = e - c * n;
+        A[r + c * lda] = r > c ? make_double2(0.0, 0.0) : at(r, c);
+    }
+    if (t == 0 && it.status && s_status && *it.status == 0) *it.status = s_status;
+    if (it.w)
+        for (int i = t; i < n; i += NT) {
+            it.w[2 * i] = at(i, i).x;
+            it.w[2 * i + 1] = at(i, i).y;
+        }
 }
 
 // ------------------------------------------------------------ eigenvectors
@@ -339,11 +667,12 @@ __global__ __launch_bounds__(NT) void k_trevc(EigArgs a)
 {
     const int p = blockIdx.y;
     const int k = blockIdx.x * NT + threadIdx.x;
-    if (p >= a.batch) return;
+    if (p >= a.sets * a.batch) return;
     const int n = a.n;
     if (k >= n) return;
-    const double* T = bptr(a.A, p, 0);
-    double* X = bptr(a.X, p, 0);
+    const EigItem it = eig_item(a, p);
+    const double* T = it.A;
+    double* X = it.X;
     const int lt = a.A.ld, lx = a.X.ld;
     for (int i = k + 1; i < n; ++i) st(X, lx, i, k, C2{0.0, 0.0});
     st(X, lx, k, k, C2{1.0, 0.0});
@@ -428,11 +757,12 @@ __global__ __launch_bounds__(NT) void k_ev_normalize(EigArgs a)
 __global__ __launch_bounds__(NT) void k_sqrt_tri(EigArgs a)
 {
     const int p = blockIdx.x;
-    if (p >= a.batch) return;
+    if (p >= a.sets * a.batch) return;
     const int n = a.n;
     const int t = threadIdx.x;
-    const double* T = bptr(a.A, p, 0);
-    double* U = bptr(a.X, p, 0);
+    const EigItem it = eig_item(a, p);
+    const double* T = it.A;
+    double* U = it.X;
     const int lt = a.A.ld, lu = a.X.ld;
     for (long e = t; e < (long)n * n; e += NT) {
         const int r = (int)(e % n), c = (int)(e / n);
@@ -455,14 +785,18 @@ hipError_t launch_schur(const EigArgs& a, hipStream_t s)
 {
     if (a.batch <= 0 || a.n <= 0) return hipSuccess;
     const size_t sm = sizeof(C2) * (size_t)a.n;
-    hipLaunchKernelGGL(k_schur, dim3(a.batch), dim3(NT), sm, s, a);
+    // the 160 KB of LDS hold the matrix up to n = 96 (128 matrices: 4.8 ms, through L2 9.6)
+    if (a.n <= 32) hipLaunchKernelGGL(k_schur_lds<32>, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
+    else if (a.n <= 64) hipLaunchKernelGGL(k_schur_lds<64>, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
+    else if (a.n <= 96) hipLaunchKernelGGL(k_schur_lds<96>, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
+    else hipLaunchKernelGGL(k_schur, dim3(a.sets * a.batch), dim3(NT), sm, s, a);
     return hipGetLastError();
 }
 
 hipError_t launch_trevc(const EigArgs& a, hipStream_t s)
 {
     if (a.batch <= 0 || a.n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_trevc, dim3((a.n + NT - 1) / NT, a.batch), dim3(NT), 0, s, a);
+    hipLaunchKernelGGL(k_trevc, dim3((a.n + NT - 1) / NT, a.sets * a.batch), dim3(NT), 0, s, a);
     return hipGetLastError();
 }
 
@@ -476,7 +810,7 @@ hipError_t launch_ev_normalize(const EigArgs& a, hipStream_t s)
 hipError_t launch_sqrt_tri(const EigArgs& a, hipStream_t s)
 {
     if (a.batch <= 0 || a.n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_sqrt_tri, dim3(a.batch), dim3(NT), 0, s, a);
+    hipLaunchKernelGGL(k_sqrt_tri, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
     return hipGetLastError();
 }
 

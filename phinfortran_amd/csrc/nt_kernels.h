@@ -66,6 +66,11 @@ struct EigArgs {
     double* w;           // optional eigenvalues (n complex per item)
     int* status;         // merged: first error of an item wins (-3: QR did not converge)
     int batch;
+    // a second set of batch matrices in the same launch (schur, trevc, sqrt_tri),
+    // same n and leading dimensions; item q of either set reports to status[q]
+    int sets = 1;
+    BMatW<double> A2, Z2, X2;
+    double* w2 = nullptr;
 };
 hipError_t launch_schur(const EigArgs& a, hipStream_t s);
 hipError_t launch_trevc(const EigArgs& a, hipStream_t s);

@@ -18,10 +18,19 @@ size_t eig_scratch(int n, int batch)
     return a.off;
 }
 
-// w, V from A (A is copied, not modified).  The eigenvector matrix is Z X
-// with X the triangular eigenvectors of T.
-void eig_run(nt_ctx* c, int n, BMat<double> A, double* w, BMatW<double> V, int* status, int batch, Arena& ar,
-             size_t off)
+// A second set of matrices for eig_run and sqrtm_run, its triple of work
+// matrices its own: a Schur decomposition is one workgroup per matrix, and the
+// two directions of a lead together fill the chip where one leaves it idle.
+struct EigSecond {
+    BMat<double> A;
+    double* w;
+    BMatW<double> V;                // eigenvectors, or the square root
+    double *T, *Z, *X;              // m x m per item, stride mm
+    long mm;
+};
+
+static EigArgs eig_args(nt_ctx* c, int n, BMat<double> A, double* w, BMatW<double> V, int* status, int batch,
+                        Arena& ar, size_t off, const EigSecond* s2)
 {
     typedef double T;
     const long nn = (long)n * n;
@@ -42,45 +51,59 @@ void eig_run(nt_ctx* c, int n, BMat<double> A, double* w, BMatW<double> V, int* 
     e.batch = batch;
     audit<T>(c, e.A, n, n, batch, 1, "schur T");
     audit<T>(c, e.Z, n, n, batch, 1, "schur Z");
-    audit<T>(c, e.X, n, n, batch, 1, "trevc X");
-    audit<T>(c, V, n, n, batch, 1, "eig V");
+    audit<T>(c, e.X, n, n, batch, 1, "schur X");
+    audit<T>(c, V, n, n, batch, 1, "eig result");
     check_range(c, w, sizeof(T) * 2 * (size_t)n * batch, "eig w");
     check_range(c, status, sizeof(int) * batch, "eig status");
+    if (s2) {
+        e.sets = 2;
+        e.A2 = bw(s2->T, s2->mm, n);
+        e.Z2 = bw(s2->Z, s2->mm, n);
+        e.X2 = bw(s2->X, s2->mm, n);
+        e.w2 = s2->w;
+        copy_op<T>(c, n, n, s2->A, e.A2, 0, (T)1, batch);
+        audit<T>(c, e.A2, n, n, batch, 1, "second schur T");
+        audit<T>(c, e.Z2, n, n, batch, 1, "second schur Z");
+        audit<T>(c, e.X2, n, n, batch, 1, "second schur X");
+        audit<T>(c, s2->V, n, n, batch, 1, "second eig result");
+        check_range(c, s2->w, sizeof(T) * 2 * (size_t)n * batch, "second eig w");
+    }
+    return e;
+}
+
+// w, V from A (A is copied, not modified).  The eigenvector matrix is Z X
+// with X the triangular eigenvectors of T.
+void eig_run(nt_ctx* c, int n, BMat<double> A, double* w, BMatW<double> V, int* status, int batch, Arena& ar,
+             size_t off, const EigSecond* s2 = nullptr)
+{
+    typedef double T;
+    EigArgs e = eig_args(c, n, A, w, V, status, batch, ar, off, s2);
     launch(c, NT_K_EIG, 0.0, "schur", [&] { return launch_schur(e, c->stream); });
     launch(c, NT_K_EIG, 0.0, "trevc", [&] { return launch_trevc(e, c->stream); });
     gemm<T>(c, n, n, n, OP_N, ro(e.Z), OP_N, ro(e.X), V, 1.0, none<T>(), 0.0, nullptr, batch);
     launch(c, NT_K_EIG, 0.0, "ev normalize", [&] { return launch_ev_normalize(e, c->stream); });
+    if (s2) {
+        gemm<T>(c, n, n, n, OP_N, ro(e.Z2), OP_N, ro(e.X2), s2->V, 1.0, none<T>(), 0.0, nullptr, batch);
+        e.V = s2->V;
+        launch(c, NT_K_EIG, 0.0, "ev normalize", [&] { return launch_ev_normalize(e, c->stream); });
+    }
 }
 
-// S = sqrtm(A) (A copied)
-void sqrtm_run(nt_ctx* c, int n, BMat<double> A, BMatW<double> S, int* status, int batch, Arena& ar, size_t off)
+// S = sqrtm(A) (A copied; S may be A)
+void sqrtm_run(nt_ctx* c, int n, BMat<double> A, BMatW<double> S, int* status, int batch, Arena& ar, size_t off,
+               const EigSecond* s2 = nullptr)
 {
     typedef double T;
-    const long nn = (long)n * n;
-    Arena sa = ar;
-    sa.off = off;
-    T* Tm = sa.ptr<T>(sa.take(sizeof(T) * 2 * nn * batch));
-    T* Zm = sa.ptr<T>(sa.take(sizeof(T) * 2 * nn * batch));
-    T* Xm = sa.ptr<T>(sa.take(sizeof(T) * 2 * nn * batch));
-    copy_op<T>(c, n, n, A, bw(Tm, nn, n), 0, (T)1, batch);
-    EigArgs e;
-    e.n = n;
-    e.A = bw(Tm, nn, n);
-    e.Z = bw(Zm, nn, n);
-    e.X = bw(Xm, nn, n);
-    e.V = bw(Xm, nn, n);
-    e.w = nullptr;
-    e.status = status;
-    e.batch = batch;
-    audit<T>(c, e.A, n, n, batch, 1, "schur T");
-    audit<T>(c, e.Z, n, n, batch, 1, "schur Z");
-    audit<T>(c, S, n, n, batch, 1, "sqrtm S");
-    check_range(c, status, sizeof(int) * batch, "sqrtm status");
+    EigArgs e = eig_args(c, n, A, nullptr, S, status, batch, ar, off, s2);
     launch(c, NT_K_EIG, 0.0, "schur", [&] { return launch_schur(e, c->stream); });
     launch(c, NT_K_EIG, 0.0, "sqrt tri", [&] { return launch_sqrt_tri(e, c->stream); });
     // S = (Z U) Z^H ; Z U into the T buffer
     gemm<T>(c, n, n, n, OP_N, ro(e.Z), OP_N, ro(e.X), e.A, 1.0, none<T>(), 0.0, nullptr, batch);
     gemm<T>(c, n, n, n, OP_N, ro(e.A), OP_C, ro(e.Z), S, 1.0, none<T>(), 0.0, nullptr, batch);
+    if (s2) {
+        gemm<T>(c, n, n, n, OP_N, ro(e.Z2), OP_N, ro(e.X2), e.A2, 1.0, none<T>(), 0.0, nullptr, batch);
+        gemm<T>(c, n, n, n, OP_N, ro(e.A2), OP_C, ro(e.Z2), s2->V, 1.0, none<T>(), 0.0, nullptr, batch);
+    }
 }
 
 // ------------------------------------------------------ mode-resolved T
@@ -383,38 +406,49 @@ void modes_run(nt_ctx* c, const nt_params* prm, int tb, int nl, int nr, int P, c
                          {nl, gl_adv, OP_C, Hamlv, gml_adv, OP_C, -1.0, false, az_l},
                          {nr, gr_ret, OP_N, Hamrv, gmr_ret, OP_N, 1.0, false, az_r},
                          {nr, gr_ret, OP_C, Hamrv, gmr_ret, OP_C, 1.0, true, az_r}};
-    for (int d = 0; d < 4; ++d) {
-        const Dir& D = dirs[d];
-        const int m = D.n;
-        double* kz = o.kz[d] ? o.kz[d] : kzs[d];
+    // the two directions of a lead go through their decompositions together
+    // (the second one's work matrices: buffers that are only filled later)
+    for (int d0 = 0; d0 < 4; d0 += 2) {
+        const int m = dirs[d0].n;
+        EigSecond e2{R(U[d0 + 1], m), w[d0 + 1], W(U[d0 + 1], m), QL, QR, T1, mm};
         // F = op(g) V  -> U (eigen input, overwritten by the eigenvectors)
-        gemm<T>(c, m, m, m, D.opg, D.g, OP_N, D.V, W(U[d], m), 1.0, none<T>(), 0.0, nullptr, P);
-        eig_run(c, m, R(U[d], m), w[d], W(U[d], m), status, P, ar, eig_off);
-        ModesArgs ma;
-        ma.n = m;
-        ma.w = w[d];
-        ma.U = W(U[d], m);
-        ma.kz = kz;
-        ma.nprop = o.nprop[d];
-        ma.lambda_eta = prm->lambda_eta;
-        ma.az = D.az;
-        ma.sign = D.sign;
-        ma.batch = P;
-        audit<T>(c, ma.U, m, m, P, 1, "modes U");
-        check_range(c, kz, sizeof(double) * (size_t)m * P, "modes kz");
-        check_range(c, o.nprop[d], sizeof(int) * P, "modes nprop");
-        launch(c, NT_K_EIG, 0.0, "modes select", [&] { return launch_modes_select(ma, s); });
-        if (prm->path_mode == 1)
-            degenerate_rotation(c, m, P, mm, E, d < 2 ? Haml : Hamr, D.V, w[d], U[d], kz, status, ar, eig_off);
-        // V = s (U^+ Gamma' U)
-        gemm<T>(c, m, m, m, OP_C, R(U[d], m), D.opgam, D.gam, W(T1, m), 1.0, none<T>(), 0.0, nullptr, P);
-        gemm<T>(c, m, m, m, OP_N, R(T1, m), OP_N, R(U[d], m), W(Vw, m), 1.0, none<T>(), 0.0, nullptr, P);
-        launch(c, NT_K_ELEM, 0.0, "scale V",
-               [&] { return launch_scale_items(Vw, mm, m, m, m, sc + 2 * (long)d * P, P, s); });
-        sqrtm_run(c, m, R(Vw, m), W(Vh[d], m), status, P, ar, eig_off);
+        for (int d = d0; d < d0 + 2; ++d)
+            gemm<T>(c, m, m, m, dirs[d].opg, dirs[d].g, OP_N, dirs[d].V, W(U[d], m), 1.0, none<T>(), 0.0, nullptr, P);
+        eig_run(c, m, R(U[d0], m), w[d0], W(U[d0], m), status, P, ar, eig_off, &e2);
+        for (int d = d0; d < d0 + 2; ++d) {
+            const Dir& D = dirs[d];
+            double* kz = o.kz[d] ? o.kz[d] : kzs[d];
+            ModesArgs ma;
+            ma.n = m;
+            ma.w = w[d];
+            ma.U = W(U[d], m);
+            ma.kz = kz;
+            ma.nprop = o.nprop[d];
+            ma.lambda_eta = prm->lambda_eta;
+            ma.az = D.az;
+            ma.sign = D.sign;
+            ma.batch = P;
+            audit<T>(c, ma.U, m, m, P, 1, "modes U");
+            check_range(c, kz, sizeof(double) * (size_t)m * P, "modes kz");
+            check_range(c, o.nprop[d], sizeof(int) * P, "modes nprop");
+            launch(c, NT_K_EIG, 0.0, "modes select", [&] { return launch_modes_select(ma, s); });
+            if (prm->path_mode == 1)
+                degenerate_rotation(c, m, P, mm, E, d < 2 ? Haml : Hamr, D.V, w[d], U[d], kz, status, ar, eig_off);
+            // V = s (U^+ Gamma' U)
+            gemm<T>(c, m, m, m, OP_C, R(U[d], m), D.opgam, D.gam, W(T1, m), 1.0, none<T>(), 0.0, nullptr, P);
+            gemm<T>(c, m, m, m, OP_N, R(T1, m), OP_N, R(U[d], m), W(Vh[d], m), 1.0, none<T>(), 0.0, nullptr, P);
+            launch(c, NT_K_ELEM, 0.0, "scale V",
+                   [&] { return launch_scale_items(Vh[d], mm, m, m, m, sc + 2 * (long)d * P, P, s); });
+        }
+        e2.A = R(Vh[d0 + 1], m);
+        e2.w = nullptr;
+        e2.V = W(Vh[d0 + 1], m);
+        sqrtm_run(c, m, R(Vh[d0], m), W(Vh[d0], m), status, P, ar, eig_off, &e2);
         // inv(U^+) for incident directions, inv(U) for outgoing ones
-        copy_op<T>(c, m, m, R(U[d], m), W(T2, m), D.incident ? 1 : 0, (T)1, P);
-        inverse<T>(c, m, W(T2, m), none<T>(), nullptr, W(iU[d], m), status, P);
+        for (int d = d0; d < d0 + 2; ++d) {
+            copy_op<T>(c, m, m, R(U[d], m), W(T2, m), dirs[d].incident ? 1 : 0, (T)1, P);
+            inverse<T>(c, m, W(T2, m), none<T>(), nullptr, W(iU[d], m), status, P);
+        }
     }
     // bulk GFs: Q = z - H00 - V^+ op(g) V - V op(g') V^+, inverted
     {

@@ -80,6 +80,29 @@ def test_zgeev_random(engine, torch_dev, n):
         assert np.all(top.imag == 0.0) and np.all(top.real > 0)
 
 
+@pytest.mark.parametrize("n", [31, 32, 33, 63, 64, 65, 66, 95, 97])
+@pytest.mark.parametrize("kind", ["random", "blocks", "scaled"])
+def test_zgeev_sizes_of_the_lds(engine, torch_dev, n, kind):
+    """The sizes where the decomposition changes its kernel or its rows per
+    lane.  "blocks": an upper part decoupled from the rest (deflation inside
+    the window) and a zero row; "scaled": entries whose squares leave the
+    range of the short rotation formula.  A V = V w to n^2 eps |A|, the backward
+    error of a QR iteration of about n sweeps of n rotations."""
+    torch, dev = torch_dev
+    rng = np.random.default_rng(100 + n)
+    A = crand(rng, n, n)
+    if kind == "blocks":
+        A[n // 2:, :n // 2] = 0.0
+        A[n // 3] = 0.0
+    scale = 1e-80 if kind == "scaled" else 1.0
+    print(f"zgeev n={n} {kind}", flush=True)
+    w, V, st, _ = geev(engine, torch, dev, [A * scale])
+    assert st[0] == 0
+    tol = n * n * np.finfo(float).eps * np.linalg.norm(A, 2)
+    assert np.abs(A @ V[0] - V[0] * (w[0] / scale)).max() < tol
+    assert abs(w[0].sum() / scale - np.trace(A)) < tol
+
+
 @pytest.mark.parametrize("n", [12, 48, 96])
 def test_zgeev_lead_transfer_matrix(engine, torch_dev, n):
     torch, dev = torch_dev

@@ -217,6 +217,7 @@ int nt_zgemm_batched_dev(nt_ctx* c, char opA, char opB, int m, int n, int k, nt_
         a.batch = batch;
         a.groups = 1;
         a.m3 = c->gemm_m3 ? 1 : 0;
+        a.tile = gemm_tile_of<T>(c, m, n);
         launch(c, NT_K_GEMM, 8.0 * m * n * k * (double)batch, "gemm", [&] { return launch_gemm<T>(a, c->stream); });
         return 0;
     });

@@ -1979,7 +1979,8 @@ void tune_gemm(nt_ctx* c, int n, int batch, int* best_tile, double* best_ms)
     const bool prof = c->prof;
     c->prof = false;
     for (int tb : tiles) {
-        c->gemm_tile[{(int)sizeof(T), n}] = tb;
+        // (64 stands for the size rule's tile)
+        c->gemm_tile[{(int)sizeof(T), n}] = tb == 64 ? 0 : tb;
         auto run = [&] {
             gemm<T>(c, n, n, n, OP_N, bm<T>(A.as<T>(), nn, n), OP_N, bm<T>(B.as<T>(), nn, n), bw(X.as<T>(), nn, n),
                     1.0, none<T>(), 0.0, nullptr, batch);
@@ -2000,7 +2001,7 @@ void tune_gemm(nt_ctx* c, int n, int batch, int* best_tile, double* best_ms)
     c->prof = prof;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    c->gemm_tile[{(int)sizeof(T), n}] = bt;
+    c->gemm_tile[{(int)sizeof(T), n}] = bt == 64 ? 0 : bt;
     if (best_tile) *best_tile = bt;
     if (best_ms) *best_ms = best;
 }

@@ -1,12 +1,13 @@
 // nt_gemm.hip -- batched complex GEMM on CDNA4 MFMA (FP64 and FP32).
 //
 // One workgroup computes a TB x TB complex tile of one batch item: TB = 64
-// with 4 wave64 (the default), or TB = 32 with one wave64 (less padding when
-// the matrix size is not a multiple of 64: 24, 96, 216, ...; chosen per size
-// by the autotuner).  Operand tiles of depth 8 are staged through two LDS
+// with 4 wave64, TB = 48 with 3 (FP64; where it covers the matrix with less
+// padding), or TB = 32 with one wave64 (chosen per size by the autotuner).
+// Operand tiles of depth 8 (16 with TB = 48) are staged through two LDS
 // buffers as separate real and imaginary planes (one barrier per stage); each
-// wave owns a 32x32 quadrant as 2x2 MFMA 16x16 tiles and issues four real
-// MFMAs per complex 16x16x4 step.
+// wave owns a 32x32 quadrant as 2x2 MFMA 16x16 tiles (a 48x16 strip as 3x1)
+// and issues four real MFMAs per complex 16x16x4 step.  The order of the sums
+// is the same in every tile: a choice of tile changes no bit.
 //
 // The product is formed transposed (C^T = B^T A^T): the MFMA output layout
 // then maps 16 consecutive lanes to 16 consecutive rows of the column-major C,
@@ -17,12 +18,16 @@ namespace nt {
 
 namespace {
 
-constexpr int BK = 8;         // operand depth per LDS stage
 constexpr int NXCD = 8;       // accelerator complex dies of the MI355X
 
-// threads of a TB x TB tile's workgroup and operand elements each stages per stage
+// A TB x TB tile's workgroup: its threads, operand depth per LDS stage,
+// padding of a staged row, 16 x 16 MFMA tiles per wave (NX along M, NY along
+// N), operand elements each thread stages per stage.
 template <int TB> struct Tile {
-    static constexpr int NT = TB == 64 ? 256 : 64;
+    static constexpr int NT = TB == 64 ? 256 : TB == 48 ? 192 : 64;
+    static constexpr int BK = TB == 48 ? 16 : 8;
+    static constexpr int PAD = TB == 48 ? 2 : 0;
+    static constexpr int NX = TB == 48 ? 3 : 2, NY = TB == 48 ? 1 : 2;
     static constexpr int EPT = TB * BK / NT;
 };
 
@@ -30,10 +35,11 @@ template <int TB> struct Tile {
 // loads are not writing, so each K-stage needs a single barrier
 template <typename T, int TB>
 struct GemmSmem {
-    T ar[2][BK][TB];
-    T ai[2][BK][TB];
-    T br[2][BK][TB];
-    T bi[2][BK][TB];
+    static constexpr int BK = Tile<TB>::BK, LD = TB + Tile<TB>::PAD;
+    T ar[2][BK][LD];
+    T ai[2][BK][LD];
+    T br[2][BK][LD];
+    T bi[2][BK][LD];
 };
 
 // Element j of thread t.  op N (A) / op C (B): row r = t % TB (contiguous in
@@ -43,7 +49,7 @@ template <typename T, int TB>
 __device__ __forceinline__ void load_a_regs(const T* __restrict__ A, int lda, int opA, int M, int K,
                                             int m0, int k0, T (&r)[Tile<TB>::EPT], T (&i)[Tile<TB>::EPT])
 {
-    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT;
+    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT, BK = Tile<TB>::BK;
     const int t = threadIdx.x;
     typedef typename vec2<T>::type V2;
     if (opA == OP_N) {
@@ -75,7 +81,7 @@ template <typename T, int TB>
 __device__ __forceinline__ void store_a_smem(GemmSmem<T, TB>& s, int buf, int opA, const T (&r)[Tile<TB>::EPT],
                                              const T (&i)[Tile<TB>::EPT])
 {
-    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT;
+    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT, BK = Tile<TB>::BK;
     const int t = threadIdx.x;
     if (opA == OP_N) {
         const int m = t % TB, kq = t / TB;
@@ -98,7 +104,7 @@ template <typename T, int TB>
 __device__ __forceinline__ void load_b_regs(const T* __restrict__ B, int ldb, int opB, int K, int N,
                                             int k0, int n0, T (&r)[Tile<TB>::EPT], T (&i)[Tile<TB>::EPT])
 {
-    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT;
+    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT, BK = Tile<TB>::BK;
     const int t = threadIdx.x;
     typedef typename vec2<T>::type V2;
     if (opB == OP_N) {
@@ -130,7 +136,7 @@ template <typename T, int TB>
 __device__ __forceinline__ void store_b_smem(GemmSmem<T, TB>& s, int buf, int opB, const T (&r)[Tile<TB>::EPT],
                                              const T (&i)[Tile<TB>::EPT])
 {
-    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT;
+    constexpr int NT = Tile<TB>::NT, EPT = Tile<TB>::EPT, BK = Tile<TB>::BK;
     const int t = threadIdx.x;
     if (opB == OP_N) {
         const int k = t % BK, nq = t / BK;
@@ -161,7 +167,7 @@ __device__ __forceinline__ void atomic_max_nonneg(unsigned long long* addr, doub
 template <typename T, bool M3, int TB>
 __global__ __launch_bounds__(Tile<TB>::NT, (M3 ? 2 : 3) * (256 / Tile<TB>::NT)) void k_gemm(GemmArgs<T> a)
 {
-    constexpr int EPT = Tile<TB>::EPT;
+    constexpr int EPT = Tile<TB>::EPT, BK = Tile<TB>::BK, NX = Tile<TB>::NX, NY = Tile<TB>::NY;
     constexpr int BM = TB, BN = TB;
     typedef typename acc4<T>::type A4;
     const int tiles_m = (a.M + BM - 1) / BM;
@@ -197,14 +203,14 @@ __global__ __launch_bounds__(Tile<TB>::NT, (M3 ? 2 : 3) * (256 / Tile<TB>::NT)) 
 
     const int lane = lane_id();
     const int wave = threadIdx.x >> 6;       // 0 when TB = 32
-    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+    const int wm = TB == 48 ? 0 : (wave & 1) * 32, wn = TB == 48 ? 16 * wave : (wave >> 1) * 32;
     const int lr = lane & 15, lk = lane >> 4;
 
-    A4 accR[2][2], accI[2][2], accS[2][2];
+    A4 accR[NX][NY], accI[NX][NY], accS[NX][NY];
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < NX; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) {
+        for (int y = 0; y < NY; ++y) {
             accR[x][y] = A4{0, 0, 0, 0};
             accI[x][y] = A4{0, 0, 0, 0};
             accS[x][y] = A4{0, 0, 0, 0};
@@ -227,27 +233,27 @@ __global__ __launch_bounds__(Tile<TB>::NT, (M3 ? 2 : 3) * (256 / Tile<TB>::NT)) 
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 4) {
             const int k = kk + lk;
-            T xr[2], xi[2], yr[2], yi[2];
+            T xr[NX], xi[NX], yr[NY], yi[NY];
 #pragma unroll
-            for (int x = 0; x < 2; ++x) {
+            for (int x = 0; x < NX; ++x) {
                 xr[x] = s.ar[cur][k][wm + 16 * x + lr];
                 xi[x] = s.ai[cur][k][wm + 16 * x + lr];
             }
 #pragma unroll
-            for (int y = 0; y < 2; ++y) {
+            for (int y = 0; y < NY; ++y) {
                 yr[y] = s.br[cur][k][wn + 16 * y + lr];
                 yi[y] = s.bi[cur][k][wn + 16 * y + lr];
             }
             if constexpr (M3) {
-                T xs[2], ys[2];
+                T xs[NX], ys[NY];
 #pragma unroll
-                for (int x = 0; x < 2; ++x) xs[x] = xr[x] + xi[x];
+                for (int x = 0; x < NX; ++x) xs[x] = xr[x] + xi[x];
 #pragma unroll
-                for (int y = 0; y < 2; ++y) ys[y] = yr[y] + yi[y];
+                for (int y = 0; y < NY; ++y) ys[y] = yr[y] + yi[y];
 #pragma unroll
-                for (int x = 0; x < 2; ++x)
+                for (int x = 0; x < NX; ++x)
 #pragma unroll
-                    for (int y = 0; y < 2; ++y) {
+                    for (int y = 0; y < NY; ++y) {
                         // accR = P1, accI = P2, accS = P3
                         accR[x][y] = mfma16x16x4(yr[y], xr[x], accR[x][y]);
                         accI[x][y] = mfma16x16x4(yi[y], xi[x], accI[x][y]);
@@ -255,9 +261,9 @@ __global__ __launch_bounds__(Tile<TB>::NT, (M3 ? 2 : 3) * (256 / Tile<TB>::NT)) 
                     }
             } else {
 #pragma unroll
-                for (int x = 0; x < 2; ++x)
+                for (int x = 0; x < NX; ++x)
 #pragma unroll
-                    for (int y = 0; y < 2; ++y) {
+                    for (int y = 0; y < NY; ++y) {
                         // (C^T) = B^T A^T: MFMA "A" operand is B, "B" operand is A.
                         accR[x][y] = mfma16x16x4(yr[y], xr[x], accR[x][y]);
                         accR[x][y] = mfma16x16x4(-yi[y], xi[x], accR[x][y]);
@@ -285,9 +291,9 @@ __global__ __launch_bounds__(Tile<TB>::NT, (M3 ? 2 : 3) * (256 / Tile<TB>::NT)) 
     }
     double vmax = 0.0;
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < NX; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
+        for (int y = 0; y < NY; ++y)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + wm + 16 * x + lr;
@@ -349,7 +355,16 @@ hipError_t launch_gemm(const GemmArgs<T>& a, hipStream_t s)
 {
     if (a.M <= 0 || a.N <= 0 || a.batch <= 0 || a.groups <= 0) return hipSuccess;
     if (a.tile != 0 && a.tile != 32 && a.tile != 64) return hipErrorInvalidValue;
-    const int tb = a.tile == 32 ? 32 : 64;
+    // FP64: 48 where it pads much less.  128 products (1024), 64 -> 48: n = 80
+    // 33 -> 26 us (202 -> 172), 96 38 -> 31 (246 -> 211), 144 113 -> 87 (754 ->
+    // 601), each with 0.56 of the padded area; at 0.88 (216) 259 -> 332 and at
+    // 0.77 (330) 849 -> 903.  A single tile (n = 48: 16 -> 13 us for 128) only
+    // while the larger workgroups leave the chip room: 40 -> 42 us for 1024.
+    const auto padded = [&](int t) { return (double)((a.M + t - 1) / t) * ((a.N + t - 1) / t) * t * t; };
+    const bool one = a.M <= 48 && a.N <= 48;
+    const bool t48 = sizeof(T) == 8 && !a.m3 && padded(48) < 0.6 * padded(64) &&
+                     !(one && (long)a.batch * a.groups >= 768);
+    const int tb = a.tile ? a.tile : t48 ? 48 : 64;
     const long tiles = (long)((a.M + tb - 1) / tb) * ((a.N + tb - 1) / tb);
     // from 8 points on the kernel interleaves points over the XCDs and the
     // grid covers the point count rounded up to a multiple of 8
@@ -361,6 +376,9 @@ hipError_t launch_gemm(const GemmArgs<T>& a, hipStream_t s)
             hipLaunchKernelGGL((k_gemm<T, true, 32>), dim3((unsigned)blocks), dim3(Tile<32>::NT), 0, s, a);
         else
             hipLaunchKernelGGL((k_gemm<T, false, 32>), dim3((unsigned)blocks), dim3(Tile<32>::NT), 0, s, a);
+    } else if (tb == 48) {
+        if constexpr (sizeof(T) == 8)
+            hipLaunchKernelGGL((k_gemm<T, false, 48>), dim3((unsigned)blocks), dim3(Tile<48>::NT), 0, s, a);
     } else {
         if (a.m3)
             hipLaunchKernelGGL((k_gemm<T, true, 64>), dim3((unsigned)blocks), dim3(Tile<64>::NT), 0, s, a);

@@ -304,6 +304,14 @@ void audit(nt_ctx* c, const M& m, int rows, int cols, int batch, int groups, con
 }
 
 // C = alpha op(A) op(B) + beta Cin + diag
+// output tile set for an M x N product, 0 for none
+template <typename T>
+int gemm_tile_of(const nt_ctx* c, int M, int N)
+{
+    const auto set = c->gemm_tile.find({(int)sizeof(T), std::max(M, N)});
+    return set == c->gemm_tile.end() ? 0 : set->second;
+}
+
 template <typename T>
 void gemm(nt_ctx* c, int M, int N, int K, int opA, BMat<T> A, int opB, BMat<T> B, BMatW<T> C, double alpha,
           BMat<T> Cin, double beta, const T* diag, int batch, double nitems = -1, const int* active = nullptr,
@@ -331,10 +339,7 @@ void gemm(nt_ctx* c, int M, int N, int K, int opA, BMat<T> A, int opB, BMat<T> B
     a.batch = batch;
     a.groups = groups;
     a.m3 = (sizeof(T) == 8 && c->gemm_m3) ? 1 : 0;
-    if (!c->gemm_tile.empty()) {
-        auto tuned = c->gemm_tile.find({(int)sizeof(T), std::max(M, N)});
-        a.tile = tuned == c->gemm_tile.end() ? 0 : tuned->second;
-    }
+    a.tile = gemm_tile_of<T>(c, M, N);
     const double items = (nitems < 0 ? (double)batch : nitems) * groups;
     audit<T>(c, A, opA == OP_N ? M : K, opA == OP_N ? K : M, batch, groups, "gemm A");
     audit<T>(c, B, opB == OP_N ? K : N, opB == OP_N ? N : K, batch, groups, "gemm B");

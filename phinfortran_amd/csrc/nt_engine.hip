@@ -201,6 +201,8 @@ __global__ void k_copy_lead_stack(const double2* a, const double2* b, double2* o
 
 
 // ------------------------------------------------------------ decimation
+constexpr int DEC_TILE_STEPS = 20000;      // in one kernel: about 0.5 s at n = 64
+
 // Q items of size n.  H00 / V addressed per item; alpha = V^+ (alpha_dagger)
 // or V.  Outputs g (and optionally Sigma = alpha0 g beta0, Gamma).
 template <typename T>
@@ -232,9 +234,6 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
     audit<T>(c, H00, n, n, Q, 1, "dec H00");
     audit<T>(c, V, n, n, Q, 1, "dec V");
     audit<T>(c, bw(ab0, 2 * nn, n, nullptr, nn), n, n, Q, 2, "dec ab");
-    launch(c, NT_K_ELEM, 0, "dec_init",
-           [&] { return launch_dec_init<T>(n, H00, V, alpha_dagger, bw(e1, nn, n), bw(es, nn, n),
-                                           bw(ab0, 2 * nn, n, nullptr, nn), Q, s); });
     check_range(c, z, sizeof(T) * 2 * Q, "dec z");
     check_range(c, status, sizeof(int) * Q, "dec status");
     check_range(c, iters, sizeof(int) * Q, "dec iters");
@@ -249,6 +248,73 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
     } else {
         launch(c, NT_K_ELEM, 0, "fill", [&] { return launch_fill_int(active, 1, Q, s); });
     }
+    // flops of the steps, from the items' counts: an inverse and six products each
+    auto add_flops = [&](int k, double per_step, double gemms) {
+        if (!c->prof) return;
+        std::vector<int> h(Q);
+        hipcheck(c, hipMemcpyAsync(h.data(), iters, sizeof(int) * Q, hipMemcpyDeviceToHost, s), "memcpy");
+        hipcheck(c, hipStreamSynchronize(s), "sync");
+        double tot = 0.0;
+        for (int q = 0; q < Q; ++q) tot += h[q];
+        const double f = 8.0 * n * (double)n * n * tot;
+        c->flops_pending[k] += per_step * f;
+        c->flops_pending[NT_K_GEMM] += gemms * f;
+    };
+    auto finish = [&] {
+        hipLaunchKernelGGL(k_dec_finish, dim3(nblk(Q)), dim3(256), 0, s, active, status, Q);
+        hipcheck(c, hipGetLastError(), "dec_finish");
+        if (std::is_same<T, double>::value)
+            launch(c, NT_K_ELEM, 0, "dec_dead",
+                   [&] { return launch_dec_dead(status, reinterpret_cast<double*>(es), nn, Q, s); });
+        const int* fin = nullptr;
+        if (mask) {
+            hipLaunchKernelGGL(k_expand_mask, dim3(nblk(Q)), dim3(256), 0, s, mask, active, Q, per);
+            hipcheck(c, hipGetLastError(), "dec mask");
+            fin = active;
+        }
+        // g = (z - es)^-1 for every item (surface.f90:497)
+        inverse<T>(c, n, bw(W, nn, n), bm<T>(es, nn, n), z, out.g, status, Q, -1, fin);
+        if (out.sigma.base) {
+            // Sigma = alpha0 g beta0 = V^+ g V (alpha_dagger) ; t1 = V^+ g
+            gemm<T>(c, n, n, n, alpha_dagger ? OP_C : OP_N, V, OP_N, ro(out.g), bw(t12, 2 * nn, n), 1.0, none<T>(), 0.0,
+                    nullptr, Q, -1, fin);
+            gemm<T>(c, n, n, n, OP_N, bm<T>(t12, 2 * nn, n), alpha_dagger ? OP_N : OP_C, V, out.sigma, 1.0, none<T>(),
+                    0.0, nullptr, Q, -1, fin);
+            if (out.gamma.base) gamma_op<T>(c, n, ro(out.sigma), out.gamma, Q);
+        }
+    };
+    // FP64: one kernel for the whole recursion (n = 48: 13.6 ms against 21 for
+    // 5978 items, 0.19 against 0.9 for two) where n <= 64 and the padded matrices
+    // fit the scratch of the steps below, that is n > 0.79 of the next multiple
+    // of 16; unless the caller chose the inverse's panel width or three-product
+    // GEMMs, and for as many steps as a kernel should last.
+    const size_t tile = dec_tile_scratch(n);
+    const bool panels = c->inv_panels || (c->inv_nb.count({8, n}) && !c->inv_tuned.count(n));
+    if (std::is_same<T, double>::value && tile && tile <= (size_t)8 * mb && !panels && !c->gemm_m3 &&
+        max_iter <= DEC_TILE_STEPS) {
+        DecTileArgs d;
+        d.n = n;
+        d.batch = Q;
+        d.max_iter = max_iter;
+        d.alpha_dagger = alpha_dagger;
+        d.conv = conv;
+        d.H00 = BMat<double>{reinterpret_cast<const double*>(H00.base), H00.stride, H00.gstride, H00.idx, H00.ld, H00.idx_n};
+        d.V = BMat<double>{reinterpret_cast<const double*>(V.base), V.stride, V.gstride, V.idx, V.ld, V.idx_n};
+        d.z = reinterpret_cast<const double*>(z);
+        d.es = bw(reinterpret_cast<double*>(es), nn, n);
+        // over the four pairs of matrices that the steps below use: ab0 to W
+        d.scratch = reinterpret_cast<double*>(ab0);
+        d.active = active;
+        d.iters = iters;
+        d.status = status;
+        check_range(c, ab0, tile * Q, "dec scratch");
+        launch(c, NT_K_PLANES, 0, "decimation", [&] { return launch_dec_tile(d, s); });
+        add_flops(NT_K_PLANES, 7.0, 0.0);
+        return finish();
+    }
+    launch(c, NT_K_ELEM, 0, "dec_init",
+           [&] { return launch_dec_init<T>(n, H00, V, alpha_dagger, bw(e1, nn, n), bw(es, nn, n),
+                                           bw(ab0, 2 * nn, n, nullptr, nn), Q, s); });
     // initial maxdiff = max|alpha| (surface.f90:484): the GEMM epilogue's
     // maxabs on a K = 0 product with Cin = alpha0 (a copy), then one update
     // (update 0: slot 0) that does not count as an iteration
@@ -305,38 +371,8 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
         });
         std::swap(abc, abn);
     }
-    if (c->prof) {
-        // every active item-iteration: one inverse and six n^3 products
-        std::vector<int> h(Q);
-        hipcheck(c, hipMemcpyAsync(h.data(), iters, sizeof(int) * Q, hipMemcpyDeviceToHost, s), "memcpy");
-        hipcheck(c, hipStreamSynchronize(s), "sync");
-        double tot = 0.0;
-        for (int q = 0; q < Q; ++q) tot += h[q];
-        const double f = 8.0 * n * (double)n * n * tot;
-        c->flops_pending[NT_K_INV] += f;
-        c->flops_pending[NT_K_GEMM] += 6.0 * f;
-    }
-    hipLaunchKernelGGL(k_dec_finish, dim3(nblk(Q)), dim3(256), 0, s, active, status, Q);
-    hipcheck(c, hipGetLastError(), "dec_finish");
-    if (std::is_same<T, double>::value)
-        launch(c, NT_K_ELEM, 0, "dec_dead",
-               [&] { return launch_dec_dead(status, reinterpret_cast<double*>(es), nn, Q, s); });
-    const int* fin = nullptr;
-    if (mask) {
-        hipLaunchKernelGGL(k_expand_mask, dim3(nblk(Q)), dim3(256), 0, s, mask, active, Q, per);
-        hipcheck(c, hipGetLastError(), "dec mask");
-        fin = active;
-    }
-    // g = (z - es)^-1 for every item (surface.f90:497)
-    inverse<T>(c, n, bw(W, nn, n), bm<T>(es, nn, n), z, out.g, status, Q, -1, fin);
-    if (out.sigma.base) {
-        // Sigma = alpha0 g beta0 = V^+ g V (alpha_dagger) ; t1 = V^+ g
-        gemm<T>(c, n, n, n, alpha_dagger ? OP_C : OP_N, V, OP_N, ro(out.g), bw(t12, 2 * nn, n), 1.0, none<T>(), 0.0,
-                nullptr, Q, -1, fin);
-        gemm<T>(c, n, n, n, OP_N, bm<T>(t12, 2 * nn, n), alpha_dagger ? OP_N : OP_C, V, out.sigma, 1.0, none<T>(),
-                0.0, nullptr, Q, -1, fin);
-        if (out.gamma.base) gamma_op<T>(c, n, ro(out.sigma), out.gamma, Q);
-    }
+    add_flops(NT_K_INV, 1.0, 6.0);
+    finish();
 }
 
 // ------------------------------------------------ circular decimation

@@ -56,6 +56,24 @@ constexpr int INV_PANELS = -1;
 constexpr int INV_MAX_WIDTHS = 6;
 template <typename T> int inv_panel_widths(int n, int* out);
 
+// The whole decimation of an FP64 lead of n <= 64 (nt_dec.hip).  active[p] in:
+// 0 leaves the item out; out: 1 if it ran into max_iter.  iters[p] steps,
+// status[p] the first error of the item (as the inverse reports it, -1 for a
+// recursion that left the finite numbers, whose iters is max_iter).  es: the
+// surface matrix, z - es being inverted last.  scratch: dec_tile_scratch(n)
+// bytes per item (0: n is too large).
+struct DecTileArgs {
+    int n, batch, max_iter, alpha_dagger;
+    double conv;
+    BMat<double> H00, V;
+    const double* z;
+    BMatW<double> es;
+    double* scratch;
+    int *active, *iters, *status;
+};
+size_t dec_tile_scratch(int n);
+hipError_t launch_dec_tile(const DecTileArgs& a, hipStream_t s);
+
 // Batched complex Schur / eigen / square-root kernels (nt_eig.hip), FP64.
 struct EigArgs {
     int n;

@@ -494,34 +494,6 @@ __device__ __forceinline__ void blk_shift(Blk<NT>& m, double zr, double zi, int 
 }
 
 // largest value over the workgroup, in every thread
-template <int NW>
-__device__ __forceinline__ double wg_max(double* red, double v)
-{
-#pragma unroll
-    for (int o = 32; o; o >>= 1) v = fmax(v, __shfl_xor(v, o));
-    __syncthreads();
-    if (lane_id() == 0) red[wave_id()] = v;
-    __syncthreads();
-    double r = red[0];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) r = fmax(r, red[i]);
-    return r;
-}
-
-template <int NT>
-__device__ __forceinline__ double blk_maxabs(const Blk<NT>& x)
-{
-    double v = 0.0;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const double a = sqrt(x.re[t][r] * x.re[t][r] + x.im[t][r] * x.im[t][r]);
-            v = a > v || a != a ? (a != a ? INFINITY : a) : v;      // NaN never converges
-        }
-    return v;
-}
-
 // ------------------------------------------------------------------ decimation
 // Lopez-Sancho decimation (negf/surface.f90:479-497) of a lead cell whose
 // couplings run from its plane B (facing the device) to plane A of the next
@@ -1625,6 +1597,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         later[1] += c->host_plan[0];
     }
     const double steps = wait ? (double)c->host_plan[1] : 0.0;
+    // of a decimation step: the inverse of two planes and eight products of one
+    if (c->prof && !big) c->flops_pending[NT_K_PLANES] += steps * 16 * 8 * (16.0 * h.nt) * (16.0 * h.nt) * (16.0 * h.nt);
     if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - left;
     TdbArgs g = a;
     g.siblings.clear();

@@ -512,4 +512,34 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
     __syncthreads();
 }
 
+// largest v of NW waves, in every lane (two barriers)
+template <int NW>
+__device__ __forceinline__ double wg_max(double* red, double v)
+{
+#pragma unroll
+    for (int o = 32; o; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+    __syncthreads();
+    if (lane_id() == 0) red[wave_id()] = v;
+    __syncthreads();
+    double r = red[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) r = fmax(r, red[i]);
+    return r;
+}
+
+// largest modulus of a wave's columns, infinite with a NaN among them
+template <int NT>
+__device__ __forceinline__ double blk_maxabs(const Blk<NT>& x)
+{
+    double v = 0.0;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const double a = sqrt(x.re[t][r] * x.re[t][r] + x.im[t][r] * x.im[t][r]);
+            v = a > v || a != a ? (a != a ? INFINITY : a) : v;      // NaN never converges
+        }
+    return v;
+}
+
 }  // namespace

@@ -50,7 +50,8 @@ enum {
     NT_PREC_FP64 = 0,      /* complex FP64 throughout (the reference's arithmetic) */
     NT_PREC_MIXED = 1      /* FP64 decimation; each sweep direction factorised in complex FP32 on
                               MFMA, its block column refined against FP64 residuals (one or two
-                              steps); points failing the error estimate recomputed in FP64 */
+                              steps); points failing the error estimate recomputed in FP64.
+                              Devices that run on planes (nt_set_planes) are solved in FP64 */
 };
 
 /* Scalar parameters that the reference keeps as module globals
@@ -295,12 +296,14 @@ int nt_set_multi_workers(nt_ctx* ctx, int n);
  * counterpart in the reference. */
 int nt_set_point_split(nt_ctx* ctx, int n);
 
-/* FP64 batched solves without extra outputs run on the planes that the zero
- * blocks of the principal layers divide them into, where every plane holds at
- * most 64 degrees of freedom (default on): the same block elimination on
- * smaller blocks.  Points with a singular or nearly singular plane are solved
- * on the layers.  on = 0: always on the layers.  No counterpart in the
- * reference. */
+/* Batched solves without extra outputs (also of several devices, and the
+ * adjoint) run on the planes that the zero blocks of the principal layers
+ * divide them into, where every plane holds at most 64 degrees of freedom, or
+ * 96 where the call may allocate and wait for the device (default on): the
+ * same block elimination on smaller blocks, in FP64, which then serves
+ * NT_PREC_MIXED calls too (faster than the FP32 factorisation it replaces).
+ * Points with a singular or nearly singular plane are solved on the layers.
+ * on = 0: always on the layers.  No counterpart in the reference. */
 int nt_set_planes(nt_ctx* ctx, int on);
 
 /* Host-pointer variant (copies in and out; same layout). */

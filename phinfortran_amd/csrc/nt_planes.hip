@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void k_pl_levels(PlanDims d, PlanView v)
 // One workgroup: wave t sums the planes of class t, the cheapest of the first
 // ncls classes wins: per plane about five products of the class size and as
 // many pivots as it has columns (5120 SIMD cycles per 16^3 of products and
-// 12000 per 16 pivots).
+// 12000 per 16 pivots, of the inverse's 53 us at 64 and the products' rate).
 __global__ __launch_bounds__(64 * PL_NCLS) void k_pl_plan(PlanDims d, PlanView v, int ncls)
 {
     const int nL = d.L + 2, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -508,6 +508,9 @@ __device__ __forceinline__ void blk_shift(Blk<NT>& m, double zr, double zi, int 
 // full cell's inverse 2.7e-10).  The elements of alpha are the ones of the
 // full recursion, so the count of steps to max|alpha| <= convergence is too.
 // 2 NT waves: the first NT own the columns of A, the others those of B.
+// Bound by the inverse's pivot chain; from NT = 3 on one workgroup has a CU to
+// itself, and its waves' registers spill.  2048 leads of a film of 192 (four
+// planes of 48): 30.7 ms.
 constexpr int DEC_SLOTS = 19;       // matrices of NP^2 per item
 
 template <int NT>
@@ -725,6 +728,14 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
 //   G = A^-1                                  in LDS
 //   R = G_{first,i}^T = G^T (U^T R)           in registers
 // and at the end T = Re Tr[(R^T Gamma_e)(R^* Gamma_s)].
+// Bound by the pivot chains of the inverses (other workgroups fill the CU
+// meanwhile) and by L2 reads of H, U and L.  Both directions go through as
+// points of one launch: the corner correction that saves the second one on
+// layers costs inverses here as well.  The couplings' zero pieces (4 columns by
+// 16 rows) are skipped by a mask, and up to 48 three waves per SIMD are built
+// for: film of 168 planes of 48, 1024 points, 54.6 -> 43.9 ms from both, 38.3
+// with the shorter pivot chain.  The whole solve of
+// them: 748 ms on layers of 192, 71 on planes, 31 of them the decimation.
 template <int NT>
 __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArgs a)
 {
@@ -837,7 +848,9 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
 // of R of all points above one another and the columns of C beside one
 // another: the sums over the points of X_{j,i}^+ = R_i^+ C_j^+ are then one
 // product per layer and k-point, over 16 NT rows per point instead of a b x b
-// block of each point summed afterwards.
+// block of each point summed afterwards.  Bound by L2 and HBM reads of the kept
+// blocks.  Gradient of 512 points over 16 layers of 192, all of it: 467 ms on
+// layers, 70 on planes, 19 of them the three products of the sums.
 template <int NT>
 __global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
 {

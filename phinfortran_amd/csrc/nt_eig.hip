@@ -788,7 +788,7 @@ hipError_t launch_schur(const EigArgs& a, hipStream_t s)
     // the 160 KB of LDS hold the matrix up to n = 96 (128 matrices: 4.8 ms, through L2 9.6)
     if (a.n <= 32) hipLaunchKernelGGL(k_schur_lds<32>, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
     else if (a.n <= 64) hipLaunchKernelGGL(k_schur_lds<64>, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
-    else if (a.n <= 96) hipLaunchKernelGGL(k_schur_lds<96>, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
+    else if (a.n <= SCHUR_LDS_MAX) hipLaunchKernelGGL(k_schur_lds<96>, dim3(a.sets * a.batch), dim3(NT), 0, s, a);
     else hipLaunchKernelGGL(k_schur, dim3(a.sets * a.batch), dim3(NT), sm, s, a);
     return hipGetLastError();
 }

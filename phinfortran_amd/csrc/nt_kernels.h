@@ -75,6 +75,7 @@ size_t dec_tile_scratch(int n);
 hipError_t launch_dec_tile(const DecTileArgs& a, hipStream_t s);
 
 // Batched complex Schur / eigen / square-root kernels (nt_eig.hip), FP64.
+constexpr int SCHUR_LDS_MAX = 96;      // up to here the decomposition keeps its matrix in LDS
 struct EigArgs {
     int n;
     BMatW<double> A;     // in: matrix; out: Schur form T (upper triangular)

@@ -414,7 +414,12 @@ void modes_run(nt_ctx* c, const nt_params* prm, int tb, int nl, int nr, int P, c
         // F = op(g) V  -> U (eigen input, overwritten by the eigenvectors)
         for (int d = d0; d < d0 + 2; ++d)
             gemm<T>(c, m, m, m, dirs[d].opg, dirs[d].g, OP_N, dirs[d].V, W(U[d], m), 1.0, none<T>(), 0.0, nullptr, P);
-        eig_run(c, m, R(U[d0], m), w[d0], W(U[d0], m), status, P, ar, eig_off, &e2);
+        // (past the LDS the decompositions live in the caches, which two sets of
+        // more than the CUs hold overflow: 1024 points of 160 with modes ran at
+        // 571 points/s together and 629 one after the other)
+        const bool both = m <= SCHUR_LDS_MAX || 2 * P <= 256;
+        if (!both) eig_run(c, m, e2.A, e2.w, e2.V, status, P, ar, eig_off);
+        eig_run(c, m, R(U[d0], m), w[d0], W(U[d0], m), status, P, ar, eig_off, both ? &e2 : nullptr);
         for (int d = d0; d < d0 + 2; ++d) {
             const Dir& D = dirs[d];
             double* kz = o.kz[d] ? o.kz[d] : kzs[d];
@@ -443,7 +448,8 @@ void modes_run(nt_ctx* c, const nt_params* prm, int tb, int nl, int nr, int P, c
         e2.A = R(Vh[d0 + 1], m);
         e2.w = nullptr;
         e2.V = W(Vh[d0 + 1], m);
-        sqrtm_run(c, m, R(Vh[d0], m), W(Vh[d0], m), status, P, ar, eig_off, &e2);
+        if (!both) sqrtm_run(c, m, e2.A, e2.V, status, P, ar, eig_off);
+        sqrtm_run(c, m, R(Vh[d0], m), W(Vh[d0], m), status, P, ar, eig_off, both ? &e2 : nullptr);
         // inv(U^+) for incident directions, inv(U) for outgoing ones
         for (int d = d0; d < d0 + 2; ++d) {
             copy_op<T>(c, m, m, R(U[d], m), W(T2, m), dirs[d].incident ? 1 : 0, (T)1, P);

@@ -303,7 +303,6 @@ void audit(nt_ctx* c, const M& m, int rows, int cols, int batch, int groups, con
     check_range(c, m.base, (size_t)(last + 1) * 2 * sizeof(T), what);
 }
 
-// C = alpha op(A) op(B) + beta Cin + diag
 // output tile set for an M x N product, 0 for none
 template <typename T>
 int gemm_tile_of(const nt_ctx* c, int M, int N)
@@ -312,6 +311,7 @@ int gemm_tile_of(const nt_ctx* c, int M, int N)
     return set == c->gemm_tile.end() ? 0 : set->second;
 }
 
+// C = alpha op(A) op(B) + beta Cin + diag
 template <typename T>
 void gemm(nt_ctx* c, int M, int N, int K, int opA, BMat<T> A, int opB, BMat<T> B, BMatW<T> C, double alpha,
           BMat<T> Cin, double beta, const T* diag, int batch, double nitems = -1, const int* active = nullptr,

@@ -993,6 +993,20 @@ __global__ __launch_bounds__(1024) void k_pl_gather(int P, const int* need, int 
     }
 }
 
+// out += the sum of S parts
+__global__ void k_pl_add_parts(long n, int S, const C2* part, C2* out)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    C2 v = out[i];
+    for (int g = 0; g < S; ++g) {
+        const C2 x = part[(long)g * n + i];
+        v.x += x.x;
+        v.y += x.y;
+    }
+    out[i] = v;
+}
+
 __global__ void k_pl_scatter(int n, const int* idx, const double* Tl, const double* Tr, const int* st, const int* it,
                              double* T_LR, double* T_RL, int* status, int* iters)
 {
@@ -1292,19 +1306,53 @@ void planes_adjoint(nt_ctx* c, const TdbArgs& a, const PlanDims& d, const PlanVi
     const long bb = (long)b * b, per = K * b;
     const T* CA = reinterpret_cast<const T*>(cv.CA);
     const T* RW = reinterpret_cast<const T*>(cv.RW);
+    // A product has the depth of all points but few tiles (17 layers of 192: 153
+    // workgroups on 256 CUs, 6.4 ms each): parts of the points are summed side by
+    // side, up to four workgroups per CU of them, into the decimation's scratch,
+    // which is free by now, and then added up; the points beyond equal parts
+    // form one more product.
+    T* part = h.nt <= PL_MAXNT ? reinterpret_cast<T*>(cv.scratch) : nullptr;
+    const long room = part ? 2L * n * DEC_SLOTS * NP * NP : 0;
+    const long tiles = (long)((b + 63) / 64) * ((b + 63) / 64);
     for (int k = 0; k < a.nk; ++k) {
-        const long q0 = (long)k0[k] * NP;
-        const int Kk = (k0[k + 1] - k0[k]) * NP;
-        if (!Kk) continue;
-        const BMat<T> Rm = bm<T>(RW + 2 * q0, per, (int)K), Cm = bm<T>(CA + 2 * q0 * b, per, b);
-        const BMat<T> Rn = bm<T>(RW + 2 * (per + q0), per, (int)K), Cn = bm<T>(CA + 2 * (per + q0 * b), per, b);
-        T* gd = reinterpret_cast<T*>(a.dHd) + 2 * (long)k * nw * bb;
-        gemm<T>(c, b, b, Kk, OP_C, Rm, OP_C, Cm, bw(gd, bb, b), 2.0, bm<T>(gd, bb, b), 1.0, nullptr, nw);
-        if (nc > 0 && a.dHdv) {
-            T* gv = reinterpret_cast<T*>(a.dHdv) + 2 * (long)k * nc * bb;
-            gemm<T>(c, b, b, Kk, OP_C, Rm, OP_C, Cn, bw(gv, bb, b), 2.0, bm<T>(gv, bb, b), 1.0, nullptr, nc);
-            gemm<T>(c, b, b, Kk, OP_N, Cm, OP_N, Rn, bw(gv, bb, b), 2.0, bm<T>(gv, bb, b), 1.0, nullptr, nc);
-        }
+        const int nk = k0[k + 1] - k0[k];
+        if (!nk) continue;
+        // out += 2 (A1 B1 + A2 B2) over the k-point's points, layers of the window
+        auto sum = [&](T* out, int layers, auto term, int terms) {
+            const long want = std::min<long>({8, (4 * 256 + tiles * layers - 1) / (tiles * layers),
+                                              room / ((long)layers * bb), (long)nk * NP / 512});
+            const int S = (int)std::max<long>(1, want), q = nk / S, rest = S > 1 ? nk - q * S : 0;
+            if (S > 1) check_range(c, part, sizeof(C2) * S * layers * bb, "gradient parts");
+            for (int i = 0; i < terms; ++i) {
+                const BMatW<T> to = S > 1 ? bw(part, bb, b, nullptr, (long)layers * bb) : bw(out, bb, b);
+                term(i, k0[k], q, to, S > 1 && i == 0 ? none<T>() : ro(to), layers, S);
+                if (rest) term(i, k0[k] + q * S, rest, bw(out, bb, b), bm<T>(out, bb, b), layers, 1);
+            }
+            if (S > 1) {
+                hipLaunchKernelGGL(k_pl_add_parts, dim3(nblk(layers * bb)), dim3(256), 0, s, layers * bb, S,
+                                   reinterpret_cast<const C2*>(part), reinterpret_cast<C2*>(out));
+                hipcheck(c, hipGetLastError(), "add parts");
+            }
+        };
+        // i of 0: R_l^+ C_l^+, 1: R_l^+ C_{l+1}^+, 2: C_l R_{l+1} over np points from p on
+        auto product = [&](int what, int p, int np, BMatW<T> to, BMat<T> from, int layers, int S) {
+            const long q0 = (long)p * NP, up = what == 0 ? 0 : per;
+            const BMat<T> Rm = bm<T>(RW + 2 * (q0 + (what == 2 ? up : 0)), per, (int)K, nullptr, (long)np * NP);
+            const BMat<T> Cm = bm<T>(CA + 2 * (q0 * b + (what == 1 ? up : 0)), per, b, nullptr, (long)np * NP * b);
+            if (what == 2)
+                gemm<T>(c, b, b, np * NP, OP_N, Cm, OP_N, Rm, to, 2.0, from, 1.0, nullptr, layers, -1, nullptr, S);
+            else
+                gemm<T>(c, b, b, np * NP, OP_C, Rm, OP_C, Cm, to, 2.0, from, 1.0, nullptr, layers, -1, nullptr, S);
+        };
+        sum(reinterpret_cast<T*>(a.dHd) + 2 * (long)k * nw * bb, nw,
+            [&](int, int p, int np, BMatW<T> to, BMat<T> from, int layers, int S) {
+                product(0, p, np, to, from, layers, S);
+            }, 1);
+        if (nc > 0 && a.dHdv)
+            sum(reinterpret_cast<T*>(a.dHdv) + 2 * (long)k * nc * bb, nc,
+                [&](int i, int p, int np, BMatW<T> to, BMat<T> from, int layers, int S) {
+                    product(1 + i, p, np, to, from, layers, S);
+                }, 2);
     }
     (void)d;
 }

@@ -226,3 +226,27 @@ def test_noalloc_and_no_check_agree(engine, T, planes_on):
                     assert np.array_equal(ref[k].cpu().numpy(), r[k].cpu().numpy()), (every, noalloc, k)
     finally:
         engine.set_decimation_check(4)
+
+
+@pytest.mark.parametrize("points", [63, 131, 300])
+def test_gradient_parts(engine, points):
+    """The window's sums over the points in parts side by side (from 1024 rows
+    of a k-point on) with points left over, against the same points in calls
+    too small to be split, whose gradients add up: the order of the sums is all
+    that differs, so they agree to the number of points times eps of the
+    largest sum of moduli."""
+    from phinfortran_amd import lattice as lt
+    from phinfortran_amd import transport as T
+    blk = lt.si_ge_interface_film(nx=2, ny=1, L=6, kfrac=(0.125, 0.25))
+    p = T.params("phonon")
+    E = np.linspace(2.0, 14.0, points) ** 2
+    d = engine.upload_blocks(blk)
+    w = np.linspace(0.5, 1.5, points)
+    print(f"gradient parts, {points} points", flush=True)
+    whole = engine.solve_tdb_adjoint(d, E, p, w, 1, 4)
+    parts = [engine.solve_tdb_adjoint(d, E[i:i + 15], p, w[i:i + 15], 1, 4) for i in range(0, points, 15)]
+    for k in ("dHamd", "dHamdv"):
+        got = whole[k].cpu().numpy()
+        each = [r[k].cpu().numpy() for r in parts]
+        bound = points * np.finfo(float).eps * sum(np.abs(x) for x in each).max()
+        assert np.abs(got - sum(each)).max() <= 16 * bound

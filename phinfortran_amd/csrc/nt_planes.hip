@@ -849,8 +849,8 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
 // another: the sums over the points of X_{j,i}^+ = R_i^+ C_j^+ are then one
 // product per layer and k-point, over 16 NT rows per point instead of a b x b
 // block of each point summed afterwards.  Bound by L2 and HBM reads of the kept
-// blocks.  Gradient of 512 points over 16 layers of 192, all of it: 467 ms on
-// layers, 70 on planes, 19 of them the three products of the sums.
+// blocks.  Gradient of 512 points over 16 layers of 192, all of it: 465 ms on
+// layers, 59 on planes: 43 forward, 10 the three products of the sums, 5 here.
 template <int NT>
 __global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
 {
@@ -1310,7 +1310,7 @@ void planes_adjoint(nt_ctx* c, const TdbArgs& a, const PlanDims& d, const PlanVi
     // workgroups on 256 CUs, 6.4 ms each): parts of the points are summed side by
     // side, up to four workgroups per CU of them, into the decimation's scratch,
     // which is free by now, and then added up; the points beyond equal parts
-    // form one more product.
+    // form one more product.  The three products 19 -> 10 ms at 512 points.
     T* part = h.nt <= PL_MAXNT ? reinterpret_cast<T*>(cv.scratch) : nullptr;
     const long room = part ? 2L * n * DEC_SLOTS * NP * NP : 0;
     const long tiles = (long)((b + 63) / 64) * ((b + 63) / 64);

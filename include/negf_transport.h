@@ -302,7 +302,10 @@ int nt_set_point_split(nt_ctx* ctx, int n);
  * 96 where the call may allocate and wait for the device (default on): the
  * same block elimination on smaller blocks, in FP64, which then serves
  * NT_PREC_MIXED calls too (faster than the FP32 factorisation it replaces).
- * Points with a singular or nearly singular plane are solved on the layers.
+ * Points with a singular or nearly singular plane are solved on the layers, and
+ * leads whose decimation lost digits on the planes are decimated on the layers
+ * (in the allocation-free entry, and where the host may not wait, the whole
+ * point is).
  * on = 0: always on the layers.  No counterpart in the reference. */
 int nt_set_planes(nt_ctx* ctx, int on);
 

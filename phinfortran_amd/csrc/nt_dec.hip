@@ -40,7 +40,6 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_dec_tile(DecTileArg
     C2 *al = sc, *aln = sc + NN, *be = sc + 2 * NN, *e = sc + 3 * NN, *G = sc + 4 * NN;
     C2* es = reinterpret_cast<C2*>(bptr(a.es, p, 0));
     const int lds = a.es.ld;
-    Grow gr;
     Blk<NT> x, y, u;
     auto load = [&](Blk<NT>& b, const C2* m) __attribute__((always_inline)) { blk_load<NT>(b, LdN{m, NP}, w); };
     auto store = [&](const Blk<NT>& b, C2* m) __attribute__((always_inline)) { blk_store<NT>(b, m, NP, w); };
@@ -104,7 +103,7 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_dec_tile(DecTileArg
                     x.im[t][r] = in ? (dg ? zi : 0.0) - x.im[t][r] : 0.0;
                 }
         }
-        wg_inverse<NT>(work, il, x, gr, [&](int i, int j, C2 v) { G[i + j * NP] = v; });
+        wg_inverse<NT>(work, il, x, [&](int i, int j, C2 v) { G[i + j * NP] = v; });
         // beta's side: u = beta' (held back: the others still read beta)
         load(x, be);
         blk_zero<NT>(y);

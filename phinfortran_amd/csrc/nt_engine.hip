@@ -208,7 +208,51 @@ constexpr int DEC_TILE_STEPS = 20000;      // in one kernel: about 0.5 s at n = 
 template <typename T>
 struct DecimationOut {
     BMatW<T> g, sigma, gamma;
+    // residual of sigma's own equation, item q's to res[q * res_stride]
+    double* res = nullptr;
+    int res_stride = 0;
+    BMatW<T> es{nullptr, 0, 0, nullptr, 0, 0};      // H00 + Sigma as the recursion adds it up
 };
+
+// The recursion adds up es = H00 + Sigma, and Sigma = V^+ (z - es)^-1 V: the
+// largest difference of the two over the largest element (NaN with a NaN
+// anywhere).  One workgroup per item.
+__global__ __launch_bounds__(256) void k_dec_residual(int n, const double2* es, BMat<double> H00, BMatW<double> sigma,
+                                                      double* res, int stride)
+{
+    const int q = blockIdx.x, t = threadIdx.x;
+    const double2* e = es + (long)q * n * n;
+    const double2* h = reinterpret_cast<const double2*>(bptr(H00, q, 0));
+    const double2* s = reinterpret_cast<const double2*>(bptr(sigma, q, 0));
+    double d = 0.0, m = 0.0;
+    int bad = 0;
+    for (int i = t; i < n * n; i += 256) {
+        const int r = i % n, c = i / n;
+        const double2 x = e[i], y = h[r + (long)c * H00.ld], v = s[r + (long)c * sigma.ld];
+        const double p = hypot(x.x - y.x - v.x, x.y - y.y - v.y), a = hypot(v.x, v.y);
+        bad |= p != p || a != a;
+        d = fmax(d, p);
+        m = fmax(m, a);
+    }
+    for (int o = 32; o; o >>= 1) {
+        d = fmax(d, __shfl_xor(d, o));
+        m = fmax(m, __shfl_xor(m, o));
+    }
+    __shared__ double wd[4], wm[4];
+    bad = __syncthreads_or(bad);
+    if ((t & 63) == 0) {
+        wd[t >> 6] = d;
+        wm[t >> 6] = m;
+    }
+    __syncthreads();
+    if (t == 0) {
+        for (int i = 1; i < 4; ++i) {
+            d = fmax(d, wd[i]);
+            m = fmax(m, wm[i]);
+        }
+        res[(long)q * stride] = bad ? __longlong_as_double(0x7ff8000000000000LL) : d == 0.0 ? 0.0 : d / m;
+    }
+}
 
 template <typename T>
 void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger, const T* z, double conv,
@@ -272,6 +316,7 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
             hipcheck(c, hipGetLastError(), "dec mask");
             fin = active;
         }
+        if (out.es.base) copy_op<T>(c, n, n, bm<T>(es, nn, n), out.es, 0, (T)1, Q);
         // g = (z - es)^-1 for every item (surface.f90:497)
         inverse<T>(c, n, bw(W, nn, n), bm<T>(es, nn, n), z, out.g, status, Q, -1, fin);
         if (out.sigma.base) {
@@ -281,6 +326,16 @@ void decimate(nt_ctx* c, int n, int Q, BMat<T> H00, BMat<T> V, int alpha_dagger,
             gemm<T>(c, n, n, n, OP_N, bm<T>(t12, 2 * nn, n), alpha_dagger ? OP_N : OP_C, V, out.sigma, 1.0, none<T>(),
                     0.0, nullptr, Q, -1, fin);
             if (out.gamma.base) gamma_op<T>(c, n, ro(out.sigma), out.gamma, Q);
+            if constexpr (std::is_same<T, double>::value)
+                if (out.res) {
+                    check_range(c, out.res, sizeof(double) * ((size_t)out.res_stride * (Q - 1) + 1), "dec residual");
+                    launch(c, NT_K_ELEM, 0, "dec residual", [&] {
+                        hipLaunchKernelGGL(k_dec_residual, dim3(Q), dim3(256), 0, s, n,
+                                           reinterpret_cast<const double2*>(es), H00, out.sigma, out.res,
+                                           out.res_stride);
+                        return hipGetLastError();
+                    });
+                }
         }
     };
     // FP64: one kernel for the whole recursion (n = 48: 13.6 ms against 21 for
@@ -1412,10 +1467,85 @@ constexpr double MIXED_BUDGET_BYTES = 64.0 * 1024 * 1024 * 1024;
 size_t lead_sigma_scratch(int n, int Q) { return decimate_scratch<double>(n, Q); }
 
 void lead_sigma(nt_ctx* c, int n, int Q, BMat<double> H00, BMat<double> V, const double* z, double conv, int max_iter,
-                BMatW<double> g, BMatW<double> sigma, int* status, int* iters, Arena& ar, size_t scratch_off)
+                BMatW<double> g, BMatW<double> sigma, int* status, int* iters, double* res, int res_stride, Arena& ar,
+                size_t scratch_off)
 {
-    DecimationOut<double> o{g, sigma, nonew<double>()};
+    DecimationOut<double> o{g, sigma, nonew<double>(), res, res_stride};
     decimate<double>(c, n, Q, H00, V, 1, z, conv, max_iter, o, status, iters, ar, scratch_off);
+}
+
+namespace {
+struct LayersSigma {
+    int *idx, *idx1, *sts, *its;
+    double *z, *zdev, *zs, *lh, *lv, *g;
+    size_t scr;
+};
+LayersSigma layers_sigma_carve(Arena& ar, const TdbArgs& a, int P)
+{
+    const size_t n2 = sizeof(nt_c128) * sigma_stride(a), P4 = sizeof(double) * 4 * (size_t)P;
+    LayersSigma v;
+    v.idx = ar.ptr<int>(ar.take(sizeof(int) * 2 * P));
+    v.idx1 = ar.ptr<int>(ar.take(sizeof(int) * P));
+    v.sts = ar.ptr<int>(ar.take(sizeof(int) * 2 * P));
+    v.its = ar.ptr<int>(ar.take(sizeof(int) * 2 * P));
+    v.z = ar.ptr<double>(ar.take(P4));
+    v.zdev = ar.ptr<double>(ar.take(P4));
+    v.zs = ar.ptr<double>(ar.take(P4));
+    v.lh = ar.ptr<double>(ar.take(a.nl == a.nr ? 2 * n2 * a.nk : 0));
+    v.lv = ar.ptr<double>(ar.take(a.nl == a.nr ? 2 * n2 * a.nk : 0));
+    v.g = ar.ptr<double>(ar.take(2 * n2 * P));
+    v.scr = ar.off;
+    ar.take(decimate_scratch<double>(std::max(a.nl, a.nr), 2 * P));
+    return v;
+}
+}  // namespace
+
+size_t layers_sigma_scratch(const TdbArgs& a, int P)
+{
+    Arena ar;
+    layers_sigma_carve(ar, a, P);
+    return ar.off;
+}
+
+void layers_sigma(nt_ctx* c, const nt_params* prm, const TdbArgs& a, int P, const double* E, const int* kidx,
+                  double* sigma, double* es, int* status, int* iters, Arena& ar, size_t scratch_off)
+{
+    typedef double T;
+    hipStream_t s = c->stream;
+    Arena la = ar;
+    la.off = scratch_off;
+    const LayersSigma v = layers_sigma_carve(la, a, P);
+    const long nn = sigma_stride(a);
+    hipLaunchKernelGGL(k_lead_setup, dim3(nblk(P)), dim3(256), 0, s, E, kidx, a.nk, P, 1, prm->eta, prm->eta0,
+                       prm->eta_mode, prm->device_eta_factor, v.idx, v.z, (double*)nullptr, v.zdev);
+    hipcheck(c, hipGetLastError(), "lead setup");
+    zero_dev(c, status, sizeof(int) * 2 * P, s);
+    const T *Haml = reinterpret_cast<const T*>(a.Haml), *Hamlv = reinterpret_cast<const T*>(a.Hamlv),
+            *Hamr = reinterpret_cast<const T*>(a.Hamr), *Hamrv = reinterpret_cast<const T*>(a.Hamrv);
+    if (a.nl == a.nr) {
+        const long n_a = nn * a.nk;
+        auto stack = [&](const T* l, const T* r, T* o) {
+            hipLaunchKernelGGL(k_copy_lead_stack, dim3(nblk(n_a)), dim3(256), 0, s, reinterpret_cast<const double2*>(l),
+                               reinterpret_cast<const double2*>(r), reinterpret_cast<double2*>(o), n_a);
+            hipcheck(c, hipGetLastError(), "lead stack");
+        };
+        stack(Haml, Hamr, v.lh);
+        stack(Hamlv, Hamrv, v.lv);
+        DecimationOut<T> o{bw(v.g, nn, a.nl), bw(sigma, nn, a.nl), nonew<T>(), nullptr, 0, bw(es, nn, a.nl)};
+        lead_gfs(c, prm, a.nl, 2 * P, 2 * a.nk, v.lh, v.lv, v.idx, 1, v.z, o, status, iters, la, v.scr);
+        return;
+    }
+    hipLaunchKernelGGL(k_lead_split, dim3(nblk(P)), dim3(256), 0, s, v.z, (const double*)nullptr, v.idx, P, v.zs,
+                       (double*)nullptr, v.idx1);
+    hipcheck(c, hipGetLastError(), "lead split");
+    zero_dev(c, v.sts, sizeof(int) * 2 * P, s);
+    DecimationOut<T> l{bw(v.g, 2 * nn, a.nl), bw(sigma, 2 * nn, a.nl), nonew<T>(), nullptr, 0, bw(es, 2 * nn, a.nl)};
+    lead_gfs(c, prm, a.nl, P, a.nk, Haml, Hamlv, v.idx1, 1, v.zs, l, v.sts, v.its, la, v.scr);
+    DecimationOut<T> r{bw(v.g + 2 * nn, 2 * nn, a.nr), bw(sigma + 2 * nn, 2 * nn, a.nr), nonew<T>(), nullptr, 0,
+                       bw(es + 2 * nn, 2 * nn, a.nr)};
+    lead_gfs(c, prm, a.nr, P, a.nk, Hamr, Hamrv, v.idx1, 1, v.zs + 2 * P, r, v.sts + P, v.its + P, la, v.scr);
+    hipLaunchKernelGGL(k_lead_merge, dim3(nblk(P)), dim3(256), 0, s, v.sts, v.its, P, status, iters);
+    hipcheck(c, hipGetLastError(), "lead merge");
 }
 
 void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)

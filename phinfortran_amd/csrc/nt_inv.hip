@@ -462,9 +462,8 @@ __global__ __launch_bounds__(64 * NT, 2) void k_inv_reg(InvArgs<double> a)
         if (nan) info = -1;
     }
     double* X = bptr(a.X, p, 0);
-    Grow gr;
     const InvLds il{piv, cinv, &info};
-    wg_inverse<NT>(work, il, m, gr, [&](int i, int j, C2 v) {
+    wg_inverse<NT>(work, il, m, [&](int i, int j, C2 v) {
         if (i < n && j < n) *reinterpret_cast<C2*>(X + 2 * (i + (long)j * a.X.ld)) = v;
     });
     // merge into the caller's status: the first error of an item wins

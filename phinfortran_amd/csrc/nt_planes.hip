@@ -41,17 +41,40 @@ constexpr int PL_PERM = 16 * PL_BIGNT;
 __host__ __device__ constexpr int class_nt(int t) { return t < PL_MAXNT ? t + 1 : PL_BIGNT; }
 constexpr int PL_WAVES = 2;          // waves per SIMD the solver kernels are built for
 constexpr int PL_NLV = 128;         // levels a layer may have
-// A decimation step whose cell is nearly singular at E loses digits that the
-// later steps do not bring back, on planes and on layers alike: two correct
-// evaluations of T then differ by more than rounding (1e-6 and more on the
-// graphene ribbon at eta = 1e-8 eV, where some points overflow).  Such points
-// are left to the layers, so that the planes do not move them.  The measure is
-// g = |z - e|_max |(z - e)^-1|_max over the steps, and as the loss grows with
-// how far the broadening is below the energy scale, g (1e-7 scale / eta)^2 is
-// what is bounded: with the bound below the rest of the ribbon's points agree
-// to 1e-8, at 250 of 2048 left to the layers; of the phonon workloads (eta
-// about 1e-6 of the scale) at most a few in a thousand are.
-constexpr double PL_GROWTH = 2.0e8;
+// Where planes and layers lose digits, they lose different ones, and the planes
+// are not to move the results: what lost digits is done on the layers.
+// Leads: steps whose cell is nearly singular at E lose digits that the later
+// steps do not bring back, on planes and on layers alike (planes about a third
+// of what the layers lose, against an 80-bit recursion).  The self-energy's own
+// equation shows the loss: the recursion adds up es = e + Sigma, and Sigma = V^+
+// (z - es)^-1 V.  Where the residual, over Sigma's largest element, passes the
+// bound, the layers' self-energy takes its place.  Films of 192, 20 times 1024
+// points, largest differences of planes and layers by residual: T 7e-7 up to
+// 3e-7, 2e-6 up to 1e-6, 1e-5 beyond (2 points); the gradient of a point, over
+// its norm, 2e-7 up to 3e-8, 2e-6 up to 3e-7, 1e-5 up to 1e-6, 7e-5 beyond.  The
+// leads of a few points of 192 take 30 ms on the layers (80: 13), whence not
+// less: 0.1 of 1024 points are beyond the bound of T, one beyond the gradient's.
+constexpr double PL_RESIDUAL = 1.0e-6, PL_RESIDUAL_ADJ = 1.0e-7;
+// A loss beyond the broadening may make the recursion grow without end instead:
+// of 360,000 energies of ribbons at eta = 1e-8 eV the layers' did at 47 where the
+// planes' did not, with residuals of 2 eta / scale and more.  So the bound is at
+// most eta / scale, and whether a recursion ends is decided on the layers: 31 of
+// 2048 points of the ribbon, 0.4 of 1024 of the film.
+constexpr double PL_RESIDUAL_ETA = 1.0;
+// Planes inside a lead cell and of the device are eliminated with pivots from
+// one plane only, and a plane may be nearly singular at E where its layer is
+// not.  With kappa = |G|max scale of the eliminated planes, T then is off by
+// 1e-16 to 5e-16 kappa of itself: layers of 13 + 14 + 13 degrees of freedom,
+// the middle ones uncoupled sites at E, eta = 1e-8: kappa 3e7, error 3e-8 (on
+// layers 3e-11), at kappa 2e5 3e-10.  Where T < 1 the error counts less, down
+// to T = 0.01.  The film reaches 4e4, the wire 2e5 (one point of 3000 beyond
+// 1e5, at T = 0.26), the ribbon 2e6 in its gap.
+constexpr double PL_KAPPA = 1.0e5;
+
+// need[p]: 0 solved on the planes, else why it is not (yet)
+enum { NEED_LAYERS = 1, NEED_AFTER_SWEEP = 2, NEED_LEADS = 3 };
+// counters of a solve (device ints; the first three of a chunk)
+enum { CNT_LAYERS = 0, CNT_AFTER_SWEEP = 1, CNT_LEADS = 2, CNT_STEPS = 3, CNT_N = 4 };
 
 // ------------------------------------------------------------------ the plan
 // Device arrays of the plan (ints), carved from one buffer.
@@ -493,7 +516,6 @@ __device__ __forceinline__ void blk_shift(Blk<NT>& m, double zr, double zi, int 
         }
 }
 
-// largest value over the workgroup, in every thread
 // ------------------------------------------------------------------ decimation
 // Lopez-Sancho decimation (negf/surface.f90:479-497) of a lead cell whose
 // couplings run from its plane B (facing the device) to plane A of the next
@@ -551,7 +573,7 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
     C2 *T1 = slot(11), *T2 = slot(13), *G = slot(15);     // NP x 2 NP twice, 2 NP square
     C2* cbn = T1;                                         // (before the steps)
     if (threadIdx.x == 0) s.info = 0;
-    Grow gr;
+    double mid = 0.0;              // |G|max of the planes inside the cell, the wave's columns
     Blk<NT> x, y;
     auto load = [&](Blk<NT>& b, const C2* m) __attribute__((always_inline)) { blk_load<NT>(b, LdN{m, NP}, wc); };
     auto store = [&](const Blk<NT>& b, C2* m) __attribute__((always_inline)) { blk_store<NT>(b, m, NP, wc); };
@@ -559,6 +581,7 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
         load(x, from);
         store(x, to);
     };
+    int it = 0, j = 1, mode = mc > 2 ? 0 : 1;
     // G = (z - [[a, b], [c, d]])^-1 of planes of n1 and n2; no second plane
     // where n2 = 0.  Wave w holds column 16 w + lane % 16 of the 2 NP.
     auto invert = [&](const C2* ma, const C2* mb, const C2* mcc, const C2* md, int n1, int n2) __attribute__((always_inline)) {
@@ -582,7 +605,11 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
                 m.im[t][r] = in ? (dg ? zi : 0.0) - m.im[t][r] : 0.0;
             }
         __syncthreads();
-        wg_inverse<2 * NT>(s.work, il, m, gr, [&](int i, int j, C2 v) { G[i + j * NP2] = v; });
+        wg_inverse<2 * NT>(s.work, il, m, [&](int i, int j, C2 v) {
+            G[i + j * NP2] = v;
+            auto in = [&](int r) { return r < NP ? r < n1 : r - NP < n2; };
+            if (mode == 0 && in(i) && in(j)) mid = fmax(mid, fabs(v.x) + fabs(v.y));
+        });
     };
     const C2 *G11 = G, *G21 = G + NP, *G12 = G + (long)NP * NP2, *G22 = G + NP + (long)NP * NP2;
     const int nA = a.psize[plane(0)], nB = a.psize[plane(mc - 1)];
@@ -601,7 +628,6 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
     // and B (cf = A -> j, cb = j -> A) while there are any, then the steps,
     // then the last one with es (one copy of the inverse's code, and the
     // registers of one).
-    int it = 0, j = 1, mode = mc > 2 ? 0 : 1;
     auto steps_begin = [&]() __attribute__((always_inline)) {
         if (cbn != T1) {              // T1's slot is needed by the steps
             copy(cbn, cb);
@@ -609,6 +635,8 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
         }
         copy(eB0, eB);
         copy(esA, eA);
+        copy(cfn, eA);                // (a free slot from here on)
+        if (mc > 2) mid = wg_max<2 * NT>(s.red, mid);
         amax = wg_max<2 * NT>(s.red, half ? 0.0 : amax);      // its barriers also publish the slots
     };
     if (mode) steps_begin();
@@ -691,7 +719,9 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
         amax = wg_max<2 * NT>(s.red, half ? 0.0 : blk_maxabs<NT>(y));
     }
     const int not_conv = amax > a.conv;
-    // Sigma = V^+ g_BB V on A with g = (z - es)^-1
+    // Sigma = V^+ g_BB V on A with g = (z - es)^-1, and its difference to what
+    // the steps added up
+    double smax = 0.0, rmax = 0.0;
     if (!half) {
         load(x, V);
         blk_zero<NT>(y);
@@ -699,6 +729,17 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
         blk_zero<NT>(x);
         blk_mul<NT>(x, LdC{V, NP}, y);
         C2* out = a.sigma + (long)item * NN;
+        smax = blk_maxabs<NT>(x);
+        load(y, cfn);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) y.re[t] += x.re[t], y.im[t] += x.im[t];
+        {
+            Blk<NT> u;
+            load(u, esA);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) y.re[t] -= u.re[t], y.im[t] -= u.im[t];
+        }
+        rmax = blk_maxabs<NT>(y);
         if (side) {
             store(x, out);
         } else {
@@ -710,13 +751,14 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
                     out[16 * wc + l15 + (16 * t + 4 * r + q) * NP] = make_double2(x.re[t][r], -x.im[t][r]);
         }
     }
-    const double ga = wg_max<2 * NT>(s.red, gr.a), gg = wg_max<2 * NT>(s.red, gr.g);
+    smax = wg_max<2 * NT>(s.red, smax);
+    rmax = wg_max<2 * NT>(s.red, rmax);
     scale = fmax(wg_max<2 * NT>(s.red, scale), fabs(E));
     if (threadIdx.x == 0) {
-        const double rb = 1.0e-7 * scale / fabs(et);
         a.iters[item] = it;
         a.status[item] = s.info ? s.info : not_conv ? NT_ERR_NOT_CONVERGED : 0;
-        a.grow[item] = ga * gg * rb * rb;      // (eta = 0: not finite, left to the layers)
+        // (a Sigma that is not finite: no number)
+        a.loss[item] = LeadLoss{mid * scale, rmax == 0.0 ? 0.0 : rmax / smax, scale};
     }
 }
 
@@ -757,7 +799,7 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
     const C2* Ss = a.sigma + (long)(2 * p + sys) * NN;
     const C2* Se = a.sigma + (long)(2 * p + 1 - sys) * NN;
     if (threadIdx.x == 0) s.info = 0;
-    Grow gr;
+    unsigned gmax = 0;             // upper word of |G|max, the wave's columns
     Blk<NT> R;
     blk_zero<NT>(R);
 #pragma unroll 1
@@ -765,9 +807,9 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
         const int j = sys ? M - 1 - i : i;
         Blk<NT> m;
         blk_load<NT>(m, LdN{Hk + (long)j * NN, NP}, w);
-        if (i == 0 || i == M - 1) {
+        if (j == 0 || j == M - 1) {
             Blk<NT> sg;
-            blk_load<NT>(sg, LdN{i ? Se : Ss, NP}, w);
+            blk_load<NT>(sg, LdN{j || !a.left ? a.sigma + (long)(2 * p + (j != 0)) * NN : a.left + (long)p * NN, NP}, w);
 #pragma unroll
             for (int t = 0; t < NT; ++t) m.re[t] += sg.re[t], m.im[t] += sg.im[t];
         }
@@ -791,7 +833,14 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
         }
         blk_shift<NT>(m, E, i < lead_planes ? et : a.dev_factor * et, a.psize[j], w);
         __syncthreads();
-        wg_inverse<NT>(s.g, il, m, gr, [&](int r, int c, C2 v) { s.g[r + c * LD] = v; });
+        double g = 0.0;
+        const int n = a.psize[j];
+        wg_inverse<NT>(s.g, il, m, [&](int r, int c, C2 v) {
+            s.g[r + c * LD] = v;
+            if (r < n && c < n) g = fmax(g, fabs(v.x) + fabs(v.y));
+        });
+        const unsigned gh = wave_max((unsigned)(__double_as_longlong(g) >> 32));
+        gmax = gh > gmax ? gh : gmax;
         if (i) {
             Blk<NT> n;
             blk_zero<NT>(n);
@@ -814,11 +863,11 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
     blk_mul<NT>(y, LdGamT{Se, NP}, R);
     __syncthreads();
     blk_store<NT>(y, s.g, LD, w);
-    Blk<NT> g;
-    blk_load<NT>(g, LdGamT{Ss, NP}, w);
+    Blk<NT> gs;
+    blk_load<NT>(gs, LdGamT{Ss, NP}, w);
     __syncthreads();
     blk_zero<NT>(y);
-    blk_mul<NT>(y, LsN{s.g, LD}, g);
+    blk_mul<NT>(y, LsN{s.g, LD}, gs);
     double tr = 0.0;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -835,6 +884,8 @@ __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArg
         a.T[item] = t;
         a.status[item] = s.info;
     }
+    const double g = wg_max<NT>(s.red, __longlong_as_double((long long)gmax << 32));
+    if (threadIdx.x == 0) a.grow[item] = g;
 }
 
 // --------------------------------------------------------------------- adjoint
@@ -919,38 +970,91 @@ __global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
     }
 }
 
-// need[p]: the point is left to the layers (plan refused, a singular plane of
-// a lead, a value not finite, too much growth); *count: how many are
-__global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const double* grow, int* need, int* count)
+// NEED_LAYERS: plan refused, a singular plane of a lead; lossy: what a point
+// needs whose leads lost digits or left the finite numbers
+__global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const LeadLoss* loss, const double* E, double eta,
+                           double eta0, int mode, double res_max, int lossy, int* need,
+                           int* count)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P) return;
-    bool bad = !h->ok;
-    if (!bad)
+    int why = h->ok ? 0 : NEED_LAYERS;
+    if (!why) {
+        const double e = E[p], et = mode == NT_ETA_RELATIVE ? e * eta + eta0 : eta;
+        bool bad = false, lost = false;
         for (int i = 0; i < 2; ++i) {
             const int d = dst[2 * p + i];
-            bad = bad || (d != 0 && d != NT_ERR_NOT_CONVERGED) || (d == 0 && !(grow[2 * p + i] <= PL_GROWTH));
+            const LeadLoss l = loss[2 * p + i];
+            bad = bad || (d != 0 && d != -1 && d != NT_ERR_NOT_CONVERGED);
+            lost = lost || d == -1 || (d == 0 && !(l.res <= fmin(res_max, PL_RESIDUAL_ETA * fabs(et) / l.scale) &&
+                                        l.mid <= PL_KAPPA));
         }
-    need[p] = bad;
-    if (bad) atomicAdd(count, 1);
+        why = bad ? NEED_LAYERS : lost ? lossy : 0;
+    }
+    need[p] = why;
+    if (why) atomicAdd(count + (why == NEED_LEADS ? CNT_LEADS : CNT_LAYERS), 1);
+}
+
+// Self-energies of the layers (layers_sigma) of the points idx onto the planes
+// that face the leads, with their statuses and step counts; a point with a
+// singular matrix on the layers is left to them.  The layers' sweep begins
+// with the left lead's es and closes with V^+ g V of the right one, which differ
+// by the digits lost: left takes the former.  blockIdx.y: item.
+__global__ void k_pl_put_sigma(PlanDims d, PlanView v, BlocksIn B, const int* idx, const int* kidx, const C2* S,
+                               const C2* ES, long stride, const int* st, const int* it, C2* sigma, C2* left, int* dst,
+                               int* dit, int* need, int* count)
+{
+    const int q = blockIdx.y, p = idx[q / 2], side = q & 1, M = v.h->M, NP = 16 * v.h->nt;
+    const int pl = side ? M - 1 : 0, n = v.psize[pl], ld = side ? d.nr : d.nl;
+    const int* pm = v.perm + (long)pl * PL_PERM;
+    const C2 *s = S + q * stride, *es = ES + q * stride;
+    const C2* H = layer_H(d, B, side ? d.L + 1 : 0, kidx ? kidx[q / 2] : 0);
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < NP * NP; e += gridDim.x * blockDim.x) {
+        const int r = e % NP, c = e / NP;
+        C2 x = make_double2(0.0, 0.0), y = x;
+        if (r < n && c < n) {
+            // (retarded = adjoint of the left lead's advanced)
+            const long o = side ? pm[r] + (long)pm[c] * ld : pm[c] + (long)pm[r] * ld;
+            x = s[o];
+            y = make_double2(es[o].x - H[o].x, es[o].y - H[o].y);
+            if (!side) x.y = -x.y, y.y = -y.y;
+        }
+        sigma[(long)(2 * p + side) * NP * NP + e] = x;
+        if (!side) left[(long)p * NP * NP + e] = y;
+    }
+    if (blockIdx.x || threadIdx.x) return;
+    dst[2 * p + side] = st[q];
+    dit[2 * p + side] = it[q];
+    if (!side) {
+        bool bad = false;
+        for (int i = 0; i < 2; ++i)
+            bad = bad || (st[q + i] != 0 && st[q + i] != -1 && st[q + i] != NT_ERR_NOT_CONVERGED);
+        need[p] = bad ? NEED_LAYERS : 0;
+        if (bad) atomicAdd(count + CNT_LAYERS, 1);
+    }
 }
 
 // Points solved on the planes: statuses, iteration counts, clamps.  A singular
-// plane in the sweep sets need[p] too (counted in count[1]); count[2] sums the
-// decimation steps.
+// or nearly singular plane in the sweep sets need[p] too; count[CNT_STEPS] sums
+// the decimation steps.
 __global__ void k_pl_finish(int P, const int* dst, const int* dit, const int* sst, const double* T,
-                            const int* first_mask, int* need, int* count, double* T_LR, double* T_RL, int* status,
-                            int* iters)
+                            const LeadLoss* loss, const double* grow, const int* first_mask, int* need, int* count,
+                            double* T_LR, double* T_RL, int* status, int* iters)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P || need[p]) return;
-    if (sst[2 * p] || sst[2 * p + 1]) {
-        need[p] = 2;
-        atomicAdd(count + 1, 1);
+    double tl = T[2 * p], tr = T[2 * p + 1];
+    // a lead's recursion that left the finite numbers on the layers: no T
+    const bool none = dst[2 * p] == -1 || dst[2 * p + 1] == -1;
+    if (none) tl = tr = __longlong_as_double(0x7ff8000000000000LL);
+    const double kappa = fmax(grow[2 * p], grow[2 * p + 1]) * fmax(loss[2 * p].scale, loss[2 * p + 1].scale);
+    if (!none && (sst[2 * p] || sst[2 * p + 1] || tl != tl || tr != tr ||
+        !(kappa * fmin(fmax(fmax(tl, tr), 0.01), 1.0) <= PL_KAPPA))) {
+        need[p] = NEED_AFTER_SWEEP;
+        atomicAdd(count + CNT_AFTER_SWEEP, 1);
         return;
     }
-    atomicAdd(count + 2, dit[2 * p] + dit[2 * p + 1]);
-    double tl = T[2 * p], tr = T[2 * p + 1];
+    atomicAdd(count + CNT_STEPS, dit[2 * p] + dit[2 * p + 1]);
     if (tl < 1.0e-60) tl = 0.0;       // negf/lesser.f90:795-800
     if (tr < 1.0e-60) tr = 0.0;
     if (first_mask && first_mask[p]) tl = tr = 0.0;      // negf/lesser.f90:802-807
@@ -1041,24 +1145,27 @@ void ensure_plan_buf(nt_ctx* c, size_t bytes)
 // gathered inputs and results of the points left to the layers
 void ensure_left_buf(nt_ctx* w, size_t bytes)
 {
-    if (w->left_bytes >= bytes) return;
-    if (w->left_buf) {
-        hipcheck(w, hipStreamSynchronize(w->stream), "hipStreamSynchronize");
-        unreg_region(w, w->left_buf);
-        hipcheck(w, hipFree(w->left_buf), "hipFree");
-        w->left_buf = nullptr;
-        w->left_bytes = 0;
+    unreg_region(w, w->left_buf);
+    if (w->left_bytes < bytes) {
+        if (w->left_buf) {
+            hipcheck(w, hipStreamSynchronize(w->stream), "hipStreamSynchronize");
+            hipcheck(w, hipFree(w->left_buf), "hipFree");
+            w->left_buf = nullptr;
+            w->left_bytes = 0;
+        }
+        hipcheck(w, hipMalloc(&w->left_buf, bytes), "hipMalloc points");
+        w->left_bytes = bytes;
     }
-    hipcheck(w, hipMalloc(&w->left_buf, 2 * bytes), "hipMalloc points");
-    w->left_bytes = 2 * bytes;
+    reg_region(w, w->left_buf, w->left_bytes);
 }
 
 // per point of a chunk: the two leads' decimation slots and self-energies,
-// statuses, counts, growth, T of both directions
+// statuses, counts, digits lost, T of both directions
 struct ChunkView {
-    C2 *scratch, *sigma;
+    C2 *scratch, *sigma, *left;
     int *dst, *dit, *sst;
-    double *dgrow, *T;
+    LeadLoss* loss;
+    double *T, *grow;
     C2 *keep = nullptr, *CA = nullptr, *RW = nullptr;      // adjoint
     int* place = nullptr;
 };
@@ -1069,10 +1176,12 @@ ChunkView chunk_carve(Arena& a, int P, int NN)
     ChunkView v;
     v.scratch = a.ptr<C2>(a.take(NN <= 256 * PL_MAXNT * PL_MAXNT ? sizeof(C2) * it * DEC_SLOTS * NN : 0));
     v.sigma = a.ptr<C2>(a.take(sizeof(C2) * it * NN));
+    v.left = a.ptr<C2>(a.take(sizeof(C2) * P * NN));
     v.dst = a.ptr<int>(a.take(sizeof(int) * it));
     v.dit = a.ptr<int>(a.take(sizeof(int) * it));
     v.sst = a.ptr<int>(a.take(sizeof(int) * it));
-    v.dgrow = a.ptr<double>(a.take(sizeof(double) * it));
+    v.loss = a.ptr<LeadLoss>(a.take(sizeof(LeadLoss) * it));
+    v.grow = a.ptr<double>(a.take(sizeof(double) * it));
     v.T = a.ptr<double>(a.take(sizeof(double) * it));
     return v;
 }
@@ -1142,8 +1251,9 @@ __global__ void k_pl_cell_mid(int M, int NP, int mc, const int* psize, const C2*
     }
 }
 
-// the cell's own blocks added to He (cleared first where add = 0); z - 1 on the
-// padding's diagonal (the decimation inverts z - He)
+// the cell's own blocks added to He (cleared first where add = 0); the padding's
+// diagonal is 0, or -1 at E = 0: the decimation inverts z - He, and z without
+// real part may be nothing, while z - (z - 1) is 0 from |E| = 2^53 on
 __global__ void k_pl_cell_own(int M, int NP, int mc, const int* psize, const C2* H, const C2* U, const C2* Lw,
                               const int* idx, const double* z, int add, C2* He)
 {
@@ -1159,13 +1269,13 @@ __global__ void k_pl_cell_own(int M, int NP, int mc, const int* psize, const C2*
             x.y += b.y;
         }
         const int pl = hr ? mc - 1 : 0;
-        if (r == c && r0 >= psize[side ? M - 1 - pl : pl]) x = make_double2(z[2 * q] - 1.0, z[2 * q + 1]);
+        if (r == c && r0 >= psize[side ? M - 1 - pl : pl]) x = make_double2(z[2 * q] == 0.0 ? -1.0 : 0.0, 0.0);
         He[(long)q * 4 * NN + e] = x;
     }
 }
 
 // retarded self-energy on plane A: the right lead's own, the left's adjoint
-__global__ void k_pl_cell_sigma(int NP, const C2* S, C2* sigma, double* grow)
+__global__ void k_pl_cell_sigma(int NP, const C2* S, C2* sigma)
 {
     const int q = blockIdx.y, N2 = 2 * NP;
     const long NN = (long)NP * NP;
@@ -1176,7 +1286,46 @@ __global__ void k_pl_cell_sigma(int NP, const C2* S, C2* sigma, double* grow)
         if (!(q & 1)) x.y = -x.y;
         sigma[(long)q * NN + e] = x;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) grow[q] = 0.0;
+}
+
+// LeadLoss of the cells but for the residual: the middle planes' inverse G1
+// (mc > 2), the cell's first plane, its coupling and E.  One workgroup per item.
+__global__ __launch_bounds__(256) void k_pl_cell_loss(int M, int NP, int mc, const int* psize, const C2* H,
+                                                      const C2* VS, const C2* G1, const int* idx, const double* z,
+                                                      LeadLoss* loss)
+{
+    const int q = blockIdx.x, ks = idx[q], side = ks & 1, N2 = 2 * NP, N4 = N2 * N2, t = threadIdx.x;
+    auto size_of = [&](C2 x) { const double a = fabs(x.x) + fabs(x.y); return a == a ? a : INFINITY; };
+    double g = 0.0, e = 0.0;
+    if (mc > 2) {
+        const int n1 = psize[side ? M - 2 : 1], n2 = mc == 4 ? psize[side ? M - 3 : 2] : 0;
+        auto in = [&](int r) { return r < NP ? r < n1 : r - NP < n2; };
+        const C2* m = G1 + (long)q * N4;
+        for (int i = t; i < N4; i += 256)
+            if (in(i % N2) && in(i / N2)) g = fmax(g, size_of(m[i]));
+    }
+    const C2 *A = cell_block(H, nullptr, nullptr, M, (long)NP * NP, ks / 2, side, 0, 0), *V = VS + (long)ks * N4;
+    for (int i = t; i < NP * NP; i += 256) e = fmax(e, size_of(A[i]));
+    for (int i = t; i < N4; i += 256) e = fmax(e, size_of(V[i]));
+    __shared__ double wg[4], we[4];
+    for (int o = 32; o; o >>= 1) {
+        g = fmax(g, __shfl_xor(g, o));
+        e = fmax(e, __shfl_xor(e, o));
+    }
+    if ((t & 63) == 0) {
+        wg[t >> 6] = g;
+        we[t >> 6] = e;
+    }
+    __syncthreads();
+    if (t == 0) {
+        for (int i = 1; i < 4; ++i) {
+            g = fmax(g, wg[i]);
+            e = fmax(e, we[i]);
+        }
+        e = fmax(e, fabs(z[2 * q]));
+        loss[q].mid = g * e;
+        loss[q].scale = e;
+    }
 }
 
 struct BigView {
@@ -1251,10 +1400,16 @@ void planes_big_leads(nt_ctx* c, const nt_params* prm, const TdbArgs& a, const P
                            mc > 2, g.He);
         return hipGetLastError();
     });
+    launch(c, NT_K_ELEM, 0, "cell loss", [&] {
+        hipLaunchKernelGGL(k_pl_cell_loss, dim3(Q), dim3(256), 0, s, h.M, NP, mc, v.psize, pH, g.VS, g.G1, g.idx,
+                           g.z, cv.loss);
+        return hipGetLastError();
+    });
     lead_sigma(c, N2, Q, bm<T>(R(g.He), N4, N2), bm<T>(R(g.VS), N4, N2, g.idx, 0, nk2), g.z, prm->convergence,
-               prm->max_iter, bw(W(g.G1), N4, N2), bw(W(g.S), N4, N2), cv.dst, cv.dit, ar, g.dec_off);
+               prm->max_iter, bw(W(g.G1), N4, N2), bw(W(g.S), N4, N2), cv.dst, cv.dit, &cv.loss->res,
+               sizeof(LeadLoss) / sizeof(double), ar, g.dec_off);
     launch(c, NT_K_ELEM, 0, "cell sigma", [&] {
-        hipLaunchKernelGGL(k_pl_cell_sigma, dim3(nblk(NN, 1024), Q), dim3(256), 0, s, NP, g.S, cv.sigma, cv.dgrow);
+        hipLaunchKernelGGL(k_pl_cell_sigma, dim3(nblk(NN, 1024), Q), dim3(256), 0, s, NP, g.S, cv.sigma);
         return hipGetLastError();
     });
 }
@@ -1393,7 +1548,11 @@ static void solve_left(nt_ctx* c, const nt_params* prm, const TdbArgs& a, int p0
     Arena la;
     const size_t oi = la.take(ni), oe = la.take(nd), ok = la.take(ni), of = la.take(ni), ol = la.take(nd),
                  orr = la.take(nd), os = la.take(ni), ot = la.take(ni), ow = la.take(nd);
-    ensure_left_buf(w, la.off);
+    if (w != c) {
+        w->regions = c->regions;
+        if (w->ws) reg_region(w, w->ws, w->ws_bytes);
+    }
+    ensure_left_buf(w, 2 * la.off);
     la.base = static_cast<char*>(w->left_buf);
     int *idx = la.ptr<int>(oi), *gk = la.ptr<int>(ok), *gf = la.ptr<int>(of);
     double* gE = la.ptr<double>(oe);
@@ -1410,11 +1569,6 @@ static void solve_left(nt_ctx* c, const nt_params* prm, const TdbArgs& a, int p0
     g.T_RL = la.ptr<double>(orr);
     g.status = la.ptr<int>(os);
     g.iters = la.ptr<int>(ot);
-    if (w != c) {
-        w->regions = c->regions;
-        if (w->ws) reg_region(w, w->ws, w->ws_bytes);
-    }
-    reg_region(w, w->left_buf, w->left_bytes);
     w->inv_panels = true;
     try {
         solve_tdb_dev(w, prm, g);
@@ -1442,6 +1596,65 @@ static void solve_left(nt_ctx* c, const nt_params* prm, const TdbArgs& a, int p0
     hipcheck(c, hipGetLastError(), "scatter");
 }
 
+// bytes the layers' self-energies of some of a chunk's points may take
+constexpr double PL_LEADS_BYTES = 512.0 * 1024 * 1024;
+
+// The leads of the m points with need == NEED_LEADS among a chunk's n, on the
+// layers.  Returns how many points are left to the layers since then.
+static int planes_redo_leads(nt_ctx* c, const nt_params* prm, const TdbArgs& a, const PlanDims& d, const PlanView& v,
+                             const BlocksIn& B, const ChunkView& cv, int NP, int p0, int n, int m, int* need, int* cnt, int had)
+{
+    hipStream_t s = c->stream;
+    Arena la;
+    int *idx = nullptr, *gk = nullptr, *st = nullptr, *it = nullptr;
+    double *gE = nullptr, *sig = nullptr, *es = nullptr;
+    size_t scr = 0;
+    auto carve = [&](int P) {
+        la.off = 0;
+        idx = la.ptr<int>(la.take(sizeof(int) * P));
+        gk = la.ptr<int>(la.take(sizeof(int) * P));
+        st = la.ptr<int>(la.take(sizeof(int) * 2 * P));
+        it = la.ptr<int>(la.take(sizeof(int) * 2 * P));
+        gE = la.ptr<double>(la.take(sizeof(double) * P));
+        sig = la.ptr<double>(la.take(sizeof(C2) * 2 * sigma_stride(a) * P));
+        es = la.ptr<double>(la.take(sizeof(C2) * 2 * sigma_stride(a) * P));
+        scr = la.off;
+        la.off += layers_sigma_scratch(a, P);
+        return la.off;
+    };
+    const double one = ((double)carve(65) - (double)carve(1)) / 64;
+    const int P = std::max(1.0, std::min<double>(m, PL_LEADS_BYTES / one));
+    carve(P);
+    ensure_left_buf(c, la.off);
+    la.base = static_cast<char*>(c->left_buf);
+    carve(P);
+    const size_t row = sizeof(C2) * NP * NP;
+    hipcheck(c, hipMemcpy2DAsync(cv.left, row, cv.sigma, 2 * row, row, n, hipMemcpyDeviceToDevice, s), "copy sigma");
+    for (int q = 0; q < m; q += P) {
+        const int k = std::min(P, m - q);
+        // (the points of earlier passes no longer need it)
+        hipLaunchKernelGGL(k_pl_gather, dim3(1), dim3(1024), 0, s, n, need, NEED_LEADS, k, a.E + p0,
+                           a.kidx ? a.kidx + p0 : nullptr, (const int*)nullptr, idx, gE, gk, (int*)nullptr,
+                           (const double*)nullptr, (double*)nullptr);
+        hipcheck(c, hipGetLastError(), "gather");
+        c->inv_panels = true;              // as on the layers before the planes
+        try {
+            layers_sigma(c, prm, a, k, gE, a.kidx ? gk : nullptr, sig, es, st, it, la, scr);
+        } catch (...) {
+            c->inv_panels = false;
+            throw;
+        }
+        c->inv_panels = false;
+        hipLaunchKernelGGL(k_pl_put_sigma, dim3(nblk((long)NP * NP, 8), 2 * k), dim3(256), 0, s, d, v, B, idx,
+                           a.kidx ? gk : nullptr, reinterpret_cast<const C2*>(sig), reinterpret_cast<const C2*>(es),
+                           sigma_stride(a), st, it, cv.sigma, cv.left, cv.dst, cv.dit, need, cnt);
+        hipcheck(c, hipGetLastError(), "put sigma");
+    }
+    hipcheck(c, hipMemcpyAsync(c->host_plan, cnt, sizeof(int), hipMemcpyDeviceToHost, s), "count D2H");
+    hipcheck(c, hipStreamSynchronize(s), "count sync");
+    return c->host_plan[0] - had;
+}
+
 bool planes_candidate(const nt_ctx* c, const nt_params* prm, const TdbArgs& a)
 {
     const nt_solve_extras& x = a.ex;
@@ -1455,8 +1668,9 @@ bool planes_candidate(const nt_ctx* c, const nt_params* prm, const TdbArgs& a)
 }
 
 // Solve a's points on their planes.  False: the blocks do not fall into planes
-// of at most 64 (nothing was written).  Points the planes are no good for (a
-// singular plane, growth) are solved by the block path before it returns.
+// of at most 96 (nothing was written).  Points the planes are no good for (a
+// singular or nearly singular plane) are solved by the block path before it
+// returns, leads whose decimation lost digits are decimated by it.
 bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
 {
     const bool wait = c->dec_check > 0;        // the host may wait for the device
@@ -1465,7 +1679,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     // the plan, the mask of points left to the block path, the counters
     Arena pa;
     plan_carve(pa, d);
-    const size_t o_need = pa.take(sizeof(int) * (size_t)a.npts), o_cnt = pa.take(sizeof(int) * 4);
+    const size_t o_need = pa.take(sizeof(int) * (size_t)a.npts), o_cnt = pa.take(sizeof(int) * CNT_N);
     const size_t plan_need = pa.off;
     size_t scratch_bytes = 0;
     char* scratch = static_cast<char*>(scratch_region(c->device, &scratch_bytes));
@@ -1486,7 +1700,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     int* cnt = pa.ptr<int>(o_cnt);
     if (c->ws_poison) poison_dev(c, pa.base, plan_need, s);
     zero_dev(c, v.h, (char*)v.level - (char*)v.h, s);
-    zero_dev(c, cnt, sizeof(int) * 4, s);
+    zero_dev(c, cnt, sizeof(int) * CNT_N, s);
     const BlocksIn B{reinterpret_cast<const C2*>(a.Haml), reinterpret_cast<const C2*>(a.Hamlv),
                      reinterpret_cast<const C2*>(a.Hamr), reinterpret_cast<const C2*>(a.Hamrv),
                      reinterpret_cast<const C2*>(a.Hamd), reinterpret_cast<const C2*>(a.Hamdv),
@@ -1509,7 +1723,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     check_range(c, a.iters, sizeof(int) * a.npts, "planes iters");
     const int nL = a.L + 2;
     // the large class where the host may wait, with workspace, and not at a
-    // fixed broadening (its decimation has no measure of the growth)
+    // fixed broadening (the electrons' eta = 1e-8 eV: only phonons were measured)
     const int ncls = wait && !a.noalloc && prm->eta_mode == NT_ETA_RELATIVE ? PL_NCLS : PL_MAXNT;
     launch(c, NT_K_ELEM, 0, "plane pattern", [&] {
         const unsigned gx = nblk((long)d.nmax * d.nmax, 1024);
@@ -1611,10 +1825,10 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         const int* kidx = a.kidx ? a.kidx + p0 : nullptr;
         const int* first = a.first_mask ? a.first_mask + p0 : nullptr;
         const DecPlArgs da{v.h, v.psize, pH, pU, pL, pV, a.E + p0, kidx, prm->eta, prm->eta0, prm->convergence,
-                           prm->eta_mode, prm->max_iter, cv.scratch, cv.sigma, cv.dst, cv.dit, cv.dgrow};
-        const SweepPlArgs sa{v.h, v.psize, pH, pU, pL, pM, a.E + p0, kidx, prm->eta, prm->eta0, prm->device_eta_factor,
-                             prm->eta_mode, need + p0, cv.sigma, cv.T, cv.sst, cv.keep, v.poff + a.adj_lo + 1, kept};
-        if (p0) zero_dev(c, cnt, sizeof(int) * 2, s);
+                           prm->eta_mode, prm->max_iter, cv.scratch, cv.sigma, cv.dst, cv.dit, cv.loss};
+        SweepPlArgs sa{v.h, v.psize, pH, pU, pL, pM, a.E + p0, kidx, prm->eta, prm->eta0, prm->device_eta_factor,
+                             prm->eta_mode, need + p0, cv.sigma, nullptr, cv.T, cv.grow, cv.sst, cv.keep, v.poff + a.adj_lo + 1, kept};
+        if (p0) zero_dev(c, cnt, sizeof(int) * CNT_STEPS, s);
         if (big) planes_big_leads(c, prm, a, v, h, bv, w, pH, pU, pL, pV, p0, n, cv);
         else launch(c, NT_K_PLANES, 0, "plane decimation", [&] {
             if (!wait || h.nt == 1) launch_decimate<1>(da, 2 * n, s);
@@ -1623,10 +1837,21 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
             if (!wait || h.nt == 4) launch_decimate<4>(da, 2 * n, s);
             return hipGetLastError();
         });
-        hipLaunchKernelGGL(k_pl_check, dim3(nblk(n)), dim3(256), 0, s, v.h, n, cv.dst, cv.dgrow, need + p0, cnt);
+        // leads that lost digits: once more on the layers, where the host may wait
+        // for their count and the call may allocate (else the whole point)
+        const int lossy = wait && !a.noalloc ? NEED_LEADS : NEED_LAYERS;
+        hipLaunchKernelGGL(k_pl_check, dim3(nblk(n)), dim3(256), 0, s, v.h, n, cv.dst, cv.loss, a.E + p0, prm->eta,
+                           prm->eta0, prm->eta_mode, adj ? PL_RESIDUAL_ADJ : PL_RESIDUAL, lossy, need + p0, cnt);
         hipcheck(c, hipGetLastError(), "plane check");
+        int n1 = 0;                        // points for the layers
         if (wait) {
-            hipcheck(c, hipMemcpyAsync(c->host_plan, cnt, sizeof(int), hipMemcpyDeviceToHost, s), "count D2H");
+            hipcheck(c, hipMemcpyAsync(c->host_plan, cnt, 3 * sizeof(int), hipMemcpyDeviceToHost, s), "count D2H");
+            hipcheck(c, hipStreamSynchronize(s), "count sync");
+            n1 = c->host_plan[CNT_LAYERS];
+            if (const int m = c->host_plan[CNT_LEADS]) {
+                n1 += planes_redo_leads(c, prm, a, d, v, B, cv, NP, p0, n, m, need + p0, cnt, n1);
+                sa.left = cv.left;
+            }
             hipcheck(c, hipEventRecord(c->chk[0], s), "event check");
         }
         const double m = 16.0 * h.nt;
@@ -1638,26 +1863,24 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
             if (big) launch_sweep<PL_BIGNT>(sa, 2 * n, s);
             return hipGetLastError();
         });
-        hipLaunchKernelGGL(k_pl_finish, dim3(nblk(n)), dim3(256), 0, s, n, cv.dst, cv.dit, cv.sst, cv.T, first,
-                           need + p0, cnt, a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr,
+        hipLaunchKernelGGL(k_pl_finish, dim3(nblk(n)), dim3(256), 0, s, n, cv.dst, cv.dit, cv.sst, cv.T, cv.loss,
+                           cv.grow, first, need + p0, cnt, a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr,
                            a.iters ? a.iters + p0 : nullptr);
         hipcheck(c, hipGetLastError(), "plane finish");
         if (adj) planes_adjoint(c, a, d, v, h, cv, pU, pL, pM, p0, n, hk, need + p0, kept, hi1);
         if (!wait) continue;
-        // the points for the layers are known while the sweep still runs:
-        // they are solved beside it, on a worker context
-        hipcheck(c, hipEventSynchronize(c->chk[0]), "event sync");
-        const int n1 = c->host_plan[0];
+        // the points for the layers are known: they are solved beside the sweep, on
+        // a worker context
         // (an adjoint solve of them adds to the same gradients: afterwards)
         const bool beside = !c->worker && !a.noalloc && !adj;
-        if (n1 && beside) solve_left(c, prm, a, p0, n, need + p0, 1, n1, true);
-        hipcheck(c, hipMemcpyAsync(c->host_plan, cnt + 1, 2 * sizeof(int), hipMemcpyDeviceToHost, s), "count D2H");
+        if (n1 && beside) solve_left(c, prm, a, p0, n, need + p0, NEED_LAYERS, n1, true);
+        hipcheck(c, hipMemcpyAsync(c->host_plan, cnt, CNT_N * sizeof(int), hipMemcpyDeviceToHost, s), "count D2H");
         hipcheck(c, hipStreamSynchronize(s), "count sync");
-        left += n1 + c->host_plan[0];
+        left += n1 + c->host_plan[CNT_AFTER_SWEEP];
         later[0] += beside ? 0 : n1;
-        later[1] += c->host_plan[0];
+        later[1] += c->host_plan[CNT_AFTER_SWEEP];
     }
-    const double steps = wait ? (double)c->host_plan[1] : 0.0;
+    const double steps = wait ? (double)c->host_plan[CNT_STEPS] : 0.0;
     // of a decimation step: the inverse of two planes and eight products of one
     if (c->prof && !big) c->flops_pending[NT_K_PLANES] += steps * 16 * 8 * (16.0 * h.nt) * (16.0 * h.nt) * (16.0 * h.nt);
     if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - left;
@@ -1679,7 +1902,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     } else {
         // (in c's own workspace, which the planes have no use for any more)
         for (int i = 0; i < 2; ++i)
-            if (later[i]) solve_left(c, prm, a, 0, a.npts, need, i + 1, later[i], false);
+            if (later[i]) solve_left(c, prm, a, 0, a.npts, need, i ? NEED_AFTER_SWEEP : NEED_LAYERS, later[i], false);
     }
     c->last_mean_iters = !wait ? -1.0 : left < a.npts ? steps / (2.0 * (a.npts - left)) : 0.0;
     return true;

@@ -225,11 +225,6 @@ __device__ __forceinline__ void blk_mul_rows(Blk<NT>& y, F A, const Blk<NT>& x, 
     }
 }
 
-// running |A|, |A^-1| maxima of a wave's inverses
-struct Grow {
-    double a = 0.0, g = 0.0;
-};
-
 __device__ __forceinline__ double read_lane(double v, int lane)
 {
     const long long b = __double_as_longlong(v);
@@ -269,15 +264,11 @@ struct InvLds {
 };
 
 template <int NT, class Out>
-__device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m, Grow& gr, Out out)
+__device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m, Out out)
 {
     constexpr int NP = 16 * NT, LD = NP + 1, RPL = (NP + 63) / 64, KM = RPL > 1 ? 255 : 127;
     const int lane = lane_new(), l15 = lane & 15, q = lane >> 4, w = wave_id();
     if (threadIdx.x < NP) s.cinv[threadIdx.x] = -1;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) gr.a = fmax(gr.a, fabs(m.re[t][r]) + fabs(m.im[t][r]));
     __syncthreads();
     C2* pb = work + 2 * 16 * LD + w * 256;
 #pragma unroll 1
@@ -505,10 +496,7 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            out(s.cinv[16 * t + 4 * r + q], oc, make_double2(m.re[t][r], m.im[t][r]));
-            gr.g = fmax(gr.g, fabs(m.re[t][r]) + fabs(m.im[t][r]));
-        }
+        for (int r = 0; r < 4; ++r) out(s.cinv[16 * t + 4 * r + q], oc, make_double2(m.re[t][r], m.im[t][r]));
     __syncthreads();
 }
 

@@ -1889,11 +1889,14 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     g.no_planes = true;
     g.scratch_reserve = reserve;
     if (!wait || (a.noalloc && left)) {
-        // every point whose need is set, masked inside the layers' kernels
+        // every point whose need is set, masked inside the layers' kernels; in FP64,
+        // as the mixed-precision kernels have no mask
+        nt_params p64 = *prm;
+        p64.precision = NT_PREC_FP64;
         g.mask = need;
         c->inv_panels = true;
         try {
-            solve_tdb_dev(c, prm, g);
+            solve_tdb_dev(c, &p64, g);
         } catch (const Fail&) {
             c->inv_panels = false;
             throw;

@@ -333,3 +333,34 @@ def test_planes_in_other_units(engine, T, planes_on, lead, dev):
         t = np.stack([r[k].cpu().numpy() for k in ("T_LR", "T_RL", "iters", "status")])
         ref = t if ref is None else ref
         assert np.array_equal(t, ref)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_some_points_left_without_waiting(engine, T, planes_on, prec):
+    """The allocation-free entry and the solve without host synchronisation with
+    some points left to the layers and some not (the ribbon's uncoupled sites at
+    E, and two energies beside them): the former by the layers' launches under a
+    mask, in FP64 whatever the precision, the latter keep what the planes gave."""
+    blk = lt.agnr_blocks(n_dimer=9, L=3, onsite_w=0.0, hop_noise=0.0)
+    E = np.array([0.7, 0.0, -1.3, 1e-14, 0.9, 0.31, 0.0, 1.1])
+    left = np.abs(E) < 0.1
+    d = engine.upload_blocks(blk)
+    par = {k: T.params("tb", eta=1e-9, convergence=1e-12, precision=k, max_iter=60) for k in ("fp64", prec)}
+    ref, used, _ = planes_launches(engine, lambda: engine.solve_tdb(d, E, par["fp64"]))
+    assert used > 0
+    engine.set_planes(False)
+    engine.set_inverse_panel(18, 16)
+    lay = engine.solve_tdb(d, E, par["fp64"])
+    engine.set_inverse_panel(18, 0)
+    engine.set_planes(True)
+    want = {k: np.where(left, lay[k].cpu().numpy(), ref[k].cpu().numpy()) for k in ("T_LR", "T_RL", "status", "iters")}
+    try:
+        for every, noalloc in ((4, True), (0, False), (0, True)):
+            print(f"left points {prec}: check every {every}, noalloc {noalloc}", flush=True)
+            engine.set_decimation_check(every)
+            r, used, _ = planes_launches(engine, lambda: engine.solve_tdb(d, E, par[prec], noalloc=noalloc))
+            assert used > 0
+            for k, v in want.items():
+                assert np.array_equal(r[k].cpu().numpy(), v, equal_nan=True), (every, noalloc, k, r[k], v)
+    finally:
+        engine.set_decimation_check(4)

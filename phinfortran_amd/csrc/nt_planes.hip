@@ -1525,6 +1525,15 @@ void launch_sweep(const SweepPlArgs& a, int items, hipStream_t s)
 
 }  // namespace
 
+namespace {
+// inverses by panels only while it lives, as on the layers before the planes
+struct PanelsOnly {
+    nt_ctx* c;
+    explicit PanelsOnly(nt_ctx* ctx) : c(ctx) { c->inv_panels = true; }
+    ~PanelsOnly() { c->inv_panels = false; }
+};
+}  // namespace
+
 // The n points of a's points [p0, p0 + P) with need == which, on the layers.
 // beside: on a worker context, from where c's stream stands at chk[0] (the
 // decimation's end) on, c's stream waiting for it; else on c's stream.
@@ -1569,15 +1578,13 @@ static void solve_left(nt_ctx* c, const nt_params* prm, const TdbArgs& a, int p0
     g.T_RL = la.ptr<double>(orr);
     g.status = la.ptr<int>(os);
     g.iters = la.ptr<int>(ot);
-    w->inv_panels = true;
     try {
+        const PanelsOnly panels(w);
         solve_tdb_dev(w, prm, g);
     } catch (const Fail&) {
-        w->inv_panels = false;
         if (w != c) c->err = w->err;
         throw;
     }
-    w->inv_panels = false;
     if (w != c) {
         hipcheck(c, hipEventRecord(w->join, s), "event join");
         hipcheck(c, hipStreamWaitEvent(c->stream, w->join, 0), "wait join");
@@ -1589,6 +1596,10 @@ static void solve_left(nt_ctx* c, const nt_params* prm, const TdbArgs& a, int p0
             w->launches[k] = 0;
             w->ms[k] = 0;
             w->flops[k] = 0;
+        }
+        for (int k = 0; k < 3; ++k) {
+            c->mixed_counts[k] += w->mixed_counts[k];
+            w->mixed_counts[k] = 0;
         }
     }
     hipLaunchKernelGGL(k_pl_scatter, dim3(nblk(n)), dim3(256), 0, c->stream, n, idx, g.T_LR, g.T_RL, g.status, g.iters,
@@ -1637,14 +1648,10 @@ static int planes_redo_leads(nt_ctx* c, const nt_params* prm, const TdbArgs& a, 
                            a.kidx ? a.kidx + p0 : nullptr, (const int*)nullptr, idx, gE, gk, (int*)nullptr,
                            (const double*)nullptr, (double*)nullptr);
         hipcheck(c, hipGetLastError(), "gather");
-        c->inv_panels = true;              // as on the layers before the planes
-        try {
+        {
+            const PanelsOnly panels(c);
             layers_sigma(c, prm, a, k, gE, a.kidx ? gk : nullptr, sig, es, st, it, la, scr);
-        } catch (...) {
-            c->inv_panels = false;
-            throw;
         }
-        c->inv_panels = false;
         hipLaunchKernelGGL(k_pl_put_sigma, dim3(nblk((long)NP * NP, 8), 2 * k), dim3(256), 0, s, d, v, B, idx,
                            a.kidx ? gk : nullptr, reinterpret_cast<const C2*>(sig), reinterpret_cast<const C2*>(es),
                            sigma_stride(a), st, it, cv.sigma, cv.left, cv.dst, cv.dit, need, cnt);
@@ -1883,7 +1890,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     const double steps = wait ? (double)c->host_plan[CNT_STEPS] : 0.0;
     // of a decimation step: the inverse of two planes and eight products of one
     if (c->prof && !big) c->flops_pending[NT_K_PLANES] += steps * 16 * 8 * (16.0 * h.nt) * (16.0 * h.nt) * (16.0 * h.nt);
-    if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - left;
+    if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - (a.noalloc ? 0 : left);      // (the layers count theirs)
     TdbArgs g = a;
     g.siblings.clear();
     g.no_planes = true;
@@ -1894,14 +1901,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         nt_params p64 = *prm;
         p64.precision = NT_PREC_FP64;
         g.mask = need;
-        c->inv_panels = true;
-        try {
-            solve_tdb_dev(c, &p64, g);
-        } catch (const Fail&) {
-            c->inv_panels = false;
-            throw;
-        }
-        c->inv_panels = false;
+        const PanelsOnly panels(c);
+        solve_tdb_dev(c, &p64, g);
     } else {
         // (in c's own workspace, which the planes have no use for any more)
         for (int i = 0; i < 2; ++i)

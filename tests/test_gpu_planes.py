@@ -364,3 +364,17 @@ def test_some_points_left_without_waiting(engine, T, planes_on, prec):
                 assert np.array_equal(r[k].cpu().numpy(), v, equal_nan=True), (every, noalloc, k, r[k], v)
     finally:
         engine.set_decimation_check(4)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_mixed_counts_all_points(engine, T, planes_on, noalloc):
+    """every point of a mixed-precision call is counted in that call, those
+    solved on the layers by a worker context too (the energy of the uncoupled
+    sites of a lead's plane, without broadening)"""
+    d = engine.upload_blocks(plane_blocks((30, 31, 30), (30, 30), 2, 7, flat_lead=0.3))
+    E = np.array([0.1, 0.3, 0.5])
+    p = T.params("tb", eta=0.0, convergence=1e-12, precision="mixed", max_iter=60)
+    for _ in range(2):
+        engine.profile_reset()
+        _, used, _ = planes_launches(engine, lambda: engine.solve_tdb(d, E, p, noalloc=noalloc))
+        assert used > 0 and engine.mixed_counts()[0] == E.size

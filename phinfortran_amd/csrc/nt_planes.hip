@@ -63,12 +63,16 @@ constexpr double PL_RESIDUAL = 1.0e-6, PL_RESIDUAL_ADJ = 1.0e-7;
 constexpr double PL_RESIDUAL_ETA = 1.0;
 // Planes inside a lead cell and of the device are eliminated with pivots from
 // one plane only, and a plane may be nearly singular at E where its layer is
-// not.  With kappa = |G|max scale of the eliminated planes, T then is off by
-// 1e-16 to 5e-16 kappa of itself: layers of 13 + 14 + 13 degrees of freedom,
-// the middle ones uncoupled sites at E, eta = 1e-8: kappa 3e7, error 3e-8 (on
-// layers 3e-11), at kappa 2e5 3e-10.  Where T < 1 the error counts less, down
-// to T = 0.01.  The film reaches 4e4, the wire 2e5 (one point of 3000 beyond
+// not.  With kappa = |G|max scale of the eliminated planes, G between the leads
+// then is off by 1e-16 to 5e-16 kappa (where all layers have such planes at one
+// energy up to ten times that): layers of 13 + 14 + 13 degrees of freedom,
+// the middle ones uncoupled sites at E, eta = 1e-8: kappa 3e7, error of T 3e-8
+// (on layers 3e-11), at kappa 2e5 3e-10.  T changes by 2 sqrt(T) times as much,
+// and by no less than its square: what is bounded is kappa sqrt(T), with T from
+// this floor (kappa <= 1e9: 1e-13) to 1, in a gradient, which is of first order
+// in G, from 0.01.  The film reaches 4e4, the wire 2e5 (one point of 3000 beyond
 // 1e5, at T = 0.26), the ribbon 2e6 in its gap.
+constexpr double PL_T_FLOOR = 1.0e-8, PL_T_FLOOR_ADJ = 0.01;
 constexpr double PL_KAPPA = 1.0e5;
 
 // need[p]: 0 solved on the planes, else why it is not (yet)
@@ -970,7 +974,7 @@ __global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
     }
 }
 
-// NEED_LAYERS: plan refused, a singular plane of a lead; lossy: what a point
+// NEED_LAYERS: plan refused, a singular or nearly singular plane of a lead; lossy: what a point
 // needs whose leads lost digits or left the finite numbers
 __global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const LeadLoss* loss, const double* E, double eta,
                            double eta0, int mode, double res_max, int lossy, int* need,
@@ -985,9 +989,10 @@ __global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const LeadLo
         for (int i = 0; i < 2; ++i) {
             const int d = dst[2 * p + i];
             const LeadLoss l = loss[2 * p + i];
-            bad = bad || (d != 0 && d != -1 && d != NT_ERR_NOT_CONVERGED);
-            lost = lost || d == -1 || (d == 0 && !(l.res <= fmin(res_max, PL_RESIDUAL_ETA * fabs(et) / l.scale) &&
-                                        l.mid <= PL_KAPPA));
+            // (the sweep goes through the planes inside the cell as well)
+            bad = bad || (d != 0 && d != -1 && d != NT_ERR_NOT_CONVERGED) || (d == 0 && l.mid > PL_KAPPA);
+            lost = lost || d == -1 ||
+                   (d == 0 && !(l.res <= fmin(res_max, PL_RESIDUAL_ETA * fabs(et) / l.scale) && l.mid <= PL_KAPPA));
         }
         why = bad ? NEED_LAYERS : lost ? lossy : 0;
     }
@@ -1038,8 +1043,8 @@ __global__ void k_pl_put_sigma(PlanDims d, PlanView v, BlocksIn B, const int* id
 // or nearly singular plane in the sweep sets need[p] too; count[CNT_STEPS] sums
 // the decimation steps.
 __global__ void k_pl_finish(int P, const int* dst, const int* dit, const int* sst, const double* T,
-                            const LeadLoss* loss, const double* grow, const int* first_mask, int* need, int* count,
-                            double* T_LR, double* T_RL, int* status, int* iters)
+                            const LeadLoss* loss, const double* grow, double T_floor, const int* first_mask, int* need,
+                            int* count, double* T_LR, double* T_RL, int* status, int* iters)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P || need[p]) return;
@@ -1049,7 +1054,7 @@ __global__ void k_pl_finish(int P, const int* dst, const int* dit, const int* ss
     if (none) tl = tr = __longlong_as_double(0x7ff8000000000000LL);
     const double kappa = fmax(grow[2 * p], grow[2 * p + 1]) * fmax(loss[2 * p].scale, loss[2 * p + 1].scale);
     if (!none && (sst[2 * p] || sst[2 * p + 1] || tl != tl || tr != tr ||
-        !(kappa * fmin(fmax(fmax(tl, tr), 0.01), 1.0) <= PL_KAPPA))) {
+        !(kappa * sqrt(fmin(fmax(fmax(tl, tr), T_floor), 1.0)) <= PL_KAPPA))) {
         need[p] = NEED_AFTER_SWEEP;
         atomicAdd(count + CNT_AFTER_SWEEP, 1);
         return;
@@ -1871,7 +1876,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
             return hipGetLastError();
         });
         hipLaunchKernelGGL(k_pl_finish, dim3(nblk(n)), dim3(256), 0, s, n, cv.dst, cv.dit, cv.sst, cv.T, cv.loss,
-                           cv.grow, first, need + p0, cnt, a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr,
+                           cv.grow, adj ? PL_T_FLOOR_ADJ : PL_T_FLOOR, first, need + p0, cnt, a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr,
                            a.iters ? a.iters + p0 : nullptr);
         hipcheck(c, hipGetLastError(), "plane finish");
         if (adj) planes_adjoint(c, a, d, v, h, cv, pU, pL, pM, p0, n, hk, need + p0, kept, hi1);

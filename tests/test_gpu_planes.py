@@ -293,7 +293,8 @@ def test_lossy_leads_come_from_the_layers(engine, T, planes_on, seed, nw, at, re
 
 @pytest.mark.parametrize("lead,dev,flat_lead,flat_dev,L", [
     ((20, 20), (13, 14, 13), None, 0.3, 3), ((20, 20), (13, 14, 13), None, 0.3, 1),
-    ((13, 14, 13), (20, 20), 0.3, None, 2), ((13, 14, 13, 12), (20, 20), 0.3, None, 2),
+    ((30, 31, 30), (30, 30), 0.3, None, 2), ((30, 31, 30, 29), (30, 30), 0.3, None, 2),
+    ((30, 30), (30, 31, 30), None, 0.3, 2),
     ((66, 65), (65, 70, 65), None, 0.3, 1), ((66, 70, 66), (66, 65), 0.3, None, 1),
     ((66, 70, 66, 65), (66, 65), 0.3, None, 1)])
 def test_nearly_singular_planes(engine, T, planes_on, lead, dev, flat_lead, flat_dev, L):

@@ -637,7 +637,10 @@ int nt_set_decimation_check(nt_ctx* ctx, int every);
  * (every = n > 0) or for about every sqrt(L - lo)-th layer (every < 0); the
  * others are recomputed from the nearest kept layer during the backward pass
  * by the same launches as the forward sweep (same values, one more
- * left-to-right pass over the recomputed layers).  No reference counterpart
+ * left-to-right pass over the recomputed layers).  On planes (nt_set_planes)
+ * the kept blocks are those of the planes, a fraction of the layers', and always
+ * all of them: this setting and nt_adjoint_bytes_per_point are the layers'.
+ * No reference counterpart
  * (the reference has no derivatives). */
 int nt_set_adjoint_checkpoint(nt_ctx* ctx, int every);
 /* Device bytes per (omega,k) point that the adjoint solve's stored blocks take

@@ -1147,6 +1147,13 @@ void ensure_plan_buf(nt_ctx* c, size_t bytes)
     reg_region(c, c->plan_buf, bytes);
 }
 
+double free_bytes(nt_ctx* c)
+{
+    size_t free_b = 0, total_b = 0;
+    hipcheck(c, hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    return (double)free_b;
+}
+
 // gathered inputs and results of the points left to the layers
 void ensure_left_buf(nt_ctx* w, size_t bytes)
 {
@@ -1357,7 +1364,9 @@ BigView big_carve(Arena& a, int P, int nk, int NP)
     return v;
 }
 
-// bytes a chunk of points may take
+// bytes a chunk of points may take (with the batch limit of the context, its
+// workspace cap and the free memory); where the host does not know the planes,
+// the packed blocks included
 constexpr double PL_CHUNK_BYTES = 6.0 * 1024 * 1024 * 1024;
 constexpr double PL_ADJ_BYTES = 24.0 * 1024 * 1024 * 1024;
 constexpr int PL_MAX_ITER = 20000;      // decimation steps inside one kernel
@@ -1639,7 +1648,9 @@ static int planes_redo_leads(nt_ctx* c, const nt_params* prm, const TdbArgs& a, 
         return la.off;
     };
     const double one = ((double)carve(65) - (double)carve(1)) / 64;
-    const int P = std::max(1.0, std::min<double>(m, PL_LEADS_BYTES / one));
+    int P = std::max(1.0, std::min<double>({(double)m, (double)c->batch_limit, PL_LEADS_BYTES / one}));
+    if (carve(P) > c->left_bytes)          // no further than the memory reaches
+        P = std::max(1.0, std::min<double>(P, 0.8 * (free_bytes(c) + (double)c->left_bytes) / one));
     carve(P);
     ensure_left_buf(c, la.off);
     la.base = static_cast<char*>(c->left_buf);
@@ -1806,13 +1817,26 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     const double per_pt = (double)one.off / 64;
     double room = adj ? PL_ADJ_BYTES : PL_CHUNK_BYTES;
     if (a.noalloc) room = (double)scratch_bytes - reserve - fixed - 65536.0;
-    else if (c->ws_cap) room = std::min(room, (double)c->ws_cap - fixed);
-    int P = std::min((double)a.npts, room / per_pt);
+    else if (!wait) room -= fixed;         // (the bound of blocks whose planes the host does not know)
+    if (!a.noalloc && c->ws_cap) room = std::min(room, (double)c->ws_cap - fixed);
+    int P = std::min({(double)a.npts, (double)c->batch_limit, room / per_pt});
     if (P < 1) {
-        if (a.noalloc || !wait) return false;
+        if (a.noalloc || !wait || c->ws_cap) return false;
         P = 1;
     }
     carve(w, P);
+    if (!a.noalloc && w.off > c->ws_bytes) {
+        // the workspace has to grow: no further than the memory reaches (ensure_ws
+        // adds an eighth)
+        const double have = 8.0 / 9.0 * (free_bytes(c) + (double)c->ws_bytes);
+        if ((double)w.off > have) {
+            const int q = std::min((double)P, (have - fixed) / per_pt) - 1;
+            if (q < 1) return false;
+            P = q;
+            w.off = fixed;
+            carve(w, P);
+        }
+    }
     if (a.noalloc) {
         if (w.off > scratch_bytes - reserve) return false;
         if (c->ws_poison) poison_dev(c, scratch, w.off, s);

@@ -379,3 +379,50 @@ def test_mixed_counts_all_points(engine, T, planes_on, noalloc):
         engine.profile_reset()
         _, used, _ = planes_launches(engine, lambda: engine.solve_tdb(d, E, p, noalloc=noalloc))
         assert used > 0 and engine.mixed_counts()[0] == E.size
+
+
+@pytest.mark.parametrize("limit", [1, 8, 21])
+def test_batch_limit_holds_on_planes(engine, T, planes_on, limit):
+    """at most that many points per chunk, a decimation and a sweep each"""
+    p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13)
+    blk = plane_blocks((20, 33), (33, 20), 3, 9)
+    E = np.linspace(0.05, 0.9, 21)
+    ref = engine.solve_tdb(engine.upload_blocks(blk), E, p)
+    eng = T.Engine(0, batch_limit=limit)
+    try:
+        d = eng.upload_blocks(blk)
+        r, used, _ = planes_launches(eng, lambda: eng.solve_tdb(d, E, p))
+        assert used == 2 * -(-E.size // limit)
+        for k in ("T_LR", "T_RL", "status", "iters"):
+            assert np.array_equal(ref[k].cpu().numpy(), r[k].cpu().numpy()), k
+    finally:
+        eng.close()
+
+
+def test_no_check_reserves_no_more_than_its_budget(engine, T, planes_on):
+    """Without host waits the planes' blocks are reserved by their bound, the
+    largest class for every plane and k-point: where that takes gigabytes (here
+    9 of them for 130 MB of blocks) the layers solve the call."""
+    import torch
+    blk = plane_blocks((16, 16), (16, 16), 30, 5)
+    nk = 256
+    E = np.full(nk, 0.4)
+    kidx = np.arange(nk, dtype=np.int32)
+    p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13, max_iter=32)
+    eng = T.Engine(0, batch_limit=64)
+    try:
+        d = eng.upload_blocks([blk] * nk)
+        ref = eng.solve_tdb(d, E, p, kidx=kidx)
+        eng.close()
+        eng = T.Engine(0, batch_limit=64)
+        eng.set_decimation_check(0)
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        r = eng.solve_tdb(d, E, p, kidx=kidx)
+        torch.cuda.synchronize()
+        took = before - torch.cuda.mem_get_info()[0]
+        print(f"took {took / 2 ** 30:.2f} GiB", flush=True)
+        assert took < 6 * 2 ** 30
+        assert np.abs(r["T_LR"].cpu().numpy() - ref["T_LR"].cpu().numpy()).max() < 1e-8
+    finally:
+        eng.close()

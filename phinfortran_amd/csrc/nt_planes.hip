@@ -1369,6 +1369,7 @@ BigView big_carve(Arena& a, int P, int nk, int NP)
 // the packed blocks included
 constexpr double PL_CHUNK_BYTES = 6.0 * 1024 * 1024 * 1024;
 constexpr double PL_ADJ_BYTES = 24.0 * 1024 * 1024 * 1024;
+constexpr int PL_MAX_GRID_Y = 65535;    // a launch's second and third dimensions
 constexpr int PL_MAX_ITER = 20000;      // decimation steps inside one kernel
 
 // self-energies of a chunk's points on leads of large planes
@@ -1435,7 +1436,7 @@ void launch_adjoint(const AdjPlArgs& a, int n, hipStream_t s)
 }
 
 // Gradients of one chunk's points, added to a's dHd and dHdv.
-void planes_adjoint(nt_ctx* c, const TdbArgs& a, const PlanDims& d, const PlanView& v, const PlanHdr& h,
+void planes_adjoint(nt_ctx* c, const TdbArgs& a, const PlanView& v, const PlanHdr& h,
                     const ChunkView& cv, const C2* pU, const C2* pL, const unsigned long long* pM, int p0, int n, const std::vector<int>& hk,
                     const int* need, long kept, int hi1)
 {
@@ -1523,7 +1524,6 @@ void planes_adjoint(nt_ctx* c, const TdbArgs& a, const PlanDims& d, const PlanVi
                     product(1 + i, p, np, to, from, layers, S);
                 }, 2);
     }
-    (void)d;
 }
 
 template <int NT>
@@ -1648,7 +1648,7 @@ static int planes_redo_leads(nt_ctx* c, const nt_params* prm, const TdbArgs& a, 
         return la.off;
     };
     const double one = ((double)carve(65) - (double)carve(1)) / 64;
-    int P = std::max(1.0, std::min<double>({(double)m, (double)c->batch_limit, PL_LEADS_BYTES / one}));
+    int P = std::max(1.0, std::min<double>({(double)m, (double)c->batch_limit, PL_LEADS_BYTES / one, PL_MAX_GRID_Y / 2}));
     if (carve(P) > c->left_bytes)          // no further than the memory reaches
         P = std::max(1.0, std::min<double>(P, 0.8 * (free_bytes(c) + (double)c->left_bytes) / one));
     carve(P);
@@ -1687,7 +1687,7 @@ bool planes_candidate(const nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     // (an adjoint solve needs the plan's sizes on the host)
     return c->planes && !a.no_planes && !a.mask && !(a.adj_w && c->dec_check == 0) && !a.probe && !extras &&
            !(prm->circular && prm->n_bloch_x * prm->n_bloch_y > 1) && c->one_sweep && !c->gemm_m3 &&
-           prm->max_iter <= PL_MAX_ITER && a.nk <= 65535 && 2 * a.L + 5 <= 65535;
+           prm->max_iter <= PL_MAX_ITER && a.nk <= PL_MAX_GRID_Y && 2 * a.L + 5 <= PL_MAX_GRID_Y;
 }
 
 // Solve a's points on their planes.  False: the blocks do not fall into planes
@@ -1745,9 +1745,10 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     check_range(c, a.status, sizeof(int) * a.npts, "planes status");
     check_range(c, a.iters, sizeof(int) * a.npts, "planes iters");
     const int nL = a.L + 2;
-    // the large class where the host may wait, with workspace, and not at a
+    // the large class where the host may wait, with workspace, with a launch's
+    // second dimension for the leads of all k-points, and not at a
     // fixed broadening (the electrons' eta = 1e-8 eV: only phonons were measured)
-    const int ncls = wait && !a.noalloc && prm->eta_mode == NT_ETA_RELATIVE ? PL_NCLS : PL_MAXNT;
+    const int ncls = wait && !a.noalloc && 2L * a.nk <= PL_MAX_GRID_Y && prm->eta_mode == NT_ETA_RELATIVE ? PL_NCLS : PL_MAXNT;
     launch(c, NT_K_ELEM, 0, "plane pattern", [&] {
         const unsigned gx = nblk((long)d.nmax * d.nmax, 1024);
         // the first k-point's pattern alone refuses dense blocks (49 k-points
@@ -1903,7 +1904,7 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
                            cv.grow, adj ? PL_T_FLOOR_ADJ : PL_T_FLOOR, first, need + p0, cnt, a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr,
                            a.iters ? a.iters + p0 : nullptr);
         hipcheck(c, hipGetLastError(), "plane finish");
-        if (adj) planes_adjoint(c, a, d, v, h, cv, pU, pL, pM, p0, n, hk, need + p0, kept, hi1);
+        if (adj) planes_adjoint(c, a, v, h, cv, pU, pL, pM, p0, n, hk, need + p0, kept, hi1);
         if (!wait) continue;
         // the points for the layers are known: they are solved beside the sweep, on
         // a worker context

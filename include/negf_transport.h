@@ -592,7 +592,11 @@ int nt_hk_assemble_orb_dev(nt_ctx* ctx, int nk, const double* kcart, int nseg, c
  * times every supported width on `batch` n x n matrices and keeps the fastest
  * for this context (precision NT_PREC_FP64: complex double, NT_PREC_MIXED:
  * complex float); best_nb / best_ms may be NULL.  nt_set_inverse_panel sets a
- * width directly (0 restores the default).  No reference counterpart. */
+ * width directly (0 restores the default).  Complex double up to n = 128 is
+ * inverted in the registers of a workgroup, faster than by any width: there
+ * the autotuner's width and time are those of the panels, which then serve only
+ * points that a solve on planes leaves over (nt_set_planes), while a width set
+ * directly holds for every inverse.  No reference counterpart. */
 int nt_autotune_inverse(nt_ctx* ctx, int n, int batch, int precision, int* best_nb, double* best_ms);
 int nt_set_inverse_panel(nt_ctx* ctx, int n, int precision, int nb);
 /* Output tile of the batched complex GEMM: 64x64 per 256-thread workgroup

@@ -2091,10 +2091,14 @@ void tune_inverse(nt_ctx* c, int n, int batch, int* best_nb, double* best_ms)
     hipcheck(c, hipEventCreate(&e1), "event");
     double best = 1e300;
     int bnb = widths[0];
-    const bool prof = c->prof;
-    c->prof = false;
-    c->tuning = true;
+    struct Tuning {
+        nt_ctx* c;
+        bool prof;
+        explicit Tuning(nt_ctx* ctx) : c(ctx), prof(ctx->prof) { c->prof = false, c->tuning = true; }
+        ~Tuning() { c->prof = prof, c->tuning = false; }
+    };
     for (int i = 0; i < k; ++i) {
+        const Tuning on(c);
         c->inv_nb[{(int)sizeof(T), n}] = widths[i];
         auto run = [&] {
             inverse<T>(c, n, bw(W.as<T>(), nn, n), bm<T>(A.as<T>(), nn, n), z.as<T>(), bw(X.as<T>(), nn, n),
@@ -2113,10 +2117,8 @@ void tune_inverse(nt_ctx* c, int n, int batch, int* best_nb, double* best_ms)
             bnb = widths[i];
         }
     }
-    c->prof = prof;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    c->tuning = false;
     c->inv_nb[{(int)sizeof(T), n}] = bnb;
     if (sizeof(T) == 8) c->inv_tuned.insert(n);
     if (best_nb) *best_nb = bnb;

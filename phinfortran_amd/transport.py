@@ -579,8 +579,10 @@ class Engine:
 
     # ------------------------------------------------------------ tuning
     def autotune_inverse(self, n: int, batch: int, precision: str = "fp64"):
-        """Time every inverse panel width for n x n batches; keeps the fastest.
-        Returns (panel width, ms per batched launch)."""
+        """Time every inverse panel width for n x n batches; keeps the fastest
+        (for FP64 up to n = 128, which is inverted in registers, for the points
+        that a solve on planes leaves over only).  Returns (panel width, ms per
+        batched launch)."""
         prec = {"fp64": N.NT_PREC_FP64, "mixed": N.NT_PREC_MIXED}[precision]
         nb, ms = C.c_int(), C.c_double()
         self._check(self._L.nt_autotune_inverse(self.ctx, int(n), int(batch), prec, C.byref(nb), C.byref(ms)),
@@ -644,8 +646,8 @@ class Engine:
         self._check(self._L.nt_set_point_split(self.ctx, int(n)), "nt_set_point_split")
 
     def set_planes(self, on: bool):
-        """FP64 batched solves on the planes of the principal layers (default)
-        or always on whole layers."""
+        """Batched and adjoint solves on the planes of the principal layers, in
+        FP64 for both precisions (default), or always on whole layers."""
         self._check(self._L.nt_set_planes(self.ctx, int(bool(on))), "nt_set_planes")
 
     def set_workspace_poison(self, on: bool):

@@ -28,3 +28,13 @@ def engine():
     eng = transport.Engine(0)
     yield eng
     eng.close()
+
+
+@pytest.fixture(params=[True, False], ids=["planes", "layers"])
+def both_paths(engine, request):
+    """Run a test twice: with batched solves on the planes of the principal
+    layers where the blocks have them (the default), and on whole layers, whose
+    mixed-precision, split and shared-lead paths the planes would bypass."""
+    engine.set_planes(request.param)
+    yield request.param
+    engine.set_planes(True)

@@ -10,7 +10,7 @@ import oracle as O
 from adjoint_ref import T_and_grad
 from phinfortran_amd import lattice as lt
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_paths")]
 
 
 def oparams(p):

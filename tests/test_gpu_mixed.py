@@ -10,7 +10,7 @@ import pytest
 
 from phinfortran_amd import lattice as lt
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_paths")]
 
 REL = 1e-6
 

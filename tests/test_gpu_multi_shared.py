@@ -8,7 +8,7 @@ import pytest
 import oracle as O
 from phinfortran_amd import lattice as lt
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_paths")]
 
 
 def test_shared_leads_equal_single_solves(engine):

@@ -74,6 +74,8 @@ def main():
                     help="before timing, run one device-to-device copy of this many MiB (HBM-counter calibration "
                          "under rocprofv3 --pmc)")
     ap.add_argument("--no-autotune", dest="autotune", action="store_false")
+    ap.add_argument("--no-planes", dest="planes", action="store_false",
+                    help="solve on the principal layers instead of the planes that their zeros divide them into")
     ap.add_argument("--point-split", type=int, default=2,
                     help="parts a solve of many points runs as, side by side on worker streams (1 = one stream)")
     ap.add_argument("--serial-sweeps", action="store_true",
@@ -134,6 +136,7 @@ def main():
     E = torch.as_tensor(omega ** 2, dtype=torch.float64, device=dev)
 
     eng = T.Engine(0, batch_limit=args.points)
+    eng.set_planes(args.planes)
     eng.set_point_split(1 if args.serial_sweeps else args.point_split)
     if args.serial_sweeps:
         eng.set_overlap(False)
@@ -845,7 +848,8 @@ def main():
                                             f"(nt_set_point_split) and launches share the GPU"},
                      "inverse_isolated": None if not iso64["inverse"]["launches"] else {"avg_launch_ms": iso64["inverse"]["ms"] / max(1, iso64["inverse"]["launches"]),
                                           "tflops": iso64["inverse"]["flops"] / max(1e-9, iso64["inverse"]["ms"] * 1e-3) / 1e12}},
-        "precision_compare": {"fp64_solves_per_s": v64, "mixed_solves_per_s": vmx,
+        "precision_compare": {"mixed_ran_in": "FP64 on planes" if planes_mixed else "FP32 with FP64 refinement",
+                              "fp64_solves_per_s": v64, "mixed_solves_per_s": vmx,
                               "mixed_speedup": vmx / v64, "mixed_max_rel_dT": rel_err,
                               "criterion": "max |T_mixed - T_fp64| / T_fp64 over T > 1e-3 max T, all timed steps",
                               "refinement": mixed_counts,

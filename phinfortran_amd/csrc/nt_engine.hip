@@ -1557,8 +1557,9 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         std::vector<const TdbArgs*> all{&a};
         all.insert(all.end(), a.siblings.begin(), a.siblings.end());
         double sum = 0.0;
+        PlanesLeads leads;
         for (const TdbArgs* d : all) {
-            if (!planes_solve(c, prm, *d)) rest.push_back(d);
+            if (!planes_solve(c, prm, *d, all.size() > 1 ? &leads : nullptr)) rest.push_back(d);
             else sum += c->last_mean_iters;
         }
         if (rest.empty()) {
@@ -2253,6 +2254,7 @@ int nt_destroy(nt_ctx* c)
     for (nt_ctx* s : c->subs) nt_destroy(s);
     if (c->plan_buf) (void)hipFree(c->plan_buf);
     if (c->left_buf) (void)hipFree(c->left_buf);
+    if (c->leads_buf) (void)hipFree(c->leads_buf);
     if (c->host_plan) (void)hipHostFree(c->host_plan);
     if (c->host_flag) (void)hipHostFree(c->host_flag);
     if (c->own) (void)hipStreamDestroy(c->own);

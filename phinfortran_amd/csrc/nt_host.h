@@ -100,6 +100,9 @@ struct nt_ctx {
     // its points left to the layers (gathered inputs and results)
     void* left_buf = nullptr;
     size_t left_bytes = 0;
+    // self-energies on planes that devices with the same leads share in a call
+    void* leads_buf = nullptr;
+    size_t leads_bytes = 0;
     bool worker = false;           // a worker context of another one
     // uneven-device calls: worker contexts (own stream and workspace, one host
     // thread each) that solve groups of devices concurrently

@@ -78,7 +78,7 @@ constexpr double PL_KAPPA = 1.0e5;
 // need[p]: 0 solved on the planes, else why it is not (yet)
 enum { NEED_LAYERS = 1, NEED_AFTER_SWEEP = 2, NEED_LEADS = 3 };
 // counters of a solve (device ints; the first three of a chunk)
-enum { CNT_LAYERS = 0, CNT_AFTER_SWEEP = 1, CNT_LEADS = 2, CNT_STEPS = 3, CNT_N = 4 };
+enum { CNT_LAYERS = 0, CNT_AFTER_SWEEP = 1, CNT_LEADS = 2, CNT_STEPS = 3, CNT_SAME = 4, CNT_N = 5 };
 
 // ------------------------------------------------------------------ the plan
 // Device arrays of the plan (ints), carved from one buffer.
@@ -1000,6 +1000,26 @@ __global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const LeadLo
     if (why) atomicAdd(count + (why == NEED_LEADS ? CNT_LEADS : CNT_LAYERS), 1);
 }
 
+// *same stays 1 where the planes of both lead cells hold the same degrees of
+// freedom in the same places as the stored ones (sizes, then PL_PERM places of
+// every plane); store: written instead.  One workgroup per plane.
+__global__ void k_pl_lead_planes(const PlanHdr* h, const int* psize, const int* perm, int* stored, int store, int* same)
+{
+    const int q = blockIdx.x, pl = q < h->m0 ? q : h->M - h->m1 + (q - h->m0), n = psize[pl];
+    int* o = stored + (long)q * (PL_PERM + 1);
+    for (int i = threadIdx.x; i <= n; i += blockDim.x) {
+        const int v = i ? perm[(long)pl * PL_PERM + i - 1] : n;
+        if (store) o[i] = v;
+        else if (o[i] != v) *same = 0;
+    }
+}
+
+__global__ void k_pl_count(int n, const int* need, int* count)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < n && need[p] == NEED_LAYERS) atomicAdd(count + CNT_LAYERS, 1);
+}
+
 // Self-energies of the layers (layers_sigma) of the points idx onto the planes
 // that face the leads, with their statuses and step counts; a point with a
 // singular matrix on the layers is left to them.  The layers' sweep begins
@@ -1198,6 +1218,27 @@ ChunkView chunk_carve(Arena& a, int P, int NN)
     return v;
 }
 
+// what devices with the same leads share (PlanesLeads): per point the leads'
+// self-energies, digits lost, statuses, step counts and need, and the lead
+// cells' planes
+struct LeadsView {
+    C2 *sigma, *left;
+    LeadLoss* loss;
+    int *dst, *dit, *need, *planes;
+};
+LeadsView leads_carve(Arena& a, int npts, int NN, int planes)
+{
+    LeadsView v;
+    v.sigma = a.ptr<C2>(a.take(sizeof(C2) * 2 * NN * (size_t)npts));
+    v.left = a.ptr<C2>(a.take(sizeof(C2) * NN * (size_t)npts));
+    v.loss = a.ptr<LeadLoss>(a.take(sizeof(LeadLoss) * 2 * (size_t)npts));
+    v.dst = a.ptr<int>(a.take(sizeof(int) * 2 * (size_t)npts));
+    v.dit = a.ptr<int>(a.take(sizeof(int) * 2 * (size_t)npts));
+    v.need = a.ptr<int>(a.take(sizeof(int) * (size_t)npts));
+    v.planes = a.ptr<int>(a.take(sizeof(int) * (PL_PERM + 1) * (size_t)planes));
+    return v;
+}
+
 // ---------------------------------------- leads whose planes hold more than 64
 // The two planes of a lead cell, as one matrix, no longer fit the decimation
 // kernel's registers: their cell (the planes between eliminated by one batched
@@ -1369,6 +1410,7 @@ BigView big_carve(Arena& a, int P, int nk, int NP)
 // the packed blocks included
 constexpr double PL_CHUNK_BYTES = 6.0 * 1024 * 1024 * 1024;
 constexpr double PL_ADJ_BYTES = 24.0 * 1024 * 1024 * 1024;
+constexpr double PL_SHARE_BYTES = 1.0 * 1024 * 1024 * 1024;      // self-energies kept for devices with the same leads
 constexpr int PL_MAX_GRID_Y = 65535;    // a launch's second and third dimensions
 constexpr int PL_MAX_ITER = 20000;      // decimation steps inside one kernel
 
@@ -1694,7 +1736,7 @@ bool planes_candidate(const nt_ctx* c, const nt_params* prm, const TdbArgs& a)
 // of at most 96 (nothing was written).  Points the planes are no good for (a
 // singular or nearly singular plane) are solved by the block path before it
 // returns, leads whose decimation lost digits are decimated by it.
-bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
+bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a, PlanesLeads* share)
 {
     const bool wait = c->dec_check > 0;        // the host may wait for the device
     const PlanDims d = plan_dims(a.nl, a.nr, a.b, a.L, a.nk);
@@ -1851,22 +1893,76 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
     w.off = fixed;
     C2 *pH = w.ptr<C2>(oH), *pU = w.ptr<C2>(oU), *pL = w.ptr<C2>(oL), *pV = w.ptr<C2>(oV);
     unsigned long long* pM = w.ptr<unsigned long long>(oM);
-    const ChunkView cv = carve(w, P);
+    const ChunkView own = carve(w, P);
     launch(c, NT_K_ELEM, 0, "plane pack", [&] {
         hipLaunchKernelGGL(k_pl_pack, dim3(h.M, a.nk, 4), dim3(256), 0, s, d, v, B, pH, pU, pL, pV, pM);
         return hipGetLastError();
     });
+    // Leads that another device of the call has or may want: the first one keeps
+    // its self-energies for those whose lead cells have the same planes (the
+    // couplings to the device take part in the plan)
+    LeadsView lv{};
+    bool reuse = false, keep_leads = false;
+    if (share && wait && !a.noalloc && !adj && h.m0 + h.m1 <= 4 * PL_NLV) {
+        Arena sa;
+        leads_carve(sa, a.npts, NN, h.m0 + h.m1);
+        const bool alike = share->have && share->nt == h.nt && share->m0 == h.m0 && share->m1 == h.m1;
+        if (!share->have && (double)sa.off <= PL_SHARE_BYTES &&
+            (sa.off <= c->leads_bytes || (double)sa.off <= 0.25 * (free_bytes(c) + (double)c->leads_bytes))) {
+            if (c->leads_bytes < sa.off) {
+                if (c->leads_buf) {
+                    hipcheck(c, hipStreamSynchronize(s), "hipStreamSynchronize");
+                    hipcheck(c, hipFree(c->leads_buf), "hipFree");
+                    c->leads_buf = nullptr;
+                    c->leads_bytes = 0;
+                }
+                hipcheck(c, hipMalloc(&c->leads_buf, sa.off), "hipMalloc leads");
+                c->leads_bytes = sa.off;
+            }
+            keep_leads = true;
+        }
+        if (alike || keep_leads) {
+            sa = Arena();
+            sa.base = static_cast<char*>(c->leads_buf);
+            lv = leads_carve(sa, a.npts, NN, h.m0 + h.m1);
+            launch(c, NT_K_ELEM, 0, "fill", [&] { return launch_fill_int(cnt + CNT_SAME, 1, 1, s); });
+            hipLaunchKernelGGL(k_pl_lead_planes, dim3(h.m0 + h.m1), dim3(128), 0, s, v.h, v.psize, v.perm, lv.planes,
+                               keep_leads ? 1 : 0, cnt + CNT_SAME);
+            hipcheck(c, hipGetLastError(), "lead planes");
+        }
+        if (alike) {
+            hipcheck(c, hipMemcpyAsync(c->host_plan, cnt + CNT_SAME, sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
+            hipcheck(c, hipStreamSynchronize(s), "sync");
+            reuse = c->host_plan[0] != 0;
+        }
+    }
+    auto copy = [&](void* to, const void* from, size_t bytes) {
+        hipcheck(c, hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, s), "copy leads");
+    };
     int left = 0, later[2] = {0, 0};      // points solved on the layers, those not beside the sweep
     for (int p0 = 0; p0 < a.npts; p0 += P) {
         const int n = std::min(P, a.npts - p0);
         const int* kidx = a.kidx ? a.kidx + p0 : nullptr;
         const int* first = a.first_mask ? a.first_mask + p0 : nullptr;
+        ChunkView cv = own;
+        if (reuse) {
+            cv.sigma = lv.sigma + 2L * p0 * NN;
+            cv.left = lv.left + (long)p0 * NN;
+            cv.loss = lv.loss + 2L * p0;
+            cv.dst = lv.dst + 2L * p0;
+            cv.dit = lv.dit + 2L * p0;
+        }
         const DecPlArgs da{v.h, v.psize, pH, pU, pL, pV, a.E + p0, kidx, prm->eta, prm->eta0, prm->convergence,
                            prm->eta_mode, prm->max_iter, cv.scratch, cv.sigma, cv.dst, cv.dit, cv.loss};
         SweepPlArgs sa{v.h, v.psize, pH, pU, pL, pM, a.E + p0, kidx, prm->eta, prm->eta0, prm->device_eta_factor,
                              prm->eta_mode, need + p0, cv.sigma, nullptr, cv.T, cv.grow, cv.sst, cv.keep, v.poff + a.adj_lo + 1, kept};
         if (p0) zero_dev(c, cnt, sizeof(int) * CNT_STEPS, s);
-        if (big) planes_big_leads(c, prm, a, v, h, bv, w, pH, pU, pL, pV, p0, n, cv);
+        if (reuse) {
+            copy(need + p0, lv.need + p0, sizeof(int) * n);
+            hipLaunchKernelGGL(k_pl_count, dim3(nblk(n)), dim3(256), 0, s, n, need + p0, cnt);
+            hipcheck(c, hipGetLastError(), "count");
+            sa.left = cv.left;
+        } else if (big) planes_big_leads(c, prm, a, v, h, bv, w, pH, pU, pL, pV, p0, n, cv);
         else launch(c, NT_K_PLANES, 0, "plane decimation", [&] {
             if (!wait || h.nt == 1) launch_decimate<1>(da, 2 * n, s);
             if (!wait || h.nt == 2) launch_decimate<2>(da, 2 * n, s);
@@ -1877,7 +1973,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         // leads that lost digits: once more on the layers, where the host may wait
         // for their count and the call may allocate (else the whole point)
         const int lossy = wait && !a.noalloc ? NEED_LEADS : NEED_LAYERS;
-        hipLaunchKernelGGL(k_pl_check, dim3(nblk(n)), dim3(256), 0, s, v.h, n, cv.dst, cv.loss, a.E + p0, prm->eta,
+        if (!reuse)
+            hipLaunchKernelGGL(k_pl_check, dim3(nblk(n)), dim3(256), 0, s, v.h, n, cv.dst, cv.loss, a.E + p0, prm->eta,
                            prm->eta0, prm->eta_mode, adj ? PL_RESIDUAL_ADJ : PL_RESIDUAL, lossy, need + p0, cnt);
         hipcheck(c, hipGetLastError(), "plane check");
         int n1 = 0;                        // points for the layers
@@ -1888,6 +1985,18 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
             if (const int m = c->host_plan[CNT_LEADS]) {
                 n1 += planes_redo_leads(c, prm, a, d, v, B, cv, NP, p0, n, m, need + p0, cnt, n1);
                 sa.left = cv.left;
+            }
+            if (keep_leads) {
+                const size_t row = z * NN;
+                copy(lv.sigma + 2L * p0 * NN, cv.sigma, 2 * row * n);
+                if (sa.left) copy(lv.left + (long)p0 * NN, cv.left, row * n);
+                else
+                    hipcheck(c, hipMemcpy2DAsync(lv.left + (long)p0 * NN, row, cv.sigma, 2 * row, row, n,
+                                                 hipMemcpyDeviceToDevice, s), "copy leads");
+                copy(lv.loss + 2L * p0, cv.loss, sizeof(LeadLoss) * 2 * n);
+                copy(lv.dst + 2L * p0, cv.dst, sizeof(int) * 2 * n);
+                copy(lv.dit + 2L * p0, cv.dit, sizeof(int) * 2 * n);
+                copy(lv.need + p0, need + p0, sizeof(int) * n);
             }
             hipcheck(c, hipEventRecord(c->chk[0], s), "event check");
         }
@@ -1917,9 +2026,10 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a)
         later[0] += beside ? 0 : n1;
         later[1] += c->host_plan[CNT_AFTER_SWEEP];
     }
+    if (keep_leads) *share = PlanesLeads{true, h.nt, h.m0, h.m1};
     const double steps = wait ? (double)c->host_plan[CNT_STEPS] : 0.0;
     // of a decimation step: the inverse of two planes and eight products of one
-    if (c->prof && !big) c->flops_pending[NT_K_PLANES] += steps * 16 * 8 * (16.0 * h.nt) * (16.0 * h.nt) * (16.0 * h.nt);
+    if (c->prof && !big && !reuse) c->flops_pending[NT_K_PLANES] += steps * 16 * 8 * (16.0 * h.nt) * (16.0 * h.nt) * (16.0 * h.nt);
     if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - (a.noalloc ? 0 : left);      // (the layers count theirs)
     TdbArgs g = a;
     g.siblings.clear();

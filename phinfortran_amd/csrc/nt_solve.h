@@ -56,7 +56,14 @@ void solve_tdb_dev(nt_ctx* c, const nt_params* prm, const TdbArgs& a);
 // sum over parts).  Throws Fail; runs inside guarded().
 void solve_split(nt_ctx* c, const nt_params* p, const TdbArgs& a, int parts);
 
+// Self-energies of the leads on planes, of all points of a call: left by the
+// first of several devices with the same leads and points for the others.
+struct PlanesLeads {
+    bool have = false;
+    int nt = 0, m0 = 0, m1 = 0;      // class, planes of the two lead cells
+};
+
 // The solve on the planes of the layers (nt_planes.hip): whether a call is of
 // its kind, and the solve itself (false: the blocks do not fall into planes).
 bool planes_candidate(const nt_ctx* c, const nt_params* prm, const TdbArgs& a);
-bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a);
+bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a, PlanesLeads* share = nullptr);

@@ -39,3 +39,43 @@ def test_shared_leads_equal_single_solves(engine):
             tl, tr, _ = O.solve_tdb(blocks[i][kidx[j]].as_dict(), E[j], op)
             assert abs(o["T_LR"][j].item() - tl) < 1e-9 * max(1, tl)
             assert abs(o["T_RL"][j].item() - tr) < 1e-9 * max(1, tr)
+
+
+def test_shared_leads_on_planes(engine):
+    """Devices with the same leads on planes: one decimation for those whose lead
+    cells have the same planes, a further one where the coupling to the device
+    reaches deeper into the cell; bit for bit the single solves, in chunks of
+    different sizes too."""
+    import dataclasses
+
+    from phinfortran_amd import _native as N
+    from phinfortran_amd import transport as T
+    from test_gpu_planes import plane_blocks
+    p = T.params("phonon", eta=1e-3, eta0=1e-4, convergence=1e-13)
+    base = plane_blocks((12, 12, 12), (12, 11), 3, 4)
+    deep = base.Hamld.copy()
+    inside = np.flatnonzero(np.any(base.Hamlv != 0, 0))                # the plane that faces the lead
+    middle = np.flatnonzero(np.any(base.Haml[inside] != 0, 0) & ~np.any(base.Hamlv != 0, 0))
+    deep[middle[0], np.flatnonzero(np.any(deep != 0, 0))[0]] = 0.3
+    sets = [base, dataclasses.replace(base, Hamd=1.1 * base.Hamd), dataclasses.replace(base, Hamld=deep),
+            dataclasses.replace(base, Hamdv=0.9 * base.Hamdv)]
+    E = np.linspace(0.05, 0.9, 33)
+    for limit in (512, 10):
+        eng = T.Engine(0, batch_limit=limit)
+        try:
+            devices = [dict(blocks=eng.upload_blocks(b), E=E) for b in sets]
+            chunks = -(-E.size // limit)
+            print(f"shared leads on planes, {limit} points a chunk", flush=True)
+            for workers in (1, 4):
+                eng.set_multi_workers(workers)
+                eng.profile_reset()
+                eng.profile(True)
+                outs = eng.solve_tdb_multi(devices, p)
+                eng.profile(False)
+                assert eng.profile_get(N.NT_K_PLANES)["launches"] == chunks * (2 + 4)
+                for d, o in zip(devices, outs):
+                    r = eng.solve_tdb(d["blocks"], E, p)
+                    for k in ("T_LR", "T_RL", "status"):
+                        assert np.array_equal(o[k].cpu().numpy(), r[k].cpu().numpy()), k
+        finally:
+            eng.close()

@@ -342,8 +342,12 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
                     double rc = __builtin_amdgcn_rcp(den);
                     rc = fma(rc, fma(-den, rc, 1.0), rc);
                     rc = fma(rc, fma(-den, rc, 1.0), rc);
-                    rc = den != 0.0 ? rc : 0.0;
-                    const double vr = dr * rc, vi = -di * rc;      // 1 / pivot
+                    double vr = dr * rc, vi = -di * rc;      // 1 / pivot
+                    // where 1 / den has no double, or den is zero or not finite
+                    if (__builtin_expect(!(den > 1e-290 && den < 1e290), 0)) {
+                        vr = den != 0.0 ? dr / den : 0.0;
+                        vi = den != 0.0 ? -di / den : 0.0;
+                    }
                     const bool own = lane == pl;
                     const double fr = xr[0][0], fi = xi[0][0];
                     const double tr = fr * vr - fi * vi, ti = fr * vi + fi * vr;
@@ -394,6 +398,11 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
                             const double rc = 1.0 / den;
                             vr = dr * rc;
                             vi = -di * rc;
+                        }
+                        // (where 1 / den has no double)
+                        if (__builtin_expect(den != 0.0 && !(den > 1e-290 && den < 1e290), 0)) {
+                            vr = dr / den;
+                            vi = -di / den;
                         }
                         if (lane == 0) {
                             s.piv[16 * J + c] = p;

@@ -321,3 +321,28 @@ def test_zinv_in_registers(engine, torch_dev, n, batch):
         ref = np.linalg.inv(A[i])
         # as for the panel kernels: eps n cond, and n for the growth of the pivots
         assert np.abs(X[i] - ref).max() < 1e-14 * np.linalg.cond(A[i]) * np.abs(ref).max() * n, i
+
+
+@pytest.mark.parametrize("n", [24, 64, 96, 128])
+@pytest.mark.parametrize("e", [-514, 505])
+def test_zinv_in_registers_of_tiny_and_huge_matrices(engine, torch_dev, n, e):
+    """Pivots of about 2^e: |pivot|^2 is a subnormal number (e = -514, 43 bits and
+    more of it left), or its reciprocal is (e = 505 only just not).  The inverse
+    is as accurate as the 43 bits, 1e-13 per pivot."""
+    from phinfortran_amd import _native as N
+    torch, dev = torch_dev
+    rng = np.random.default_rng(n)
+    A = [crand(rng, n, n) + 0.5 * n ** 0.5 * np.eye(n) for _ in range(2)]
+    ref = [np.linalg.inv(a) for a in A]
+    dA = to_dev(torch, dev, [a * 2.0 ** e for a in A])
+    dX = torch.zeros_like(dA)
+    info = torch.zeros(2, dtype=torch.int32, device=dev)
+    print(f"zinv n={n}, elements of 2^{e}", flush=True)
+    st = N.lib().nt_zinv_batched_dev(engine.ctx, n, C.c_void_p(dA.data_ptr()), n * n, C.c_void_p(dX.data_ptr()), n * n,
+                                     C.c_void_p(info.data_ptr()), 2)
+    assert st == 0
+    engine.sync()
+    assert (info.cpu().numpy() == 0).all()
+    for x, r, a in zip(from_dev(dX), ref, A):
+        err = np.abs(x * 2.0 ** (e / 2) * 2.0 ** (e - e / 2) - r).max()
+        assert err <= 1e-13 * n * np.linalg.cond(a) * np.abs(r).max(), err

@@ -57,10 +57,13 @@ constexpr int PL_NLV = 128;         // levels a layer may have
 constexpr double PL_RESIDUAL = 1.0e-6, PL_RESIDUAL_ADJ = 1.0e-7;
 // A loss beyond the broadening may make the recursion grow without end instead:
 // of 360,000 energies of ribbons at eta = 1e-8 eV the layers' did at 47 where the
-// planes' did not, with residuals of 2 eta / scale and more.  So the bound is at
-// most eta / scale, and whether a recursion ends is decided on the layers: 31 of
-// 2048 points of the ribbon, 0.4 of 1024 of the film.
-constexpr double PL_RESIDUAL_ETA = 1.0;
+// planes' did not, all with residuals of 2 eta / scale and more, 46 of 5 and
+// more; of 740,000 frequencies of films, 117 with more than eta / scale, none
+// did.  Whether a recursion ends is decided on the layers from the bound
+// PL_RESIDUAL_ETA eta / scale on (0.1 of 1024 points of the film), from eta / scale
+// itself where that is less than PL_SMALL_ETA: the electrons' calls have such
+// leads anyway (31 of 2048 points of the ribbon), and a few more take no longer.
+constexpr double PL_RESIDUAL_ETA = 5.0, PL_SMALL_ETA = 1.0e-8;
 // Planes inside a lead cell and of the device are eliminated with pivots from
 // one plane only, and a plane may be nearly singular at E where its layer is
 // not.  With kappa = |G|max scale of the eliminated planes, G between the leads
@@ -70,10 +73,10 @@ constexpr double PL_RESIDUAL_ETA = 1.0;
 // (on layers 3e-11), at kappa 2e5 3e-10.  T changes by 2 sqrt(T) times as much,
 // and by no less than its square: what is bounded is kappa sqrt(T), with T from
 // this floor (kappa <= 1e9: 1e-13) to 1, in a gradient, which is of first order
-// in G, from 0.01.  The film reaches 4e4, the wire 2e5 (one point of 3000 beyond
-// 1e5, at T = 0.26), the ribbon 2e6 in its gap.
+// in G, from 0.01.  Films reach 1.2e5 (40,000 points), the wire 2e5, the ribbon
+// 1.5e5 and, in its gap, 2e6; a point on layers of 192 takes 100 ms.
 constexpr double PL_T_FLOOR = 1.0e-8, PL_T_FLOOR_ADJ = 0.01;
-constexpr double PL_KAPPA = 1.0e5;
+constexpr double PL_KAPPA = 3.0e5;
 
 // need[p]: 0 solved on the planes, else why it is not (yet)
 enum { NEED_LAYERS = 1, NEED_AFTER_SWEEP = 2, NEED_LEADS = 3 };
@@ -991,8 +994,8 @@ __global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const LeadLo
             const LeadLoss l = loss[2 * p + i];
             // (the sweep goes through the planes inside the cell as well)
             bad = bad || (d != 0 && d != -1 && d != NT_ERR_NOT_CONVERGED) || (d == 0 && l.mid > PL_KAPPA);
-            lost = lost || d == -1 ||
-                   (d == 0 && !(l.res <= fmin(res_max, PL_RESIDUAL_ETA * fabs(et) / l.scale) && l.mid <= PL_KAPPA));
+            const double r = fabs(et) / l.scale, b = fmin(res_max, r < PL_SMALL_ETA ? r : PL_RESIDUAL_ETA * r);
+            lost = lost || d == -1 || (d == 0 && !(l.res <= b && l.mid <= PL_KAPPA));
         }
         why = bad ? NEED_LAYERS : lost ? lossy : 0;
     }

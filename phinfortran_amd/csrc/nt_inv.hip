@@ -888,9 +888,9 @@ hipError_t launch_inv_any(const InvArgs<T>& a, hipStream_t s)
     if (a.batch <= 0 || a.n <= 0) return hipSuccess;
     if (a.n > inv_max_n()) return hipErrorInvalidValue;
     if constexpr (sizeof(T) == 8) {
-        // 4096 inverses in registers, by panels of 16: n = 24 0.115, 0.636 ms; 48
-        // 0.260, 1.26; 64 0.531, 1.79; 96 2.51, 3.50; 128 4.38, 5.27.  Two of
-        // n = 48 40, 147 us; of 96 149, 351.  From 129 on a wave's columns and a
+        // 4096 inverses in registers, by panels of 16: n = 24 0.117, 0.635 ms; 48
+        // 0.268, 1.26; 64 0.542, 1.80; 96 2.56, 3.50; 128 4.43, 5.27.  Two of
+        // n = 48 42, 148 us; of 96 154, 349.  From 129 on a wave's columns and a
         // panel no longer fit its 256 registers.
         if (a.n <= INV_REG_MAX && a.nb == 0) return launch_inv_reg(a, s);
     }

@@ -539,7 +539,7 @@ __device__ __forceinline__ void blk_shift(Blk<NT>& m, double zr, double zi, int 
 // 2 NT waves: the first NT own the columns of A, the others those of B.
 // Bound by the inverse's pivot chain; from NT = 3 on one workgroup has a CU to
 // itself, and its waves' registers spill.  2048 leads of a film of 192 (four
-// planes of 48): 30.7 ms.
+// planes of 48): 29.8 ms.
 constexpr int DEC_SLOTS = 19;       // matrices of NP^2 per item
 
 template <int NT>
@@ -783,8 +783,8 @@ __global__ __launch_bounds__(128 * NT, PL_WAVES) void k_pl_decimate(DecPlArgs a)
 // layers costs inverses here as well.  The couplings' zero pieces (4 columns by
 // 16 rows) are skipped by a mask, and up to 48 three waves per SIMD are built
 // for: film of 168 planes of 48, 1024 points, 54.6 -> 43.9 ms from both, 38.3
-// with the shorter pivot chain.  The whole solve of
-// them: 748 ms on layers of 192, 71 on planes, 31 of them the decimation.
+// with the shorter pivot chain, 39.5 with the measure of the planes' inverses.  The whole solve of
+// them: 748 ms on layers of 192, 71 on planes, 30 of them the decimation.
 template <int NT>
 __global__ __launch_bounds__(64 * NT, NT < 4 ? 3 : 2) void k_pl_sweep(SweepPlArgs a)
 {
@@ -977,11 +977,10 @@ __global__ __launch_bounds__(64 * NT, PL_WAVES) void k_pl_adjoint(AdjPlArgs a)
     }
 }
 
-// NEED_LAYERS: plan refused, a singular or nearly singular plane of a lead; lossy: what a point
-// needs whose leads lost digits or left the finite numbers
+// NEED_LAYERS: plan refused, a singular or nearly singular plane of a lead;
+// lossy: what a point needs whose leads lost digits or left the finite numbers
 __global__ void k_pl_check(const PlanHdr* h, int P, const int* dst, const LeadLoss* loss, const double* E, double eta,
-                           double eta0, int mode, double res_max, int lossy, int* need,
-                           int* count)
+                           double eta0, int mode, double res_max, int lossy, int* need, int* count)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P) return;
@@ -1793,7 +1792,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a, PlanesLeads
     // the large class where the host may wait, with workspace, with a launch's
     // second dimension for the leads of all k-points, and not at a
     // fixed broadening (the electrons' eta = 1e-8 eV: only phonons were measured)
-    const int ncls = wait && !a.noalloc && 2L * a.nk <= PL_MAX_GRID_Y && prm->eta_mode == NT_ETA_RELATIVE ? PL_NCLS : PL_MAXNT;
+    const bool large = wait && !a.noalloc && 2L * a.nk <= PL_MAX_GRID_Y && prm->eta_mode == NT_ETA_RELATIVE;
+    const int ncls = large ? PL_NCLS : PL_MAXNT;
     launch(c, NT_K_ELEM, 0, "plane pattern", [&] {
         const unsigned gx = nblk((long)d.nmax * d.nmax, 1024);
         // the first k-point's pattern alone refuses dense blocks (49 k-points
@@ -1958,7 +1958,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a, PlanesLeads
         const DecPlArgs da{v.h, v.psize, pH, pU, pL, pV, a.E + p0, kidx, prm->eta, prm->eta0, prm->convergence,
                            prm->eta_mode, prm->max_iter, cv.scratch, cv.sigma, cv.dst, cv.dit, cv.loss};
         SweepPlArgs sa{v.h, v.psize, pH, pU, pL, pM, a.E + p0, kidx, prm->eta, prm->eta0, prm->device_eta_factor,
-                             prm->eta_mode, need + p0, cv.sigma, nullptr, cv.T, cv.grow, cv.sst, cv.keep, v.poff + a.adj_lo + 1, kept};
+                       prm->eta_mode, need + p0, cv.sigma, nullptr, cv.T, cv.grow, cv.sst, cv.keep,
+                       v.poff + a.adj_lo + 1, kept};
         if (p0) zero_dev(c, cnt, sizeof(int) * CNT_STEPS, s);
         if (reuse) {
             copy(need + p0, lv.need + p0, sizeof(int) * n);
@@ -2013,8 +2014,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a, PlanesLeads
             return hipGetLastError();
         });
         hipLaunchKernelGGL(k_pl_finish, dim3(nblk(n)), dim3(256), 0, s, n, cv.dst, cv.dit, cv.sst, cv.T, cv.loss,
-                           cv.grow, adj ? PL_T_FLOOR_ADJ : PL_T_FLOOR, first, need + p0, cnt, a.T_LR + p0, a.T_RL + p0, a.status ? a.status + p0 : nullptr,
-                           a.iters ? a.iters + p0 : nullptr);
+                           cv.grow, adj ? PL_T_FLOOR_ADJ : PL_T_FLOOR, first, need + p0, cnt, a.T_LR + p0,
+                           a.T_RL + p0, a.status ? a.status + p0 : nullptr, a.iters ? a.iters + p0 : nullptr);
         hipcheck(c, hipGetLastError(), "plane finish");
         if (adj) planes_adjoint(c, a, v, h, cv, pU, pL, pM, p0, n, hk, need + p0, kept, hi1);
         if (!wait) continue;
@@ -2033,7 +2034,8 @@ bool planes_solve(nt_ctx* c, const nt_params* prm, const TdbArgs& a, PlanesLeads
     const double steps = wait ? (double)c->host_plan[CNT_STEPS] : 0.0;
     // of a decimation step: the inverse of two planes and eight products of one
     if (c->prof && !big && !reuse) c->flops_pending[NT_K_PLANES] += steps * 16 * 8 * (16.0 * h.nt) * (16.0 * h.nt) * (16.0 * h.nt);
-    if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - (a.noalloc ? 0 : left);      // (the layers count theirs)
+    // (the layers count theirs)
+    if (prm->precision == NT_PREC_MIXED && wait && !adj) c->mixed_counts[0] += a.npts - (a.noalloc ? 0 : left);
     TdbArgs g = a;
     g.siblings.clear();
     g.no_planes = true;

@@ -318,10 +318,10 @@ __device__ __forceinline__ void wg_inverse(C2* work, const InvLds& s, Blk<NT>& m
             // scalars at once, the next column is updated first and its pivot
             // search overlaps the other columns' updates, the pivot row is
             // scaled after the panel (a row's multipliers scale with it) and
-            // there is no branch in a step: 4096 matrices of 48 take 262 us
-            // (293 with the step below), of 64 534 (603).  With two rows per
+            // no branch is taken in a step: 4096 matrices of 48 take 268 us
+            // (293 with the step below), of 64 542 (603).  With two rows per
             // lane the registers do not hold that row beside the panel: the
-            // same order spills (96: 2830 us, against 2507), so there the
+            // same order spills (96: 2830 us, against 2557), so there the
             // pivot row is read as it is used and scaled in its step.
             if constexpr (RPL == 1) {
                 unsigned key = pivot_key();
